@@ -7,6 +7,8 @@
 // (mu, eo, i) and adds all terms of that link to its 8 momentum coordinates,
 // so no atomics are needed and the result is deterministic.  Momenta are
 // device SoA P[4 mu][2 eo][8][vh].
+#include <algorithm>
+
 #include "hb_ops.h"
 #include "hb_su3.h"
 
@@ -73,6 +75,33 @@ __device__ __forceinline__ M3 outer(const double2 (&ga)[12], const double2 (&b)[
       w.m[3 * ca + cb] = acc;
     }
   return w;
+}
+
+// The gauge force's grid: a workgroup holds the four directions of 64
+// consecutive sites of one parity (one wave per direction), its neighbour in
+// the launch the other parity of the same sites.  All links of a neighbourhood
+// are then read at about the same time, instead of by eight passes over the
+// lattice, one per (direction, parity).  The XCDs share out every time slice
+// in contiguous runs of `run` workgroups, so that the slices t and t +- 1 that
+// all of them read stay in the last-level cache.  At 32^3x64 the gauge force
+// takes 3.39 ms in eight passes, 1.78 ms with one contiguous eighth of the
+// lattice per XCD, and 1.73 ms (1.54 ms in a single launch) with shared slices.
+constexpr int kLinkBlock = 256;
+struct LinkGrid {
+  int grid, run;
+  explicit LinkGrid(const Geom &g)
+      : grid(2 * nblocks(g.vh, 64)), run(std::max(1, nblocks(g.vh / g.L[3], 256))) {}
+};
+__device__ __forceinline__ bool link_slot(const Geom &g, int run, int &mu, int &e, int &i) {
+  int b = blockIdx.x;
+  if (b < (int)gridDim.x / (8 * run) * (8 * run)) {
+    const int x = b & 7, k = b >> 3;  // XCD (see xcd_block) and the workgroup's place in it
+    b = k / run * (8 * run) + x * run + k % run;
+  }
+  mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  e = b & 1;
+  i = (b >> 1) * 64 + ((int)threadIdx.x & 63);
+  return i < g.vh;
 }
 
 __device__ __forceinline__ double *mom(double *P, int mu, int eo, int vh) {
@@ -386,11 +415,10 @@ __global__ __launch_bounds__(64) void k_clover_force(double *P, const double2 *_
 // ---------------------------------------------------------------------------
 // gauge force (dsg.F90:28-63) with the staple of staple.F90:28-76
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(128) void k_gauge_force(double *P, const double2 *__restrict__ U, Geom g, double s) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int me = blockIdx.y, mu = me >> 1, e = me & 1, o = 1 - e;
-  if (i >= g.vh) return;
-  const int vh = g.vh;
+__global__ __launch_bounds__(kLinkBlock) void k_gauge_force(double *P, const double2 *__restrict__ U, Geom g, int run, double s) {
+  int mu, e, i;
+  if (!link_slot(g, run, mu, e, i)) return;
+  const int vh = g.vh, o = 1 - e;
   int x[4];
   site_coords(g, e, i, x[0], x[1], x[2], x[3]);
   M3 st = m3_zero();
@@ -550,7 +578,8 @@ int clover_action_parity_dev(Context *c, const double2 *Cb, int eo, double *res_
 
 int dsg_dev(Context *c, double *P, double step, double beta) {
   if (beta == 0.0) return HB_OK;
-  k_gauge_force<<<dim3(nblocks(c->g.vh, 128), 8), 128, 0, c->stream>>>(P, c->gauge, c->g, -step * beta / 3.0);
+  const LinkGrid lg(c->g);
+  k_gauge_force<<<lg.grid, kLinkBlock, 0, c->stream>>>(P, c->gauge, c->g, lg.run, -step * beta / 3.0);
   HB_HIP(hipGetLastError());
   return HB_OK;
 }
