@@ -22,62 +22,7 @@ __device__ __forceinline__ void ld_spinor(double2 (&v)[12], const double2 *__res
   for (int k = 0; k < 12; k++) v[k] = f[(size_t)k * vh + i];
 }
 
-// (1 - sg*gamma_mu) a, all four spin components (d/DSFxyzt.F90:26-56):
-// sg = +1 for the forward term, -1 for the backward term
-template <int MU>
-__device__ __forceinline__ void gamma_a(double2 (&ga)[12], const double2 (&a)[12], double sg) {
-#pragma unroll
-  for (int c = 0; c < 3; c++) {
-    double2 a0 = a[c], a1 = a[3 + c], a2 = a[6 + c], a3 = a[9 + c];
-    if constexpr (MU == 3) {
-      const double2 z = make_double2(0.0, 0.0);
-      if (sg > 0) {
-        ga[c] = z; ga[3 + c] = z;
-        ga[6 + c] = cscale<double2>(2.0, a2); ga[9 + c] = cscale<double2>(2.0, a3);
-      } else {
-        ga[c] = cscale<double2>(2.0, a0); ga[3 + c] = cscale<double2>(2.0, a1);
-        ga[6 + c] = z; ga[9 + c] = z;
-      }
-    } else {
-      // h = a_up - sg*G a_lo ; lower = -sg*G^+ h
-      double2 h0, h1, l0, l1;
-      if constexpr (MU == 0) {  // G = [[0,i],[i,0]]
-        h0 = csub(a0, cscale<double2>(sg, ci(a3)));
-        h1 = csub(a1, cscale<double2>(sg, ci(a2)));
-        l0 = cscale<double2>(sg, ci(h1));   // -sg * (-i h1)
-        l1 = cscale<double2>(sg, ci(h0));
-      } else if constexpr (MU == 1) {  // G = [[0,1],[-1,0]]
-        h0 = csub(a0, cscale<double2>(sg, a3));
-        h1 = cadd(a1, cscale<double2>(sg, a2));
-        l0 = cscale<double2>(sg, h1);       // -sg * (-h1)
-        l1 = cscale<double2>(-sg, h0);      // -sg * h0
-      } else {  // G = [[i,0],[0,-i]]
-        h0 = csub(a0, cscale<double2>(sg, ci(a2)));
-        h1 = cadd(a1, cscale<double2>(sg, ci(a3)));
-        l0 = cscale<double2>(sg, ci(h0));   // -sg * (-i h0)
-        l1 = cscale<double2>(-sg, ci(h1));  // -sg * (i h1)
-      }
-      ga[c] = h0; ga[3 + c] = h1; ga[6 + c] = l0; ga[9 + c] = l1;
-    }
-  }
-}
-
-// w(ca, cb) = sum_s ga_s(ca) conj(b_s(cb))
-__device__ __forceinline__ M3 outer(const double2 (&ga)[12], const double2 (&b)[12]) {
-  M3 w;
-#pragma unroll
-  for (int ca = 0; ca < 3; ca++)
-#pragma unroll
-    for (int cb = 0; cb < 3; cb++) {
-      double2 acc = make_double2(0.0, 0.0);
-#pragma unroll
-      for (int s = 0; s < 4; s++) cfma(acc, ga[3 * s + ca], cconj(b[3 * s + cb]));
-      w.m[3 * ca + cb] = acc;
-    }
-  return w;
-}
-
-// The gauge force's grid: a workgroup holds the four directions of 64
+// The force kernels' grid: a workgroup holds the four directions of 64
 // consecutive sites of one parity (one wave per direction), its neighbour in
 // the launch the other parity of the same sites.  All links of a neighbourhood
 // are then read at about the same time, instead of by eight passes over the
@@ -116,44 +61,78 @@ __device__ __forceinline__ void mom_add(double *P, int mu, int eo, int i, int vh
 // ---------------------------------------------------------------------------
 // hopping part of the fermion force (dsf.F90:77-98 with DSFxyzt.F90:77-117)
 // ---------------------------------------------------------------------------
+// The half spinor of the projector (1 + SG gamma_MU), index 2*colour + spin.
+// ((1 + SG gamma) a) (x) conj(b), summed over the four spins, is the sum over
+// two of h(a) (x) conj(h(b)): gamma is Hermitian and the projector of rank two.
+template <int MU, int SG>
+__device__ __forceinline__ void half_spinor(double2 (&h)[6], const SpinorView<SF64> &f, int i) {
+  if constexpr (MU == 3) {
+    double2 p[6];
+    f.load_pair_raw(p, i, SG < 0 ? 2 : 0);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      h[2 * c] = p[c];
+      h[2 * c + 1] = p[3 + c];
+    }
+  } else {
+    double2 p[12];
+    f.load(p, i);
+    project<MU, SG>(h, p);
+  }
+}
+
+// q += s Im Tr(lambda_j x y^+), x and y 3 x 2
+__device__ __forceinline__ void im_tr_j_outer(double (&q)[8], const double2 (&x)[6], const double2 (&y)[6], double s) {
+  M3 v;
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+      double2 t = make_double2(0.0, 0.0);
+      cfma3<false, true>(t, x[2 * a], y[2 * b]);
+      cfma3<false, true>(t, x[2 * a + 1], y[2 * b + 1]);
+      v.m[3 * a + b] = t;
+    }
+  im_tr_j(q, v, s);
+}
+
 // Bvec/Avec of parity E (index 0) and of the other parity (index 1):
 // E = EVEN: forward term (b_i, at_j), backward (a_i, bt_j);
 // E = ODD : forward term (bt_i, a_j), backward (at_i, b_j).
+// The link multiplies a half spinor, before the outer product with the other.
 template <int MU>
 __device__ void hop_force_link(double (&q)[8], const double2 *__restrict__ U, const Geom &g, int e, int i,
                                const int (&x)[4], const double2 *Bi, const double2 *Aj,
                                const double2 *Ai, const double2 *Bj, double s) {
   const int vh = g.vh;
   int c[4] = {x[0], x[1], x[2], x[3]};
-  double sgn = 1.0;
+  double sg = MU == 3 ? 2.0 * s : s;  // the t projector's factor 2
   c[MU] += 1;
-  if (c[MU] == g.L[MU]) { c[MU] = 0; sgn = (double)g.bc[MU]; }
+  if (c[MU] == g.L[MU]) { c[MU] = 0; sg *= (double)g.bc[MU]; }  // flip_bc's sign of the link
   const int j = site_index(g, c[0], c[1], c[2], c[3]);
-  M3 u = link(U, MU, e, i, vh);
-  m3_scale(u, sgn);  // the reference applies the boundary sign to the links (flip_bc)
-  double2 av[12], ga[12], bv[12];
-  {  // forward: v = U w, w = ((1 - g) A_j) (x) conj(B_i); p -= s Im Tr(lambda v)
-    ld_spinor(av, Aj, j, vh);
-    ld_spinor(bv, Bi, i, vh);
-    gamma_a<MU>(ga, av, 1.0);
-    M3 v = m3_mul(u, outer(ga, bv));
-    im_tr_j(q, v, -s);
-  }
-  {  // backward: v = w U^+, w = ((1 + g) A_i) (x) conj(B_j); p += s Im Tr(lambda v)
-    ld_spinor(av, Ai, i, vh);
-    ld_spinor(bv, Bj, j, vh);
-    gamma_a<MU>(ga, av, -1.0);
-    M3 v = m3_muld(outer(ga, bv), u);
-    im_tr_j(q, v, s);
-  }
+  const M3 u = link_b(U, MU, e, i, vh);
+  const auto view = [vh](const double2 *f) {
+    return SpinorView<SF64>(SpinorPtr<SF64>{const_cast<double2 *>(f), nullptr}, vh);
+  };
+  double2 h[6], k[6], w[6];
+  // forward: p -= s Im Tr(lambda U w), w = ((1 - g) A_j) (x) conj(B_i)
+  half_spinor<MU, -1>(h, view(Aj), j);
+  half_spinor<MU, -1>(k, view(Bi), i);
+  su3_mul_half(w, u.m, h);
+  im_tr_j_outer(q, w, k, -sg);
+  __builtin_amdgcn_sched_barrier(0);
+  // backward: p += s Im Tr(lambda w U^+), w = ((1 + g) A_i) (x) conj(B_j)
+  half_spinor<MU, 1>(h, view(Ai), i);
+  half_spinor<MU, 1>(k, view(Bj), j);
+  su3_mul_half(w, u.m, k);
+  im_tr_j_outer(q, h, w, sg);
 }
 
-__global__ __launch_bounds__(128) void k_hop_force(double *P, const double2 *__restrict__ U, Geom g,
-                                                   const double2 *a, const double2 *b, const double2 *at,
-                                                   const double2 *bt, double s) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int me = blockIdx.y, mu = me >> 1, e = me & 1;
-  if (i >= g.vh) return;
+__global__ __launch_bounds__(kLinkBlock) void k_hop_force(double *P, const double2 *__restrict__ U, Geom g, int run,
+                                                          const double2 *a, const double2 *b, const double2 *at,
+                                                          const double2 *bt, double s) {
+  int mu, e, i;
+  if (!link_slot(g, run, mu, e, i)) return;
   int x[4];
   site_coords(g, e, i, x[0], x[1], x[2], x[3]);
   const double2 *Bi = e == 0 ? b : bt, *Aj = e == 0 ? at : a;
@@ -169,246 +148,393 @@ __global__ __launch_bounds__(128) void k_hop_force(double *P, const double2 *__r
 }
 
 // ---------------------------------------------------------------------------
-// clover parts: the six sigma_mu_nu fields w (clover_bsa / clover_ts) and the
-// derivative of the clover leaves (clover_d)
+// clover parts.  The six sigma_mu_nu fields w_k of clover_bsa / clover_ts
+// (planes k = 12, 13, 14, 23, 24, 34) enter the derivative of the clover
+// leaves (clover_d) once for each orientation of a leaf, as w and as w^+ on
+// the reversed path, so only the Hermitian H_k = s (w_k + w_k^+) is needed;
+// the scale s of the force is part of it.
+//
+// Field of one parity: nine real planes of vh sites per k, addressed as the
+// double2 planes H01, H02, H12, (H00, H11) and the double plane H22.
 // ---------------------------------------------------------------------------
-__constant__ int c_pairs[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
-// spin matrices of clover_bsa_12..34: (S a)_s = sum S[s][s'] a_s'  (entries 0, +-1, +-i)
-__constant__ double2 c_bsa[6][4][4] = {
-    {{{-1, 0}, {0, 0}, {0, 0}, {0, 0}}, {{0, 0}, {1, 0}, {0, 0}, {0, 0}}, {{0, 0}, {0, 0}, {-1, 0}, {0, 0}}, {{0, 0}, {0, 0}, {0, 0}, {1, 0}}},
-    {{{0, 0}, {0, -1}, {0, 0}, {0, 0}}, {{0, 1}, {0, 0}, {0, 0}, {0, 0}}, {{0, 0}, {0, 0}, {0, 0}, {0, -1}}, {{0, 0}, {0, 0}, {0, 1}, {0, 0}}},
-    {{{0, 0}, {0, 0}, {0, 0}, {1, 0}}, {{0, 0}, {0, 0}, {1, 0}, {0, 0}}, {{0, 0}, {1, 0}, {0, 0}, {0, 0}}, {{1, 0}, {0, 0}, {0, 0}, {0, 0}}},
-    {{{0, 0}, {-1, 0}, {0, 0}, {0, 0}}, {{-1, 0}, {0, 0}, {0, 0}, {0, 0}}, {{0, 0}, {0, 0}, {0, 0}, {-1, 0}}, {{0, 0}, {0, 0}, {-1, 0}, {0, 0}}},
-    {{{0, 0}, {0, 0}, {0, 0}, {0, -1}}, {{0, 0}, {0, 0}, {0, 1}, {0, 0}}, {{0, 0}, {0, -1}, {0, 0}, {0, 0}}, {{0, 1}, {0, 0}, {0, 0}, {0, 0}}},
-    {{{0, 0}, {0, 0}, {1, 0}, {0, 0}}, {{0, 0}, {0, 0}, {0, 0}, {-1, 0}}, {{1, 0}, {0, 0}, {0, 0}, {0, 0}}, {{0, 0}, {-1, 0}, {0, 0}, {0, 0}}},
-};
-// coefficients of t(s1,c1,s2,c2) in clover_ts_12..34
-__constant__ double2 c_ts[6][4][4] = {
-    {{{-1, 0}, {0, 0}, {0, 0}, {0, 0}}, {{0, 0}, {1, 0}, {0, 0}, {0, 0}}, {{0, 0}, {0, 0}, {-1, 0}, {0, 0}}, {{0, 0}, {0, 0}, {0, 0}, {1, 0}}},
-    {{{0, 0}, {0, 1}, {0, 0}, {0, 0}}, {{0, -1}, {0, 0}, {0, 0}, {0, 0}}, {{0, 0}, {0, 0}, {0, 0}, {0, 1}}, {{0, 0}, {0, 0}, {0, -1}, {0, 0}}},
-    {{{0, 0}, {0, 0}, {0, 0}, {1, 0}}, {{0, 0}, {0, 0}, {1, 0}, {0, 0}}, {{0, 0}, {1, 0}, {0, 0}, {0, 0}}, {{1, 0}, {0, 0}, {0, 0}, {0, 0}}},
-    {{{0, 0}, {-1, 0}, {0, 0}, {0, 0}}, {{-1, 0}, {0, 0}, {0, 0}, {0, 0}}, {{0, 0}, {0, 0}, {0, 0}, {-1, 0}}, {{0, 0}, {0, 0}, {-1, 0}, {0, 0}}},
-    {{{0, 0}, {0, 0}, {0, 0}, {0, 1}}, {{0, 0}, {0, 0}, {0, -1}, {0, 0}}, {{0, 0}, {0, 1}, {0, 0}, {0, 0}}, {{0, -1}, {0, 0}, {0, 0}, {0, 0}}},
-    {{{0, 0}, {0, 0}, {1, 0}, {0, 0}}, {{0, 0}, {0, 0}, {0, 0}, {-1, 0}}, {{1, 0}, {0, 0}, {0, 0}, {0, 0}}, {{0, 0}, {-1, 0}, {0, 0}, {0, 0}}},
+struct H3 {
+  double2 o[3];  // H01, H02, H12
+  double d[3];
 };
 
-// W[6][9][vh]: w_k = transpose(conj(b) S_k a) at the sites of one parity (clover_bsa)
-__global__ __launch_bounds__(kBlock) void k_w_bsa(double2 *__restrict__ W, const double2 *__restrict__ b, const double2 *__restrict__ a,
-                        int vh) {
+// s (w + w^+) of a general w
+__device__ __forceinline__ H3 herm(const M3 &w, double s) {
+  H3 h;
+  h.d[0] = 2.0 * s * w.m[0].x;
+  h.d[1] = 2.0 * s * w.m[4].x;
+  h.d[2] = 2.0 * s * w.m[8].x;
+  h.o[0] = cscale<double2>(s, cadd(w.m[1], cconj(w.m[3])));
+  h.o[1] = cscale<double2>(s, cadd(w.m[2], cconj(w.m[6])));
+  h.o[2] = cscale<double2>(s, cadd(w.m[5], cconj(w.m[7])));
+  return h;
+}
+__device__ __forceinline__ void store_h(double *__restrict__ F, int k, int i, int vh, const H3 &h) {
+  double *b = F + (size_t)k * 9 * vh;
+  double2 *c = reinterpret_cast<double2 *>(b) + i;
+  c[0] = h.o[0];
+  c[vh] = h.o[1];
+  c[2 * (size_t)vh] = h.o[2];
+  c[3 * (size_t)vh] = make_double2(h.d[0], h.d[1]);
+  b[8 * (size_t)vh + i] = h.d[2];
+}
+__device__ __forceinline__ H3 load_h(const double *__restrict__ F, int k, int i, int vh) {
+  const uint32_t plane = (uint32_t)vh * 16u;
+  const rsrc_t r = make_rsrc(F + (size_t)k * 9 * vh, (uint32_t)vh * 72u);
+  const uint32_t vo = (uint32_t)i * 16u;
+  H3 h;
+#pragma unroll
+  for (int q = 0; q < 3; q++) h.o[q] = bld_f64x2(r, vo, plane * (uint32_t)q);
+  const double2 d = bld_f64x2(r, vo, plane * 3u);
+  h.d[0] = d.x;
+  h.d[1] = d.y;
+  h.d[2] = __builtin_bit_cast(double, bld_u32x2(r, (uint32_t)i * 8u, plane * 4u));
+  return h;
+}
+
+// w_k = sum over spins of (S_k a)_s (x) conj(b_s) (clover_bsa_12..34) from the
+// sixteen products T(s, s') = a_s' (x) conj(b_s): S_k has one entry per row,
+//   12: -00 +11 -22 +33    13: i (10 - 01 + 32 - 23)   23: -(01 + 10 + 23 + 32)
+//   14: 03 + 12 + 21 + 30  24: i (12 - 03 + 30 - 21)   34: 02 - 13 + 20 - 31
+__global__ __launch_bounds__(kBlock) void k_h_spinors(double *__restrict__ F, const double2 *__restrict__ b,
+                                                      const double2 *__restrict__ a, int vh, double s) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= vh) return;
   double2 av[12], bv[12];
   ld_spinor(av, a, i, vh);
   ld_spinor(bv, b, i, vh);
-  for (int k = 0; k < 6; k++) {
-    double2 sa[12];
+  // t += or -= a_s' (x) conj(b_s)
+  const auto add = [&](M3 &t, int sb, int sa, double sign) {
 #pragma unroll
-    for (int c = 0; c < 3; c++)
+    for (int ca = 0; ca < 3; ca++)
 #pragma unroll
-      for (int s = 0; s < 4; s++) {
-        double2 acc = make_double2(0.0, 0.0);
-#pragma unroll
-        for (int s2 = 0; s2 < 4; s2++) cfma(acc, c_bsa[k][s][s2], av[3 * s2 + c]);
-        sa[3 * s + c] = acc;
+      for (int cb = 0; cb < 3; cb++) {
+        const double2 z = make_double2(sign * av[3 * sa + ca].x, sign * av[3 * sa + ca].y);
+        cfma3<false, true>(t.m[3 * ca + cb], z, bv[3 * sb + cb]);
       }
-    M3 w = outer(sa, bv);
+  };
+  // both combinations of a pair of planes: f - e times i, and +-(e + f)
+  const auto pair = [&](const M3 &e, const M3 &f, int ki, int kr, double sr) {
+    M3 w;
 #pragma unroll
-    for (int m = 0; m < 9; m++) W[((size_t)k * 9 + m) * vh + i] = w.m[m];
+    for (int m = 0; m < 9; m++) w.m[m] = ci(csub(f.m[m], e.m[m]));
+    store_h(F, ki, i, vh, herm(w, s));
+#pragma unroll
+    for (int m = 0; m < 9; m++) w.m[m] = cadd(e.m[m], f.m[m]);
+    store_h(F, kr, i, vh, herm(w, sr * s));
+  };
+  {
+    M3 w = m3_zero();
+    add(w, 0, 0, -1.0); add(w, 1, 1, 1.0); add(w, 2, 2, -1.0); add(w, 3, 3, 1.0);
+    store_h(F, 0, i, vh, herm(w, s));
+  }
+  {
+    M3 e = m3_zero(), f = m3_zero();
+    add(e, 0, 1, 1.0); add(e, 2, 3, 1.0);
+    add(f, 1, 0, 1.0); add(f, 3, 2, 1.0);
+    pair(e, f, 1, 3, -1.0);
+  }
+  {
+    M3 e = m3_zero(), f = m3_zero();
+    add(e, 0, 3, 1.0); add(e, 2, 1, 1.0);
+    add(f, 1, 2, 1.0); add(f, 3, 0, 1.0);
+    pair(e, f, 4, 2, 1.0);
+  }
+  {
+    M3 w = m3_zero();
+    add(w, 0, 2, 1.0); add(w, 1, 3, -1.0); add(w, 2, 0, 1.0); add(w, 3, 1, -1.0);
+    store_h(F, 5, i, vh, herm(w, s));
   }
 }
 
-// W from T = A^-1 (12x12, by LDL^+ solves with the B field, clover_t_init) and
-// the coefficients of clover_ts
-__global__ __launch_bounds__(128) void k_w_ts(double2 *__restrict__ W, const double2 *__restrict__ Cb, int eo,
-                                              int vh) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
-  double2 w[6][9];
+// Z = (L D L^+)^-1 of one stored block (L unit lower triangular, D_k the
+// stored 1/2 * 1/d_k), upper triangle: M = L^-1, Z_rc = sum_k conj(M_kr) D_k M_kc
+__device__ __forceinline__ void ldl6_inverse(double2 (&Z)[6][6], const double2 (&w)[18]) {
+  double2 M[6][6];
+  const double d[6] = {w[15].x, w[15].y, w[16].x, w[16].y, w[17].x, w[17].y};
 #pragma unroll
-  for (int k = 0; k < 6; k++)
+  for (int c = 0; c < 6; c++)
 #pragma unroll
-    for (int m = 0; m < 9; m++) w[k][m] = make_double2(0.0, 0.0);
-  for (int s2 = 0; s2 < 4; s2++)
-    for (int c2 = 0; c2 < 3; c2++) {
-      double2 e[12], col[12];
+    for (int r = c + 1; r < 6; r++) {
+      double2 t = w[r * (r - 1) / 2 + c];
 #pragma unroll
-      for (int k = 0; k < 12; k++) e[k] = make_double2(k == 3 * s2 + c2 ? 1.0 : 0.0, 0.0);
-      clover_apply<SF64, 1>(col, e, Cb, nullptr, eo, i, vh);  // column (s2,c2) of A^-1
-#pragma unroll
-      for (int k = 0; k < 6; k++)
-#pragma unroll
-        for (int s1 = 0; s1 < 4; s1++) {
-          const double2 cf = c_ts[k][s1][s2];
-          if (cf.x == 0.0 && cf.y == 0.0) continue;
-#pragma unroll
-          for (int c1 = 0; c1 < 3; c1++) cfma(w[k][3 * c1 + c2], cf, col[3 * s1 + c1]);
-        }
+      for (int k = c + 1; k < r; k++) cfma3<false, false>(t, w[r * (r - 1) / 2 + k], M[k][c]);
+      M[r][c] = make_double2(-t.x, -t.y);
     }
 #pragma unroll
-  for (int k = 0; k < 6; k++)
+  for (int r = 0; r < 6; r++)
 #pragma unroll
-    for (int m = 0; m < 9; m++) W[((size_t)k * 9 + m) * vh + i] = w[k][m];
+    for (int c = r; c < 6; c++) {
+      // k = c first: M_cc = 1
+      double2 t = r == c ? make_double2(d[c], 0.0) : cscale<double2>(d[c], cconj(M[c][r]));
+#pragma unroll
+      for (int k = c + 1; k < 6; k++) cfma3<true, false>(t, cscale<double2>(d[k], M[k][r]), M[k][c]);
+      Z[r][c] = t;
+    }
 }
 
-__device__ __forceinline__ M3 wmat(const double2 *__restrict__ W, int k, int i, int vh) {
-  M3 r;
+// H_k of T = A^-1 (clover_t_init, clover_ts) from the LDL^+ field of parity eo.
+// T's spin blocks are T_uu = T_ll = Z_1 + Z_2 and T_ul = T_lu = Z_1 - Z_2 with
+// the inverses Z of the two chiral blocks, so that with P = Z_1 + Z_2 and
+// Q = Z_1 - Z_2 (2 x 2 spin blocks of 3 x 3 matrices)
+//   w_12 = 2 (P_11 - P_00)  w_13 = 2i (P_01 - P_10)  w_23 = -2 (P_01 + P_10)
+//   w_14 = 2 (Q_01 + Q_10)  w_24 = 2i (Q_01 - Q_10)  w_34 = 2 (Q_00 - Q_11)
+__global__ __launch_bounds__(kBlock) void k_h_inverse(double *__restrict__ F, const double2 *__restrict__ Cb, int eo,
+                                                      int vh, double s) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= vh) return;
+  double2 P[6][6], Q[6][6];
+  {
+    double2 w[18];
+    load_clover_block<SF64>(w, Cb, nullptr, eo, 0, i, vh);
+    ldl6_inverse(P, w);
+  }
+  {
+    double2 w[18], z[6][6];
+    load_clover_block<SF64>(w, Cb, nullptr, eo, 1, i, vh);
+    ldl6_inverse(z, w);
 #pragma unroll
-  for (int m = 0; m < 9; m++) r.m[m] = W[((size_t)k * 9 + m) * vh + i];
-  return r;
-}
-// the same through a buffer resource over matrix k's nine planes (k uniform)
-__device__ __forceinline__ M3 wmat_b(const double2 *__restrict__ W, int k, int i, int vh) {
-  const uint32_t plane = (uint32_t)vh * 16u;
-  const rsrc_t r = make_rsrc(W + (size_t)k * 9 * vh, plane * 9u);
-  const uint32_t vo = (uint32_t)i * 16u;
-  M3 m;
+    for (int r = 0; r < 6; r++)
 #pragma unroll
-  for (int q = 0; q < 9; q++) m.m[q] = bld_f64x2(r, vo, plane * (uint32_t)q);
-  return m;
+      for (int c = r; c < 6; c++) {
+        Q[r][c] = csub(P[r][c], z[r][c]);
+        P[r][c] = cadd(P[r][c], z[r][c]);
+      }
+  }
+  // 4 s (X_11 - X_00) or its negative, X Hermitian: from the upper triangle
+  const auto diag = [&](const double2 (&X)[6][6], int k, double f) {
+    H3 h;
+#pragma unroll
+    for (int c = 0; c < 3; c++) h.d[c] = f * (X[3 + c][3 + c].x - X[c][c].x);
+    h.o[0] = cscale<double2>(f, csub(X[3][4], X[0][1]));
+    h.o[1] = cscale<double2>(f, csub(X[3][5], X[0][2]));
+    h.o[2] = cscale<double2>(f, csub(X[4][5], X[1][2]));
+    store_h(F, k, i, vh, h);
+  };
+  // X_01 =: Y: 4i s (Y - Y^+) and 4 fr s (Y + Y^+)
+  const auto off = [&](const double2 (&X)[6][6], int ki, int kr, double fr) {
+    M3 y, w;
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+      for (int b = 0; b < 3; b++) y.m[3 * a + b] = X[a][3 + b];
+#pragma unroll
+    for (int m = 0; m < 9; m++) w.m[m] = ci(y.m[m]);
+    store_h(F, ki, i, vh, herm(w, 4.0 * s));  // i (Y - Y^+) = iY + (iY)^+
+    store_h(F, kr, i, vh, herm(y, 4.0 * fr * s));
+  };
+  diag(P, 0, 4.0 * s);
+  off(P, 1, 3, -1.0);
+  off(Q, 4, 2, 1.0);
+  diag(Q, 5, -4.0 * s);
 }
 
-// clover_d_loop (clover/clover_d.F90:152-200) for one link (mu, e, i) and
-// plane partner nu; the w fields live on parity weo.  The eight terms of
-// clover_d_same_eo (:203-233) or clover_d_diff_eo (:236-266) are evaluated in
-// groups that load their links and w matrices when needed (reloads hit the
-// caches), with a scheduling barrier between groups, so that at most five
-// 3x3 matrices are live: loading all seven links and three w matrices first
-// needs ~360 registers and spills.
-#define HB_GROUP_END() __builtin_amdgcn_sched_barrier(0)
+// r += H a (LEFT) or a H
+template <bool LEFT>
+__device__ __forceinline__ void h_prod_acc(M3 &r, const H3 &h, const M3 &a) {
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      double2 &t = r.m[3 * i + j];
+      const double d = LEFT ? h.d[i] : h.d[j];
+      t.x = fma(d, a.m[3 * i + j].x, t.x);
+      t.y = fma(d, a.m[3 * i + j].y, t.y);
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const int p = LEFT ? i : k, q = LEFT ? k : j;  // H_pq
+        if (p == q) continue;
+        const double2 x = LEFT ? a.m[3 * k + j] : a.m[3 * i + k];
+        if (p < q) cfma3<false, false>(t, h.o[p + q - 1], x);
+        else cfma3<true, false>(t, h.o[p + q - 1], x);
+      }
+    }
+}
 // an index the compiler cannot prove equal to its argument: a matrix loaded
 // again through it is a fresh load, not a register kept live since the first
 __device__ __forceinline__ int fresh(int i) {
   asm volatile("" : "+v"(i));
   return i;
 }
-__device__ void d_loop(double (&q)[8], const double2 *__restrict__ U, const Geom &g, int e, int mu, int nu,
-                       int i, const int (&x)[4], const double2 *__restrict__ W, int k, int weo, double s) {
-  const int o = 1 - e, vh = g.vh;
-  const int id = nb(g, x[0], x[1], x[2], x[3], mu, 1);
-  const int ie = nb(g, x[0], x[1], x[2], x[3], nu, 1);
-  const int iff = nb(g, x[0], x[1], x[2], x[3], nu, -1);
-  if (e == weo) {
-    // clover_d_same_eo
-    const int ib = nb2(g, x[0], x[1], x[2], x[3], mu, 1, nu, 1);
-    const int ic = nb2(g, x[0], x[1], x[2], x[3], mu, 1, nu, -1);
-    {
-      const M3 u = m3_mul(link_b(U, mu, e, i, vh), link_b(U, nu, o, id, vh));   // u0 u1
-      HB_GROUP_END();
-      const M3 v = m3_mul(link_b(U, nu, e, i, vh), link_b(U, mu, o, ie, vh));   // u3 u2
-      HB_GROUP_END();
-      {
-        const M3 wa = wmat_b(W, k, i, vh);
-        re_tr_j_prod<0>(q, m3_muld(u, v), wa, s);
-        HB_GROUP_END();
-        re_tr_j_prod<2>(q, m3_mul(wa, v), u, s);
-      }
-      HB_GROUP_END();
-      {
-        const M3 wb = wmat_b(W, k, ib, vh);
-        re_tr_j_prod<2>(q, m3_mul(u, wb), v, s);
-        HB_GROUP_END();
-        re_tr_j_prod<2>(q, m3_mul(v, wb), u, s);
-      }
-    }
-    HB_GROUP_END();
-    {
-      const M3 u = m3_muld(link_b(U, mu, e, fresh(i), vh), link_b(U, nu, e, ic, vh));  // u0 u6^+
-      HB_GROUP_END();
-      const M3 v = m3_dmul(link_b(U, nu, o, iff, vh), link_b(U, mu, o, iff, vh));  // u4^+ u5
-      HB_GROUP_END();
-      {
-        const M3 wa = wmat_b(W, k, fresh(i), vh);
-        re_tr_j_prod<2>(q, m3_mul(wa, v), u, -s);
-        HB_GROUP_END();
-        re_tr_j_prod<0>(q, m3_muld(u, v), wa, -s);
-      }
-      HB_GROUP_END();
-      {
-        const M3 wc = wmat_b(W, k, ic, vh);
-        re_tr_j_prod<2>(q, m3_mul(v, wc), u, -s);
-        HB_GROUP_END();
-        re_tr_j_prod<2>(q, m3_mul(u, wc), v, -s);
-      }
-    }
-  } else {
-    // clover_d_diff_eo
-    {
-      const M3 t = m3_muld(link_b(U, nu, o, id, vh), link_b(U, mu, o, ie, vh));  // u1 u2^+
-      HB_GROUP_END();
-      const M3 u = m3_muld(t, link_b(U, nu, e, i, vh));                          // u1 u2^+ u3^+
-      HB_GROUP_END();
-      {
-        const M3 wd = wmat_b(W, k, id, vh);
-        const M3 u0 = link_b(U, mu, e, fresh(i), vh);
-        re_tr_j_prod<0>(q, m3_mul(u0, wd), u, s);
-        HB_GROUP_END();
-        re_tr_j_prod<2>(q, m3_dmul(u, wd), u0, s);
-      }
-      HB_GROUP_END();
-      const M3 v = m3_dmul(t, m3_dag(link_b(U, mu, e, fresh(i), vh)));                  // u2 u1^+ u0^+
-      HB_GROUP_END();
-      {
-        const M3 we = wmat_b(W, k, ie, vh);
-        const M3 u3 = link_b(U, nu, e, fresh(i), vh);
-        re_tr_j_prod<2>(q, m3_dmul(v, we), u3, s);
-        HB_GROUP_END();
-        re_tr_j_prod<0>(q, m3_mul(u3, we), v, s);
-      }
-    }
-    HB_GROUP_END();
-    {
-      const M3 t = m3_mul(link_b(U, mu, o, iff, vh), link_b(U, nu, e, nb2(g, x[0], x[1], x[2], x[3], mu, 1, nu, -1), vh));  // u5 u6
-      HB_GROUP_END();
-      const M3 u = m3_dmul(t, link_b(U, nu, o, iff, vh));                        // u6^+ u5^+ u4
-      HB_GROUP_END();
-      {
-        const M3 wd = wmat_b(W, k, fresh(id), vh);
-        const M3 u0 = link_b(U, mu, e, fresh(i), vh);
-        re_tr_j_prod<2>(q, m3_dmul(u, wd), u0, -s);
-        HB_GROUP_END();
-        re_tr_j_prod<0>(q, m3_mul(u0, wd), u, -s);
-      }
-      HB_GROUP_END();
-      const M3 v = m3_muld(link_b(U, mu, e, fresh(i), vh), t);                          // u0 u6^+ u5^+
-      HB_GROUP_END();
-      {
-        const M3 wf = wmat_b(W, k, iff, vh);
-        const M3 u4 = link_b(U, nu, o, fresh(iff), vh);
-        re_tr_j_prod<2>(q, m3_dmul(u4, wf), v, -s);
-        HB_GROUP_END();
-        re_tr_j_prod<0>(q, m3_mul(v, wf), u4, -s);
-      }
-    }
+
+// Ends a step of a kernel: the matrix is complete in registers here, and no
+// load of a later step is issued before.
+__device__ __forceinline__ void pin(M3 &m) {
+#pragma unroll
+  for (int k = 0; k < 9; k++) asm volatile("" : "+v"(m.m[k].x), "+v"(m.m[k].y));
+}
+__device__ __forceinline__ void step_end(M3 &m) {
+  pin(m);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The four products of a leaf pair below.  The inner product is formed a row
+// or column at a time, so that no third matrix of temporaries is live.
+//   S += l (c b)^+
+__device__ __forceinline__ void acc_l_cb(M3 &S, const M3 &l, const M3 &c, const M3 &b) {
+#pragma unroll
+  for (int j = 0; j < 3; j++) {
+    double2 t[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) t[k] = m3_elem<0>(c, b, j, k);
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int k = 0; k < 3; k++) cfma3<false, true>(S.m[3 * i + j], l.m[3 * i + k], t[k]);
+    pin(S);
   }
 }
-#undef HB_GROUP_END
+//   S += (a b^+) l^+
+__device__ __forceinline__ void acc_ab_l(M3 &S, const M3 &a, const M3 &b, const M3 &l) {
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    double2 t[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) t[k] = m3_elem<2>(a, b, i, k);
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+#pragma unroll
+      for (int k = 0; k < 3; k++) cfma3<false, true>(S.m[3 * i + j], t[k], l.m[3 * j + k]);
+    pin(S);
+  }
+}
+//   S += l^+ (b^+ c)
+__device__ __forceinline__ void acc_ld_bdc(M3 &S, const M3 &l, const M3 &b, const M3 &c) {
+#pragma unroll
+  for (int j = 0; j < 3; j++) {
+    double2 t[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) t[k] = m3_elem<1>(b, c, k, j);
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int k = 0; k < 3; k++) cfma3<true, false>(S.m[3 * i + j], l.m[3 * k + i], t[k]);
+    pin(S);
+  }
+}
+//   S += (b a)^+ l
+__device__ __forceinline__ void acc_bad_l(M3 &S, const M3 &b, const M3 &a, const M3 &l) {
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    double2 t[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) t[k] = m3_elem<0>(b, a, k, i);
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+#pragma unroll
+      for (int k = 0; k < 3; k++) cfma3<true, false>(S.m[3 * i + j], t[k], l.m[3 * k + j]);
+    pin(S);
+  }
+}
 
-// all clover_d contributions of one link: up to two (W, parity, scale) sets
-__global__ __launch_bounds__(64) void k_clover_force(double *P, const double2 *__restrict__ U, Geom g,
-                                                     const double2 *W0, int weo0, double s0,
-                                                     const double2 *W1, int weo1, double s1) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int me = blockIdx.y, mu = me >> 1, e = me & 1;
-  if (i >= g.vh) return;
+// the H pair of a dressed link: H(y) and H(y + nu), where their parity has a
+// field, times sg = +-1
+template <bool Y, bool N>
+struct HPair {
+  H3 y, n;
+  __device__ __forceinline__ HPair(const double *Hy, int iy, const double *Hn, int in, int k, int vh) {
+    if constexpr (Y) y = load_h(Hy, k, iy, vh);
+    if constexpr (N) n = load_h(Hn, k, in, vh);
+  }
+  __device__ __forceinline__ static H3 times(const H3 &h, double s) {
+    H3 r;
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      r.o[q] = cscale<double2>(s, h.o[q]);
+      r.d[q] = h.d[q] * s;
+    }
+    return r;
+  }
+  // L(y) = H(y) a + a H(y + nu) of the link a = U_nu(y)
+  __device__ __forceinline__ M3 dress(const M3 &a, double sg) const {
+    M3 r = m3_zero();
+    if constexpr (Y) h_prod_acc<true>(r, times(y, sg), a);
+    if constexpr (N) h_prod_acc<false>(r, times(n, sg), a);
+    return r;
+  }
+};
+
+// All clover_d contributions (clover/clover_d.F90:152-266) of one link: H0 and
+// H1 are the H fields of the even and the odd sites (null: none).
+//
+// For the link U = U_mu(x) and a plane partner nu the leaf above is U A B C
+// with A = U_nu(x+mu), B = U_mu(x+nu)^+, C = U_nu(x)^+, and the derivative
+// takes H at its four corners; with L_nu(y) = H(y) U_nu(y) + U_nu(y) H(y+nu)
+// their sum is
+//   S_above = L_nu(x+mu) (U_nu(x) U_mu(x+nu))^+ + U_nu(x+mu) U_mu(x+nu)^+ L_nu(x)^+
+//   S_below = L_nu(x+mu-nu)^+ U_mu(x-nu)^+ U_nu(x-nu)
+//             + (U_mu(x-nu) U_nu(x+mu-nu))^+ L_nu(x-nu)
+// and the force is Re Tr(lambda U sum_nu +-(S_above - S_below)): 16 matrix
+// products per plane for both parities together and one trace per link, where
+// the leaves of each parity and orientation taken apart need 37 and 16.
+//
+// FP64 issue alone is 78 us of the fermion force's 138 us at 16^3x32 (both
+// parities; 693 us leaf by leaf).  The rest is the latency of the loads, at
+// two waves per SIMD: the operands of a step are therefore fetched during the
+// step before, in 250 registers (fetched when needed, in 178 registers and
+// still two waves, it took 193 us; one wave with 360 registers 181 us).  The
+// parities that carry a field are template arguments: tested inside the steps,
+// they split them into blocks across which the compiler keeps 100 registers more.
+template <bool E, bool O>  // H on the link's parity, on the other
+__device__ __forceinline__ void clover_leaves(M3 &S, const double2 *__restrict__ U, const Geom &g, int mu, int e, int i,
+                                              const int (&x)[4], const double *He, const double *Ho) {
+  const int o = 1 - e, vh = g.vh;
+  const int id = nb(g, x[0], x[1], x[2], x[3], mu, 1);
+#pragma unroll 1
+  for (int nu = 0; nu < 4; nu++) {
+    if (nu == mu) continue;
+    const int lo = mu < nu ? mu : nu, hi = mu < nu ? nu : mu;
+    const int k = lo == 0 ? hi - 1 : lo + hi;  // plane (lo, hi): 01 02 03 12 13 23
+    const double sg = mu < nu ? 1.0 : -1.0;
+    const int in = nb(g, x[0], x[1], x[2], x[3], nu, 1);
+    const int idn = nb2(g, x[0], x[1], x[2], x[3], mu, 1, nu, 1);
+    const int im = nb(g, x[0], x[1], x[2], x[3], nu, -1);
+    const int idm = nb2(g, x[0], x[1], x[2], x[3], mu, 1, nu, -1);
+    // every step's operands are loaded while the step before it computes
+    const M3 a = link_b(U, nu, o, id, vh);
+    const HPair<O, E> ha(Ho, id, He, idn, k, vh);
+    const M3 b = link_b(U, mu, o, in, vh), c = link_b(U, nu, e, i, vh);
+    M3 l = ha.dress(a, sg);
+    step_end(l);
+    const HPair<E, O> hc(He, i, Ho, in, k, vh);
+    acc_l_cb(S, l, c, b);
+    step_end(S);
+    l = hc.dress(c, sg);
+    step_end(l);
+    const M3 a2 = link_b(U, nu, e, idm, vh);
+    const HPair<E, O> ha2(He, idm, Ho, fresh(id), k, vh);
+    acc_ab_l(S, a, b, l);
+    step_end(S);
+    const M3 b2 = link_b(U, mu, o, im, vh), c2 = link_b(U, nu, o, im, vh);
+    l = ha2.dress(a2, -sg);
+    step_end(l);
+    const HPair<O, E> hc2(Ho, im, He, fresh(i), k, vh);
+    acc_ld_bdc(S, l, b2, c2);
+    step_end(S);
+    l = hc2.dress(c2, -sg);
+    step_end(l);
+    acc_bad_l(S, b2, a2, l);
+    step_end(S);
+  }
+}
+
+__global__ __launch_bounds__(kLinkBlock, 2) void k_clover_force(double *P, const double2 *__restrict__ U, Geom g, int run,
+                                                             const double *H0, const double *H1) {
+  int mu, e, i;
+  if (!link_slot(g, run, mu, e, i)) return;
+  const double *He = e == 0 ? H0 : H1, *Ho = e == 0 ? H1 : H0;
   int x[4];
   site_coords(g, e, i, x[0], x[1], x[2], x[3]);
+  M3 S = m3_zero();
+  if (He && Ho) clover_leaves<true, true>(S, U, g, mu, e, i, x, He, Ho);
+  else if (He) clover_leaves<true, false>(S, U, g, mu, e, i, x, He, Ho);
+  else clover_leaves<false, true>(S, U, g, mu, e, i, x, He, Ho);
   double q[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  // kept as loops: unrolled, the compiler merges the link loads of all twelve
-  // (set, plane) bodies and keeps them live across the kernel
-#pragma unroll 1
-  for (int set = 0; set < 2; set++) {
-    const double2 *W = set == 0 ? W0 : W1;
-    const double s = set == 0 ? s0 : s1;
-    const int weo = set == 0 ? weo0 : weo1;
-    if (!W || s == 0.0) continue;
-#pragma unroll 1
-    for (int k = 0; k < 6; k++) {
-      const int a = c_pairs[k][0], b = c_pairs[k][1];
-      if (a != mu && b != mu) continue;
-      const int nu = a == mu ? b : a;
-      d_loop(q, U, g, e, mu, nu, i, x, W, k, weo, a == mu ? s : -s);
-    }
-  }
+  re_tr_j_prod<0>(q, link_b(U, mu, e, i, g.vh), S, 1.0);
   mom_add(P, mu, e, i, g.vh, q);
 }
 
@@ -485,6 +611,11 @@ double *mom_scratch(Context *c, int *rc) {
   return static_cast<double *>(scratch(c, SLOT_MOM, sizeof(double) * 64 * (size_t)c->g.vh, rc));
 }
 
+// H field of one parity (k_h_spinors, k_h_inverse)
+static double *h_scratch(Context *c, int slot, int *rc) {
+  return static_cast<double *>(scratch(c, slot, sizeof(double) * 54 * (size_t)c->g.vh, rc));
+}
+
 // dsf.F90:28-110 on device spinors a, b (even parity); P accumulates
 int dsf_dev(Context *c, double *P, double step, double kappa, double csw_kappa, const double2 *a,
             const double2 *b) {
@@ -492,8 +623,8 @@ int dsf_dev(Context *c, double *P, double step, double kappa, double csw_kappa, 
   int rc = 0;
   double2 *at = spinor_scratch(c, SLOT_FORCE0, &rc); HB_TRY(rc);
   double2 *bt = spinor_scratch(c, SLOT_FORCE1, &rc); HB_TRY(rc);
-  double2 *W = static_cast<double2 *>(scratch(c, SLOT_FORCE2, sizeof(double2) * 54 * (size_t)vh, &rc)); HB_TRY(rc);
-  double2 *W2 = static_cast<double2 *>(scratch(c, SLOT_FORCE3, sizeof(double2) * 54 * (size_t)vh, &rc)); HB_TRY(rc);
+  double *H0 = h_scratch(c, SLOT_FORCE2, &rc); HB_TRY(rc);
+  double *H1 = h_scratch(c, SLOT_FORCE3, &rc); HB_TRY(rc);
   double2 *tmp = spinor_scratch(c, SLOT_FORCE4, &rc); HB_TRY(rc);
   const bool clov = csw_kappa != 0.0;
   if (clov) HB_CHECK(c->have_clover[HB_CLOVER_B], HB_E_STATE, "dsf: clover B field not present");
@@ -510,32 +641,29 @@ int dsf_dev(Context *c, double *P, double step, double kappa, double csw_kappa, 
     HB_TRY(zero_f64(c, bt, 12 * (size_t)vh));
   }
   const double s = -step * 2.0 * kappa * kappa;
+  const LinkGrid lg(c->g);
   if (s != 0.0) {
-    k_hop_force<<<dim3(nblocks(vh, 128), 8), 128, 0, c->stream>>>(P, c->gauge, c->g, a, b, at, bt, s);
+    k_hop_force<<<lg.grid, kLinkBlock, 0, c->stream>>>(P, c->gauge, c->g, lg.run, a, b, at, bt, s);
     HB_HIP(hipGetLastError());
   }
   // clover part (dsf.F90:103-109) on physical links
   const double s1 = -step * 2.0 * (csw_kappa / 8.0);
   const double s2 = s1 * kappa * kappa;
   if (s1 != 0.0 || s2 != 0.0) {
-    k_w_bsa<<<nblocks(vh), kBlock, 0, c->stream>>>(W, b, a, vh);
-    k_w_bsa<<<nblocks(vh), kBlock, 0, c->stream>>>(W2, bt, at, vh);
-    k_clover_force<<<dim3(nblocks(vh, 64), 8), 64, 0, c->stream>>>(P, c->gauge, c->g, W, 0, s1, W2, 1, s2);
+    if (s1 != 0.0) k_h_spinors<<<nblocks(vh), kBlock, 0, c->stream>>>(H0, b, a, vh, s1);
+    if (s2 != 0.0) k_h_spinors<<<nblocks(vh), kBlock, 0, c->stream>>>(H1, bt, at, vh, s2);
+    k_clover_force<<<lg.grid, kLinkBlock, 0, c->stream>>>(P, c->gauge, c->g, lg.run, s1 != 0.0 ? H0 : nullptr,
+                                                          s2 != 0.0 ? H1 : nullptr);
     HB_HIP(hipGetLastError());
   }
   return HB_OK;
 }
 
-// dsd.F90:28-49 (clover_dsd on the odd sites)
-int dsd_dev(Context *c, double *P, double step, double csw_kappa) {
-  const double s = -step * 2.0 * (csw_kappa / 8.0);
-  if (s == 0.0) return HB_OK;
-  HB_CHECK(c->have_clover[HB_CLOVER_B], HB_E_STATE, "dsd: clover B field not present");
-  const int vh = c->g.vh;
-  int rc = 0;
-  double2 *W = static_cast<double2 *>(scratch(c, SLOT_FORCE2, sizeof(double2) * 54 * (size_t)vh, &rc)); HB_TRY(rc);
-  k_w_ts<<<nblocks(vh, 128), 128, 0, c->stream>>>(W, c->clov[HB_CLOVER_B], 1, vh);
-  k_clover_force<<<dim3(nblocks(vh, 64), 8), 64, 0, c->stream>>>(P, c->gauge, c->g, W, 1, s, nullptr, 0, 0.0);
+// the clover force of one parity's H field
+static int clover_force_one(Context *c, double *P, int eo, const double *H) {
+  const LinkGrid lg(c->g);
+  k_clover_force<<<lg.grid, kLinkBlock, 0, c->stream>>>(P, c->gauge, c->g, lg.run, eo == 0 ? H : nullptr,
+                                                        eo == 0 ? nullptr : H);
   HB_HIP(hipGetLastError());
   return HB_OK;
 }
@@ -544,26 +672,27 @@ int dsd_dev(Context *c, double *P, double step, double csw_kappa) {
 // scale s, on the loaded (physical) links; P accumulates
 int clover_dsf_dev(Context *c, double *P, int eo, const double2 *b, const double2 *a, double s) {
   if (s == 0.0) return HB_OK;
-  const int vh = c->g.vh;
   int rc = 0;
-  double2 *W = static_cast<double2 *>(scratch(c, SLOT_FORCE2, sizeof(double2) * 54 * (size_t)vh, &rc)); HB_TRY(rc);
-  k_w_bsa<<<nblocks(vh), kBlock, 0, c->stream>>>(W, b, a, vh);
-  k_clover_force<<<dim3(nblocks(vh, 64), 8), 64, 0, c->stream>>>(P, c->gauge, c->g, W, eo, s, nullptr, 0, 0.0);
-  HB_HIP(hipGetLastError());
-  return HB_OK;
+  double *H = h_scratch(c, SLOT_FORCE2, &rc); HB_TRY(rc);
+  k_h_spinors<<<nblocks(c->g.vh), kBlock, 0, c->stream>>>(H, b, a, c->g.vh, s);
+  return clover_force_one(c, P, eo, H);
 }
 
 // clover_dsd (clover/clover_d.F90:40-75) with the loaded LDL^+ field of parity eo
 int clover_dsd_dev(Context *c, double *P, int eo, double s) {
   if (s == 0.0) return HB_OK;
   HB_CHECK(c->have_clover[HB_CLOVER_B], HB_E_STATE, "clover_dsd: clover B field not present");
-  const int vh = c->g.vh;
   int rc = 0;
-  double2 *W = static_cast<double2 *>(scratch(c, SLOT_FORCE2, sizeof(double2) * 54 * (size_t)vh, &rc)); HB_TRY(rc);
-  k_w_ts<<<nblocks(vh, 128), 128, 0, c->stream>>>(W, c->clov[HB_CLOVER_B], eo, vh);
-  k_clover_force<<<dim3(nblocks(vh, 64), 8), 64, 0, c->stream>>>(P, c->gauge, c->g, W, eo, s, nullptr, 0, 0.0);
-  HB_HIP(hipGetLastError());
-  return HB_OK;
+  double *H = h_scratch(c, SLOT_FORCE2, &rc); HB_TRY(rc);
+  k_h_inverse<<<nblocks(c->g.vh), kBlock, 0, c->stream>>>(H, c->clov[HB_CLOVER_B], eo, c->g.vh, s);
+  return clover_force_one(c, P, eo, H);
+}
+
+// dsd.F90:28-49 (clover_dsd on the odd sites)
+int dsd_dev(Context *c, double *P, double step, double csw_kappa) {
+  const double s = -step * 2.0 * (csw_kappa / 8.0);
+  if (s != 0.0) HB_CHECK(c->have_clover[HB_CLOVER_B], HB_E_STATE, "dsd: clover B field not present");
+  return clover_dsd_dev(c, P, 1, s);
 }
 
 // clover_action (clover/clover_action.F90:29-62) of parity eo of the LDL^+

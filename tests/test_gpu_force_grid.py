@@ -35,3 +35,48 @@ def close(got, want):
 def test_gauge_force(case):
     g, lat, u, _ = case
     close(g.dsg(STEP, BETA), lat.dsg(u, STEP, BETA))
+
+
+def test_fermion_force(case):
+    g, lat, u, (a, ai, b) = case
+    x, y = lat.spinor_gauss(6, 0), lat.spinor_gauss(7, 0)
+    flipped = lat.flip_bc(u)
+    want = lat.dsf(lat.op(flipped, a, ai, KAPPA, CSW * KAPPA), flipped, STEP, x, y, b)
+    close(g.dsf(x, y, STEP, KAPPA, CSW * KAPPA), want)
+
+
+def test_clover_determinant_force(case):
+    g, lat, u, (a, ai, b) = case
+    close(g.dsd(STEP, CSW * KAPPA), lat.dsd(b, STEP, CSW * KAPPA, u))
+
+
+def shifted(lat, f, eo_axis, site_axis):
+    """a field moved by one site in t: the parities swap and the site index, whose
+    slowest coordinate is t, moves by one slice"""
+    return np.ascontiguousarray(np.roll(np.flip(f, eo_axis), lat.volh // lat.L[3], site_axis))
+
+
+def test_one_parity(case):
+    """clover_dsf and clover_dsd of one parity: even spinors against dsf at kappa = 0
+    (no hopping and no odd part), odd factors against dsd; the other parities
+    against these on fields moved by one site"""
+    import bqcd_hip
+    g, lat, u, (a, ai, b) = case
+    x, y = lat.spinor_gauss(8, 0), lat.spinor_gauss(9, 0)
+    ck = CSW * KAPPA
+    s = -STEP * 2.0 * ck / 8.0
+    even, odd = lat.gen(), lat.gen()
+    g.clover_dsf(0, even, y, x, s)
+    close(even, lat.dsf(lat.op(u, a, ai, 0.0, ck), u, STEP, x, y, b))
+    g.clover_dsd(1, odd, s)
+    close(odd, lat.dsd(b, STEP, ck, u))
+    moved = bqcd_hip.Lattice(lat.L)
+    moved.load_gauge(shifted(lat, u, 1, 2))
+    moved.load_clover(*[shifted(lat, f, 0, 1) for f in (a, ai, b)])
+    p, q = lat.gen(), lat.gen()
+    n = lat.volh // lat.L[3]
+    moved.clover_dsf(1, p, np.roll(y, n, 0), np.roll(x, n, 0), s)
+    close(p, shifted(lat, even, 1, 2))
+    moved.clover_dsd(0, q, s)
+    close(q, shifted(lat, odd, 1, 2))
+    moved.close()
