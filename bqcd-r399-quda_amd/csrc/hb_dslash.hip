@@ -18,7 +18,7 @@
 
 namespace hb {
 
-template <class S, class G, bool DAG, int EPI>
+template <class S, class G, bool DAG, int EPI, int POL>
 __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<S, G> a) {
   using V = typename S::V;
   using A = typename S::A;
@@ -39,9 +39,9 @@ __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<S, G> a) {
       uint32_t w[13];
       in.load_words(w, i);
       const WaveView16 wv{in, w, i - (int)(threadIdx.x & 63), g.L[0] / 2 <= 32};
-      hop_all<S, G, DAG, 1, WaveView16>(acc, a.U, wv, g, e, i, xc);
+      hop_all<S, G, DAG, 1, WaveView16, POL>(acc, a.U, wv, g, e, i, xc);
     } else {
-      hop_all<S, G, DAG>(acc, a.U, in, g, e, i, xc);
+      hop_all<S, G, DAG, 1, SpinorView<S>, POL>(acc, a.U, in, g, e, i, xc);
     }
   }
 
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<S, G> a) {
     if (active) {
       if (a.C) {
         V r[12];
-        clover_apply<G, 0>(r, acc, a.C, a.Cn, e, i, vh);
+        clover_apply<G, 0, POL>(r, acc, a.C, a.Cn, e, i, vh);
         store_spinor<S>(a.out, i, vh, r);
       } else {
         store_spinor<S>(a.out, i, vh, acc);
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<S, G> a) {
       // the hop sum is complete; keep it from being interleaved with the
       // clover loads
       HB_SCHED_FENCE();
-      if (a.C) clover_apply<G, 0>(r, x0, a.C, a.Cn, e, i, vh);
+      if (a.C) clover_apply<G, 0, POL>(r, x0, a.C, a.Cn, e, i, vh);
       else {
 #pragma unroll
         for (int k = 0; k < 12; k++) r[k] = x0[k];
@@ -91,10 +91,10 @@ __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<S, G> a) {
   }
 }
 
-template <class S, class G>
-int launch_dslash(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
+template <class S, class G, int POL>
+static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
   dim3 grid(nblocks(a.g.vh)), block(kBlock);
-#define HB_DS(D, E) hipLaunchKernelGGL((k_dslash<S, G, D, E>), grid, block, 0, st, a)
+#define HB_DS(D, E) hipLaunchKernelGGL((k_dslash<S, G, D, E, POL>), grid, block, 0, st, a)
   if (!dag) {
     switch (epi) {
       case EPI_PLAIN: HB_DS(false, EPI_PLAIN); break;
@@ -111,8 +111,14 @@ int launch_dslash(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) 
     }
   }
 #undef HB_DS
+}
+
+template <class S, class G>
+int launch_dslash(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
+  if (operator_policy<S, G>(a.g.vh) == kNT) launch_pol<S, G, kNT>(a, dag, epi, st);
+  else launch_pol<S, G, 0>(a, dag, epi, st);
   if (epi == EPI_MTDOT)
-    k_finalize<1><<<1, kFinThreads, 0, st>>>(a.partials, (int)grid.x, a.skip, FinStore1{a.dot_out});
+    k_finalize<1><<<1, kFinThreads, 0, st>>>(a.partials, nblocks(a.g.vh), a.skip, FinStore1{a.dot_out});
   HB_HIP(hipGetLastError());
   return HB_OK;
 }

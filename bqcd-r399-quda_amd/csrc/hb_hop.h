@@ -10,7 +10,7 @@ namespace hb {
 // U_mu(x - mu)^+ backward, with the boundary sign when the hop wraps.
 // For a block of NR right-hand sides stored RHS-fastest, the spinor of site j
 // for RHS r sits at index j*NR + r of the view (NR = 1: plain layout).
-template <class S, class G, int MU, bool FWD, int SG, int NR = 1, class View = SpinorView<S>>
+template <class S, class G, int MU, bool FWD, int SG, int NR = 1, class View = SpinorView<S>, int POL = kNT>
 __device__ __forceinline__ void hop(typename S::V (&acc)[12], const typename G::ST *U,
                                     const View &in, const Geom &g, int e, int i,
                                     const int (&xc)[4], int r = 0) {
@@ -47,8 +47,8 @@ __device__ __forceinline__ void hop(typename S::V (&acc)[12], const typename G::
       project<MU, SG>(h, p);
     }
     V u[9];
-    if (FWD) f *= load_link_f<G>(u, U, MU, e, i, vh);
-    else f *= load_link_f<G>(u, U, MU, 1 - e, j, vh);
+    if (FWD) f *= load_link_f<G, POL>(u, U, MU, e, i, vh);
+    else f *= load_link_f<G, POL>(u, U, MU, 1 - e, j, vh);
     if (FWD) su3_mul_half(w, u, h);
     else su3_adj_mul_half(w, u, h);
     reconstruct<MU, SG, true>(acc, w, f);
@@ -73,10 +73,10 @@ __device__ __forceinline__ void hop(typename S::V (&acc)[12], const typename G::
     }
     V u[9];
     if (FWD) {
-      load_link<G>(u, U, MU, e, i, vh);
+      load_link<G, POL>(u, U, MU, e, i, vh);
       su3_mul_half(w, u, h);
     } else {
-      load_link<G>(u, U, MU, 1 - e, j, vh);
+      load_link<G, POL>(u, U, MU, 1 - e, j, vh);
       su3_adj_mul_half(w, u, h);
     }
     reconstruct<MU, SG>(acc, w);
@@ -124,7 +124,7 @@ struct HopWords16 {
   float sgn;       // boundary sign of the hop
 };
 
-template <class S, class G, int MU, bool FWD, int SG, int NR, class View>
+template <class S, class G, int MU, bool FWD, int SG, int NR, class View, int POL>
 __device__ __forceinline__ void hop_fetch16(HopWords16 &d, const typename G::ST *U, const View &in,
                                             const Geom &g, int e, int i, const int (&xc)[4], int r) {
   int c[4] = {xc[0], xc[1], xc[2], xc[3]};
@@ -139,8 +139,8 @@ __device__ __forceinline__ void hop_fetch16(HopWords16 &d, const typename G::ST 
   const int j = site_index(g, c[0], c[1], c[2], c[3]);
   if constexpr (MU == 3) in.fetch_pair(d.s, j * NR + r, SG < 0 ? 2 : 0);
   else in.template fetch_dir<MU>(d.s, j * NR + r);
-  if (FWD) fetch_link16(d.l, U, MU, e, i, g.vh);
-  else fetch_link16(d.l, U, MU, 1 - e, j, g.vh);
+  if (FWD) fetch_link16<POL>(d.l, U, MU, e, i, g.vh);
+  else fetch_link16<POL>(d.l, U, MU, 1 - e, j, g.vh);
 }
 
 template <int MU, bool FWD, int SG>
@@ -175,14 +175,14 @@ __device__ __forceinline__ void hop_finish16(float2 (&acc)[12], const HopWords16
   }
 }
 
-template <class S, class G, bool DAG, int NR, class View>
+template <class S, class G, bool DAG, int NR, class View, int POL>
 __device__ __forceinline__ void hop_all_pipelined16(float2 (&acc)[12], const typename G::ST *U,
                                                     const View &in, const Geom &g, int e, int i,
                                                     const int (&xc)[4], int r) {
   constexpr int SF = DAG ? 1 : -1;
   constexpr int SB = -SF;
   HopWords16 a, b;
-#define HB_F(MU, FWD, SG, D) hop_fetch16<S, G, MU, FWD, SG, NR, View>(D, U, in, g, e, i, xc, r); \
+#define HB_F(MU, FWD, SG, D) hop_fetch16<S, G, MU, FWD, SG, NR, View, POL>(D, U, in, g, e, i, xc, r); \
   __builtin_amdgcn_sched_barrier(0);
 #define HB_C(MU, FWD, SG, D) hop_finish16<MU, FWD, SG>(acc, D); HB_SCHED_FENCE();
   HB_F(3, true, SF, a)
@@ -201,19 +201,19 @@ __device__ __forceinline__ void hop_all_pipelined16(float2 (&acc)[12], const typ
 // all 8 hops of the hopping matrix into acc, t first (the reference's
 // direction order does not matter for the sum); the forward projector sign is
 // (1 - gamma) for D and (1 + gamma) for D^+
-template <class S, class G, bool DAG, int NR = 1, class View = SpinorView<S>>
+template <class S, class G, bool DAG, int NR = 1, class View = SpinorView<S>, int POL = kNT>
 __device__ __forceinline__ void hop_all(typename S::V (&acc)[12], const typename G::ST *U,
                                         const View &in, const Geom &g, int e, int i,
                                         const int (&xc)[4], int r = 0) {
   if constexpr (HB_HOP_PIPELINE && std::is_same<S, SF16>::value && std::is_same<G, SF16>::value) {
-    hop_all_pipelined16<S, G, DAG, NR, View>(acc, U, in, g, e, i, xc, r);
+    hop_all_pipelined16<S, G, DAG, NR, View, POL>(acc, U, in, g, e, i, xc, r);
     return;
   }
   constexpr int F = hops_per_fence<S>();
   constexpr int SF = DAG ? 1 : -1;
   constexpr int SB = -SF;
 #define HB_HOP(MU, FWD, SG, N)                                    \
-  hop<S, G, MU, FWD, SG, NR, View>(acc, U, in, g, e, i, xc, r);   \
+  hop<S, G, MU, FWD, SG, NR, View, POL>(acc, U, in, g, e, i, xc, r);   \
   if constexpr ((N) % F == 0) HB_SCHED_FENCE();
   HB_HOP(3, true, SF, 1) HB_HOP(3, false, SB, 2)
   HB_HOP(2, true, SF, 3) HB_HOP(2, false, SB, 4)

@@ -32,10 +32,7 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void *p, uint32_t bytes) {
 // data read once per kernel, e.g. links, so that it does not evict the
 // neighbour spinors that other sites reuse)
 constexpr int kNT = 2;
-// load policy of the 16-bit links and clover words (kNT unless tuned otherwise)
-#ifndef HB_REDUCED_OPERATOR_POLICY
-#define HB_REDUCED_OPERATOR_POLICY kNT
-#endif
+// (the POL argument of the loads below; operator_policy in hb_dslash.h chooses)
 template <int POL = 0>
 __device__ __forceinline__ double2 bld_f64x2(rsrc_t r, uint32_t vo, uint32_t so) {
   return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, POL));
@@ -458,7 +455,7 @@ __device__ __forceinline__ void load_link(typename S::V (&u)[9], const typename 
 template <class G> constexpr bool link_raw() { return std::is_same<G, SF16>::value; }
 
 // the six stored words of a 16-bit link (rows 0 and 1), fetched ahead of use
-template <int POL = HB_REDUCED_OPERATOR_POLICY>
+template <int POL = kNT>
 __device__ __forceinline__ void fetch_link16(uint32_t (&w)[6], const SF16::ST *U, int mu, int eo, int i, int vh) {
   rsrc_t r = make_rsrc(U + (size_t)((mu * 2 + eo) * 6) * vh, (uint32_t)vh * 24u);
   const u32x4 a = bld_u32x4<POL>(r, (uint32_t)i * 16u, 0);
@@ -483,7 +480,7 @@ __device__ __forceinline__ void decode_link16(float2 (&u)[9], const uint32_t (&w
   u[8] = cross(u[0], u[4], u[1], u[3]);
 }
 
-template <class G, int POL = HB_REDUCED_OPERATOR_POLICY>
+template <class G, int POL = kNT>
 __device__ __forceinline__ typename G::A load_link_f(typename G::V (&u)[9], const typename G::ST *U,
                                                      int mu, int eo, int i, int vh) {
   if constexpr (link_raw<G>()) {
@@ -706,7 +703,7 @@ __device__ __forceinline__ float2 clover_block_word(double2 v, int k, float2 mc)
 
 // loads block J of the FP64 / FP32 clover field of parity eo at site i (16-bit
 // fields are site-packed, see load_clover_block_raw)
-template <class S>
+template <class S, int POL = kNT>
 __device__ __forceinline__ void load_clover_block(typename S::V (&w)[18], const typename S::ST *C,
                                                   const float *Cn, int eo, int J, int i, int vh) {
   static_assert(!S::kNorm, "16-bit clover blocks are read with load_clover_block_raw");
@@ -714,7 +711,7 @@ __device__ __forceinline__ void load_clover_block(typename S::V (&w)[18], const 
   rsrc_t r = make_rsrc(C + (size_t)(eo * 36 + J * 18) * vh, plane * 18u);
   const uint32_t vo = (uint32_t)i * S::kBytes;
 #pragma unroll
-  for (int k = 0; k < 18; k++) w[k] = S::template bld<kNT>(r, vo, plane * k);
+  for (int k = 0; k < 18; k++) w[k] = S::template bld<POL>(r, vo, plane * k);
 }
 
 // 16-bit clover blocks: per block and element five 16-byte planes (see
@@ -727,10 +724,11 @@ constexpr int kClov16Words = 20;  // the same in short2 units
 // block of element e of a slab (buffer r, plane = 16 * elements per slab
 // bytes): Q as stored (the integers as floats) and the block's factors: the
 // block is c 1 + (m / 32767) Q_int; returns (m / 32767, c)
+template <int POL = kNT>
 __device__ __forceinline__ float2 load_clover_rec16(float2 (&w)[18], rsrc_t r, uint32_t e, uint32_t plane) {
   u32x4 q[5];
 #pragma unroll
-  for (int k = 0; k < 5; k++) q[k] = bld_u32x4<HB_REDUCED_OPERATOR_POLICY>(r, e * 16u, plane * k);
+  for (int k = 0; k < 5; k++) q[k] = bld_u32x4<POL>(r, e * 16u, plane * k);
 #pragma unroll
   for (int k = 0; k < 18; k++) {
     const uint32_t x = q[k >> 2][k & 3];
@@ -742,11 +740,12 @@ __device__ __forceinline__ float2 load_clover_rec16(float2 (&w)[18], rsrc_t r, u
 
 // block J of the 16-bit clover field of parity eo at site i (Cn is unused: the
 // factors are stored with the words)
+template <int POL = kNT>
 __device__ __forceinline__ float2 load_clover_block_raw(float2 (&w)[18], const SF16::ST *C,
                                                         const float *Cn, int eo, int J, int i,
                                                         int vh) {
   rsrc_t r = make_rsrc(C + (size_t)((eo * 2 + J) * kClov16Words) * vh, (uint32_t)vh * kClov16);
-  return load_clover_rec16(w, r, (uint32_t)i, (uint32_t)vh * 16u);
+  return load_clover_rec16<POL>(w, r, (uint32_t)i, (uint32_t)vh * 16u);
 }
 
 // writes the block of element e of a slab of n elements: the words Q (in
@@ -801,7 +800,7 @@ __device__ __forceinline__ void clover_raw_finish(V (&y)[6], const V (&x)[6], fl
 // out = A in (Dirac basis) with A stored as two chiral blocks of A/2
 // (clover_mult_a.F90:44-95); mode 0 = Hermitian product, 1 = LDL^+ solve.
 // SG is the clover storage policy, V the arithmetic complex type.
-template <class SG, int MODE, class V>
+template <class SG, int MODE, int POL = kNT, class V>
 __device__ __forceinline__ void clover_apply(V (&out)[12], const V (&in)[12],
                                              const typename SG::ST *C, const float *Cn, int eo,
                                              int i, int vh) {
@@ -813,8 +812,8 @@ __device__ __forceinline__ void clover_apply(V (&out)[12], const V (&in)[12],
   {
     typename SG::V w[18];
     float2 mc;
-    if constexpr (kRaw) mc = load_clover_block_raw(w, C, Cn, eo, 0, i, vh);
-    else load_clover_block<SG>(w, C, Cn, eo, 0, i, vh);
+    if constexpr (kRaw) mc = load_clover_block_raw<POL>(w, C, Cn, eo, 0, i, vh);
+    else load_clover_block<SG, POL>(w, C, Cn, eo, 0, i, vh);
     V ww[18];
 #pragma unroll
     for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);
@@ -830,8 +829,8 @@ __device__ __forceinline__ void clover_apply(V (&out)[12], const V (&in)[12],
   {
     typename SG::V w[18];
     float2 mc;
-    if constexpr (kRaw) mc = load_clover_block_raw(w, C, Cn, eo, 1, i, vh);
-    else load_clover_block<SG>(w, C, Cn, eo, 1, i, vh);
+    if constexpr (kRaw) mc = load_clover_block_raw<POL>(w, C, Cn, eo, 1, i, vh);
+    else load_clover_block<SG, POL>(w, C, Cn, eo, 1, i, vh);
     V ww[18];
 #pragma unroll
     for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);

@@ -52,7 +52,7 @@ template <class S, class G> struct MultiArgs {
 };
 
 // clover block J of parity eo at site i for kappa group gidx (FP32 planes)
-template <class SG>
+template <class SG, int POL>
 __device__ __forceinline__ void load_clover_block_g(typename SG::V (&w)[18], const typename SG::ST *C,
                                                     const float *Cn, int ngroups, int gidx, int eo,
                                                     int J, int i, int vh) {
@@ -62,22 +62,23 @@ __device__ __forceinline__ void load_clover_block_g(typename SG::V (&w)[18], con
   const uint32_t vo = ((uint32_t)gidx * 72u * (uint32_t)vh + (uint32_t)i) * SG::kBytes;
   const uint32_t base = (uint32_t)(eo * 36 + J * 18);
 #pragma unroll
-  for (int k = 0; k < 18; k++) w[k] = SG::template bld<kNT>(r, vo, plane * (base + k));
+  for (int k = 0; k < 18; k++) w[k] = SG::template bld<POL>(r, vo, plane * (base + k));
 }
 
 // the same block of a 16-bit field: [eo][J] slabs of 16-byte planes whose
 // elements are gidx * vh + i (one buffer per slab spans all groups; see
 // load_clover_rec16); returns (m / 32767, c) -- the block is
 // c 1 + (m / 32767) Q_int.  Cn is unused.
+template <int POL>
 __device__ __forceinline__ float2 load_clover_block_g_raw(float2 (&w)[18], const SF16::ST *C,
                                                           const float *Cn, int ngroups, int gidx,
                                                           int eo, int J, int i, int vh) {
   const size_t slab = (size_t)ngroups * vh;
   rsrc_t r = make_rsrc(C + (size_t)(eo * 2 + J) * slab * kClov16Words, (uint32_t)(slab * kClov16));
-  return load_clover_rec16(w, r, (uint32_t)gidx * (uint32_t)vh + (uint32_t)i, (uint32_t)slab * 16u);
+  return load_clover_rec16<POL>(w, r, (uint32_t)gidx * (uint32_t)vh + (uint32_t)i, (uint32_t)slab * 16u);
 }
 
-template <class SG, class V>
+template <class SG, int POL, class V>
 __device__ __forceinline__ void clover_apply_g(V (&out)[12], const V (&in)[12], const typename SG::ST *C,
                                                const float *Cn, int ngroups, int gidx, int eo, int i,
                                                int vh) {
@@ -88,8 +89,8 @@ __device__ __forceinline__ void clover_apply_g(V (&out)[12], const V (&in)[12], 
   {
     typename SG::V w[18];
     float2 mc;
-    if constexpr (kRaw) mc = load_clover_block_g_raw(w, C, Cn, ngroups, gidx, eo, 0, i, vh);
-    else load_clover_block_g<SG>(w, C, Cn, ngroups, gidx, eo, 0, i, vh);
+    if constexpr (kRaw) mc = load_clover_block_g_raw<POL>(w, C, Cn, ngroups, gidx, eo, 0, i, vh);
+    else load_clover_block_g<SG, POL>(w, C, Cn, ngroups, gidx, eo, 0, i, vh);
     V ww[18];
 #pragma unroll
     for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);
@@ -104,8 +105,8 @@ __device__ __forceinline__ void clover_apply_g(V (&out)[12], const V (&in)[12], 
   {
     typename SG::V w[18];
     float2 mc;
-    if constexpr (kRaw) mc = load_clover_block_g_raw(w, C, Cn, ngroups, gidx, eo, 1, i, vh);
-    else load_clover_block_g<SG>(w, C, Cn, ngroups, gidx, eo, 1, i, vh);
+    if constexpr (kRaw) mc = load_clover_block_g_raw<POL>(w, C, Cn, ngroups, gidx, eo, 1, i, vh);
+    else load_clover_block_g<SG, POL>(w, C, Cn, ngroups, gidx, eo, 1, i, vh);
     V ww[18];
 #pragma unroll
     for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);
@@ -119,7 +120,7 @@ __device__ __forceinline__ void clover_apply_g(V (&out)[12], const V (&in)[12], 
   }
 }
 
-template <class S, class G, int NR, bool DAG, int EPI>
+template <class S, class G, int NR, bool DAG, int EPI, int POL>
 __global__ __launch_bounds__(kBlock) void k_dslash_multi(MultiArgs<S, G> a) {
   using V = typename S::V;
   using A = typename S::A;
@@ -144,9 +145,9 @@ __global__ __launch_bounds__(kBlock) void k_dslash_multi(MultiArgs<S, G> a) {
       uint32_t w[13];
       in.load_words(w, tid);
       const WaveView16 wv{in, w, tid - (int)(threadIdx.x & 63), g.L[0] / 2 * NR <= 32};
-      hop_all<S, G, DAG, NR, WaveView16>(acc, a.U, wv, g, e, site, xc, r);
+      hop_all<S, G, DAG, NR, WaveView16, POL>(acc, a.U, wv, g, e, site, xc, r);
     } else {
-      hop_all<S, G, DAG, NR>(acc, a.U, in, g, e, site, xc, r);
+      hop_all<S, G, DAG, NR, SpinorView<S>, POL>(acc, a.U, in, g, e, site, xc, r);
     }
   }
   const int ie = site * NR + r;
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(kBlock) void k_dslash_multi(MultiArgs<S, G> a) {
     if (active) {
       if (a.C) {
         V o[12];
-        clover_apply_g<G>(o, acc, a.C, a.Cn, a.ngroups, a.grp[r], e, site, vh);
+        clover_apply_g<G, POL>(o, acc, a.C, a.Cn, a.ngroups, a.grp[r], e, site, vh);
         store_spinor<S>(a.out, ie, vhe, o);
       } else {
         store_spinor<S>(a.out, ie, vhe, acc);
@@ -168,7 +169,7 @@ __global__ __launch_bounds__(kBlock) void k_dslash_multi(MultiArgs<S, G> a) {
       V x0[12], o[12];
       load_spinor<S>(x0, a.x0, ie, vhe);
       HB_SCHED_FENCE();
-      if (a.C) clover_apply_g<G>(o, x0, a.C, a.Cn, a.ngroups, a.grp[r], e, site, vh);
+      if (a.C) clover_apply_g<G, POL>(o, x0, a.C, a.Cn, a.ngroups, a.grp[r], e, site, vh);
       else {
 #pragma unroll
         for (int k = 0; k < 12; k++) o[k] = x0[k];
@@ -442,11 +443,10 @@ struct MultiFields {
 
 template <class G> size_t st_bytes() { return sizeof(typename G::ST); }
 
-template <class S, class G, int NR>
-int launch_multi_dslash(Context *c, const MultiArgs<S, G> &a, bool dag, int epi) {
-  const int n = c->g.vh * NR;
-  dim3 grid(nblocks(n, c->multi_tile)), block(c->multi_tile);
-#define HB_DM(D, E) hipLaunchKernelGGL((k_dslash_multi<S, G, NR, D, E>), grid, block, 0, c->stream, a)
+template <class S, class G, int NR, int POL>
+void launch_multi_pol(Context *c, const MultiArgs<S, G> &a, bool dag, int epi) {
+  dim3 grid(nblocks(c->g.vh * NR, c->multi_tile)), block(c->multi_tile);
+#define HB_DM(D, E) hipLaunchKernelGGL((k_dslash_multi<S, G, NR, D, E, POL>), grid, block, 0, c->stream, a)
   if (!dag) {
     if (epi == EPI_CLINV) HB_DM(false, EPI_CLINV);
     else if (epi == EPI_MTIL) HB_DM(false, EPI_MTIL);
@@ -457,8 +457,15 @@ int launch_multi_dslash(Context *c, const MultiArgs<S, G> &a, bool dag, int epi)
     else HB_DM(true, EPI_MTDOT);
   }
 #undef HB_DM
+}
+
+template <class S, class G, int NR>
+int launch_multi_dslash(Context *c, const MultiArgs<S, G> &a, bool dag, int epi) {
+  const int grid = nblocks(c->g.vh * NR, c->multi_tile);
+  if (operator_policy<S, G>(c->g.vh, NR) == kNT) launch_multi_pol<S, G, NR, kNT>(c, a, dag, epi);
+  else launch_multi_pol<S, G, NR, 0>(c, a, dag, epi);
   if (epi == EPI_MTDOT)
-    k_finalize<NR><<<1, kFinThreads, 0, c->stream>>>(a.partials, (int)grid.x, nullptr,
+    k_finalize<NR><<<1, kFinThreads, 0, c->stream>>>(a.partials, grid, nullptr,
                                             FinMultiStore<NR>{a.dot_out, a.flag});
   HB_HIP(hipGetLastError());
   return HB_OK;
