@@ -91,6 +91,134 @@ __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<S, G> a) {
   }
 }
 
+// The same for lattices with few sites per compute unit, where a kernel takes
+// as long as the chain of one thread's eight hops: NW waves of a workgroup
+// share 64 sites, each computes part of the hops, and the parts meet in LDS.
+// Waves 0 and 1 apply one chiral block of the clover term each (to x0 before
+// the barrier, or to the sum of the parts after it); wave 0 writes the result.
+template <class S, class G, bool DAG, int EPI, int NW, int POL>
+__global__ __launch_bounds__(64 * NW) void k_dslash_split(DslashArgs<S, G> a) {
+  using V = typename S::V;
+  using A = typename S::A;
+  __shared__ V part[NW][12][64];
+  __shared__ V y1s[EPI == EPI_PLAIN ? 1 : 6][64];
+  if (a.skip && *a.skip) return;
+  const Geom g = a.g;
+  const int vh = g.vh, e = a.out_parity;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int i = xcd_block(blockIdx.x, gridDim.x) * 64 + lane;
+  const bool active = i < vh;
+  constexpr bool kClovSum = EPI == EPI_CLINV, kClovX0 = EPI == EPI_MTIL || EPI == EPI_MTDOT;
+  V acc[12], x0[12], y[6], dv[12];
+#pragma unroll
+  for (int k = 0; k < 12; k++) acc[k] = cmk<V>((A)0, (A)0);
+  if (active) {
+    int xc[4];
+    site_coords(g, e, i, xc[0], xc[1], xc[2], xc[3]);
+    const SpinorView<S> in(a.in, vh);
+#define HB_PART(W) case W: if constexpr (W < NW) hop_part<S, G, DAG, NW, W % NW, POL>(acc, a.U, in, g, e, i, xc); break;
+    switch (w) {
+      HB_PART(0) HB_PART(1) HB_PART(2) HB_PART(3)
+    }
+#undef HB_PART
+    if constexpr (kClovX0) {
+      if (w < 2) {
+        load_spinor<S>(x0, a.x0, i, vh);
+        if (a.C) {
+          V xp[6];
+#pragma unroll
+          for (int m = 0; m < 6; m++) xp[m] = w == 0 ? cadd(x0[m], x0[m + 6]) : csub(x0[m], x0[m + 6]);
+          clover_block_apply<G, 0, POL>(y, xp, a.C, a.Cn, e, w, i, vh);
+          if (w == 1) {
+#pragma unroll
+            for (int m = 0; m < 6; m++) y1s[m][lane] = y[m];
+          }
+        }
+        if (EPI == EPI_MTDOT && w == 0) load_spinor<S>(dv, a.dotv, i, vh);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 12; k++) part[w][k][lane] = acc[k];
+  }
+  __syncthreads();
+  if (w < (kClovSum ? 2 : 1) && active) {
+#pragma unroll
+    for (int k = 0; k < 12; k++) acc[k] = part[0][k][lane];
+#pragma unroll
+    for (int q = 1; q < NW; q++) {
+#pragma unroll
+      for (int k = 0; k < 12; k++) acc[k] = cadd(acc[k], part[q][k][lane]);
+      HB_SCHED_FENCE();  // one part's reads in flight at a time (registers)
+    }
+    if (kClovSum && a.C) {
+      V xp[6];
+#pragma unroll
+      for (int m = 0; m < 6; m++) xp[m] = w == 0 ? cadd(acc[m], acc[m + 6]) : csub(acc[m], acc[m + 6]);
+      clover_block_apply<G, 0, POL>(y, xp, a.C, a.Cn, e, w, i, vh);
+      if (w == 1) {
+#pragma unroll
+        for (int m = 0; m < 6; m++) y1s[m][lane] = y[m];
+      }
+    }
+  }
+  if (kClovSum && a.C) __syncthreads();
+  if (w > 0) return;
+  double dot = 0.0;
+  if (active) {
+    V r[12];
+    if (EPI != EPI_PLAIN && a.C) {
+#pragma unroll
+      for (int m = 0; m < 6; m++) {
+        const V z = y1s[m][lane];
+        r[m] = cadd(y[m], z);
+        r[m + 6] = csub(y[m], z);
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 12; k++) r[k] = kClovX0 ? x0[k] : acc[k];
+    }
+    if constexpr (kClovX0) {
+      const A mk2 = (A)a.mkappa2, rho = (A)a.rho;
+#pragma unroll
+      for (int k = 0; k < 12; k++) {
+        r[k].x += mk2 * acc[k].x + rho * x0[k].x;
+        r[k].y += mk2 * acc[k].y + rho * x0[k].y;
+      }
+    }
+    store_spinor<S, false>(a.out, i, vh, r);
+    if constexpr (EPI == EPI_MTDOT) {
+#pragma unroll
+      for (int k = 0; k < 12; k++) dot += (double)dv[k].x * (double)r[k].x + (double)dv[k].y * (double)r[k].y;
+    }
+  }
+  if constexpr (EPI == EPI_MTDOT) {
+    dot = wave_sum(dot);
+    if (lane == 0) a.partials[blockIdx.x] = dot;
+  }
+}
+
+template <class S, class G, int NW, int POL>
+static void launch_split(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
+  dim3 grid(nblocks(a.g.vh, 64)), block(64 * NW);
+#define HB_DS(D, E) hipLaunchKernelGGL((k_dslash_split<S, G, D, E, NW, POL>), grid, block, 0, st, a)
+  if (!dag) {
+    switch (epi) {
+      case EPI_PLAIN: HB_DS(false, EPI_PLAIN); break;
+      case EPI_CLINV: HB_DS(false, EPI_CLINV); break;
+      case EPI_MTIL: HB_DS(false, EPI_MTIL); break;
+      default: HB_DS(false, EPI_MTDOT); break;
+    }
+  } else {
+    switch (epi) {
+      case EPI_PLAIN: HB_DS(true, EPI_PLAIN); break;
+      case EPI_CLINV: HB_DS(true, EPI_CLINV); break;
+      case EPI_MTIL: HB_DS(true, EPI_MTIL); break;
+      default: HB_DS(true, EPI_MTDOT); break;
+    }
+  }
+#undef HB_DS
+}
+
 template <class S, class G, int POL>
 static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
   dim3 grid(nblocks(a.g.vh)), block(kBlock);
@@ -113,12 +241,37 @@ static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t
 #undef HB_DS
 }
 
+// Waves that share a site (1: k_dslash).  us per CG iteration at 1 / 2 / 4:
+//   FP64    8^4 (2 k sites per parity) 58.9 / 47.1 / 45.0, 12^3x24 (21 k)
+//           80.3 / 61.5 / 58.4, 16^4 (33 k) 85.4 / 69.0 / 69.2,
+//           16x16x18x18 (41 k) 91.3 / 79.4 / 89.8, 16^3x32 (66 k) 117 / 112 / 112;
+//           M~^+M~ with 18-real links 41 k 66.8 / 63.4 / 68.8, 50 k 74.2 / 80.2 / 82.1
+//   FP32    12^3x24 70.7 / 58.7 / 57.6, 16^4 69.5 / 61.5 / 59.4, 50 k 77.0 / 71.1 /
+//           72.2, 24^3x48 (332 k) 365 / 356 / 358, 32^3x64 1010 / 1056 / 1067
+//   16-bit  12^3x24 60.9 / 55.4 / 52.2, 50 k 62.9 / 58.7 / 60.6, 24^3x48
+//           207 / 200 / 214, 32^3x64 522 / 548 / 580
+// Eight waves (one hop each) were slower than four from 4 k sites on.
+template <class S, class G> static int split_waves(int vh) {
+  if (vh <= (1 << 15)) return 4;
+  constexpr int two = !std::is_same<S, SF64>::value ? 1 << 19 : G::kRecon ? 1 << 16 : 3 << 14;
+  return vh <= two ? 2 : 1;
+}
+
 template <class S, class G>
 int launch_dslash(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
-  if (operator_policy<S, G>(a.g.vh) == kNT) launch_pol<S, G, kNT>(a, dag, epi, st);
-  else launch_pol<S, G, 0>(a, dag, epi, st);
+  const int nw = split_waves<S, G>(a.g.vh), pol = operator_policy<S, G>(a.g.vh);
+  if (nw == 4) {
+    launch_split<S, G, 4, 0>(a, dag, epi, st);
+  } else if (nw == 2) {
+    if (pol == kNT) launch_split<S, G, 2, kNT>(a, dag, epi, st);
+    else launch_split<S, G, 2, 0>(a, dag, epi, st);
+  } else {
+    if (pol == kNT) launch_pol<S, G, kNT>(a, dag, epi, st);
+    else launch_pol<S, G, 0>(a, dag, epi, st);
+  }
   if (epi == EPI_MTDOT)
-    k_finalize<1><<<1, kFinThreads, 0, st>>>(a.partials, nblocks(a.g.vh), a.skip, FinStore1{a.dot_out});
+    k_finalize<1><<<1, kFinThreads, 0, st>>>(a.partials, nblocks(a.g.vh, nw > 1 ? 64 : kBlock), a.skip,
+                                             FinStore1{a.dot_out});
   HB_HIP(hipGetLastError());
   return HB_OK;
 }

@@ -222,4 +222,32 @@ __device__ __forceinline__ void hop_all(typename S::V (&acc)[12], const typename
 #undef HB_HOP
 }
 
+// The hops of wave W of the NW (2 or 4) that share a site: two directions or
+// one; the two hops of a direction have their loads in flight together.
+template <class S, class G, bool DAG, int NW, int W, int POL, class View>
+__device__ __forceinline__ void hop_part(typename S::V (&acc)[12], const typename G::ST *U, const View &in,
+                                         const Geom &g, int e, int i, const int (&xc)[4]) {
+  constexpr int SF = DAG ? 1 : -1;
+  constexpr int SB = -SF;
+#define HB_DIR(MU)                                                                      \
+  if constexpr (std::is_same<S, SF16>::value && std::is_same<G, SF16>::value) {         \
+    HopWords16 a, b;                                                                    \
+    hop_fetch16<S, G, MU, true, SF, 1, View, POL>(a, U, in, g, e, i, xc, 0);            \
+    hop_fetch16<S, G, MU, false, SB, 1, View, POL>(b, U, in, g, e, i, xc, 0);           \
+    hop_finish16<MU, true, SF>(acc, a);                                                 \
+    hop_finish16<MU, false, SB>(acc, b);                                                \
+  } else {                                                                              \
+    hop<S, G, MU, true, SF, 1, View, POL>(acc, U, in, g, e, i, xc);                     \
+    hop<S, G, MU, false, SB, 1, View, POL>(acc, U, in, g, e, i, xc);                    \
+  }
+  if constexpr (NW == 4) {
+    HB_DIR(W)
+  } else {
+    HB_DIR(2 * W)
+    HB_SCHED_FENCE();
+    HB_DIR(2 * W + 1)
+  }
+#undef HB_DIR
+}
+
 }  // namespace hb

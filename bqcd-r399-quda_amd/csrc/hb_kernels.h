@@ -378,7 +378,7 @@ __device__ __forceinline__ void load_spinor(typename S::V (&v)[12], const Spinor
 // streaming it past L2 keeps the L2 for the neighbour spinors the current
 // kernel re-reads (the FP64 hopping matrix gains ~9% from this).  The 4- and
 // 8-byte stores of the reduced precisions measured slower non-temporal.
-template <class S, class VIn>
+template <class S, bool NT = true, class VIn>
 __device__ __forceinline__ void store_spinor(const SpinorPtr<S> &f, int i, int vh,
                                              const VIn (&v)[12]) {
   using V = typename S::V;
@@ -405,7 +405,7 @@ __device__ __forceinline__ void store_spinor(const SpinorPtr<S> &f, int i, int v
 #pragma unroll
     for (int q = 0; q < 3; q++) P[(size_t)q * vh + i] = u32x4{w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]};
 #endif
-  } else if constexpr (sizeof(typename S::ST) == 16) {
+  } else if constexpr (NT && sizeof(typename S::ST) == 16) {
 #pragma unroll
     for (int k = 0; k < 12; k++) S::st_nt(f.p, (size_t)k * vh + i, cmk<V>((A)v[k].x, (A)v[k].y));
   } else {
@@ -797,6 +797,24 @@ __device__ __forceinline__ void clover_raw_finish(V (&y)[6], const V (&x)[6], fl
   }
 }
 
+// y = A_J x for chiral block J of the clover field C: mode 0 = Hermitian
+// product, 1 = LDL^+ solve
+template <class SG, int MODE, int POL = kNT, class V>
+__device__ __forceinline__ void clover_block_apply(V (&y)[6], const V (&x)[6], const typename SG::ST *C,
+                                                   const float *Cn, int eo, int J, int i, int vh) {
+  constexpr bool kRaw = std::is_same<SG, SF16>::value;
+  static_assert(!kRaw || MODE == 0, "16-bit clover blocks hold A/2 or A^-1/2, not LDL factors");
+  typename SG::V w[18];
+  float2 mc;
+  if constexpr (kRaw) mc = load_clover_block_raw<POL>(w, C, Cn, eo, J, i, vh);
+  else load_clover_block<SG, POL>(w, C, Cn, eo, J, i, vh);
+  V ww[18];
+#pragma unroll
+  for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);
+  if constexpr (MODE == 0) herm6(y, ww, x); else ldl6(y, ww, x);
+  if constexpr (kRaw) clover_raw_finish(y, x, mc);
+}
+
 // out = A in (Dirac basis) with A stored as two chiral blocks of A/2
 // (clover_mult_a.F90:44-95); mode 0 = Hermitian product, 1 = LDL^+ solve.
 // SG is the clover storage policy, V the arithmetic complex type.
@@ -805,38 +823,16 @@ __device__ __forceinline__ void clover_apply(V (&out)[12], const V (&in)[12],
                                              const typename SG::ST *C, const float *Cn, int eo,
                                              int i, int vh) {
   V xp[6], y1[6], y2[6];
-  constexpr bool kRaw = std::is_same<SG, SF16>::value;
-  static_assert(!kRaw || MODE == 0, "16-bit clover blocks hold A/2 or A^-1/2, not LDL factors");
 #pragma unroll
   for (int m = 0; m < 6; m++) xp[m] = cadd(in[m], in[m + 6]);
-  {
-    typename SG::V w[18];
-    float2 mc;
-    if constexpr (kRaw) mc = load_clover_block_raw<POL>(w, C, Cn, eo, 0, i, vh);
-    else load_clover_block<SG, POL>(w, C, Cn, eo, 0, i, vh);
-    V ww[18];
-#pragma unroll
-    for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);
-    if constexpr (MODE == 0) herm6(y1, ww, xp); else ldl6(y1, ww, xp);
-    if constexpr (kRaw) clover_raw_finish(y1, xp, mc);
-  }
+  clover_block_apply<SG, MODE, POL>(y1, xp, C, Cn, eo, 0, i, vh);
   // finish block 0 before loading block 1 (bounds live registers)
 #pragma unroll
   for (int m = 0; m < 6; m++) asm volatile("" : "+v"(y1[m].x), "+v"(y1[m].y));
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int m = 0; m < 6; m++) xp[m] = csub(in[m], in[m + 6]);
-  {
-    typename SG::V w[18];
-    float2 mc;
-    if constexpr (kRaw) mc = load_clover_block_raw<POL>(w, C, Cn, eo, 1, i, vh);
-    else load_clover_block<SG, POL>(w, C, Cn, eo, 1, i, vh);
-    V ww[18];
-#pragma unroll
-    for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);
-    if constexpr (MODE == 0) herm6(y2, ww, xp); else ldl6(y2, ww, xp);
-    if constexpr (kRaw) clover_raw_finish(y2, xp, mc);
-  }
+  clover_block_apply<SG, MODE, POL>(y2, xp, C, Cn, eo, 1, i, vh);
 #pragma unroll
   for (int m = 0; m < 6; m++) {
     out[m] = cadd(y1[m], y2[m]);
