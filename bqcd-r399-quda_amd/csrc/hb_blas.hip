@@ -2,6 +2,8 @@
 // clover multiplies, and precision conversions of spinors, links and clover.
 #include "hb_blas.h"
 
+#include "hb_dslash.h"
+
 namespace hb {
 
 // ---------------------------------------------------------------------------
@@ -49,16 +51,6 @@ int clover_mult_f64(Context *c, int which, int eo, double2 *out, const double2 *
 // coalesced planes (component k of site i at k*vh + i).
 #define HB_SITE_LOOP for (int k = 0; k < 12; k++)
 #define HB_AT(ptr, k) (ptr)[(size_t)(k) * vh + i]
-// streaming (non-temporal) store of one complex number, see store_spinor
-#ifndef HB_CG_NT_STORE
-#define HB_CG_NT_STORE 1
-#endif
-#if HB_CG_NT_STORE
-#define HB_ST(ptr, k, v) SF64::st_nt((ptr), (size_t)(k) * vh + i, (v))
-#else
-#define HB_ST(ptr, k, v) ((ptr)[(size_t)(k) * vh + i] = (v))
-#endif
-
 // r = b - r, p = r, rtr_old = |r|^2  (cg.F90:84-89)
 __global__ __launch_bounds__(kBlock) void k_cg_start(double2 *__restrict__ r, double2 *__restrict__ p,
                                                      const double2 *__restrict__ b, int vh,
@@ -79,46 +71,61 @@ __global__ __launch_bounds__(kBlock) void k_cg_start(double2 *__restrict__ r, do
   block_partials<1>(vals, partials);
 }
 
+// The updates of an iteration have one thread per complex number, not per
+// site: small lattices have too few sites to fill the chip.  NT: the results
+// are streamed past the caches, as the hopping kernels' (store_spinor).
+template <bool NT> __device__ __forceinline__ void st_cg(double2 *p, int i, double2 v) {
+  if constexpr (NT) SF64::st_nt(p, i, v);
+  else p[i] = v;
+}
 // alpha = rtr_old / pAp; r -= alpha q; rtr = |r|^2 (cg.F90:96-109).  The
 // x update of the same iteration is done by k_cg_pupdate, which reads p anyway.
-__global__ __launch_bounds__(kBlock) void k_cg_update(double2 *__restrict__ r, const double2 *__restrict__ q,
-                                                      int vh, const CgState *st, double *partials) {
-  if (st->done) return;
-  const double alpha = st->rtr_old / st->pap;
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+template <bool NT>
+__global__ __launch_bounds__(kBlock) void k_cg_update(double2 *__restrict__ r, const double2 *__restrict__ q, int n,
+                                                      CgState *st, int k, const double *pa, int na, double *pb) {
+  const CgSlot c = st->s[k & 1];
+  if (c.done) return;
+  const double pap = partials_total(pa, na);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->pap = pap;
+  const double alpha = c.rtr / pap;
   double s = 0.0;
-  if (i < vh) {
-#pragma unroll
-    HB_SITE_LOOP {
-      double2 qq = HB_AT(q, k), rr = HB_AT(r, k);
-      rr.x -= alpha * qq.x; rr.y -= alpha * qq.y;
-      HB_ST(r, k, rr);
-      s += rr.x * rr.x + rr.y * rr.y;
-    }
+#pragma unroll 4
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    double2 qq = q[i], rr = r[i];
+    rr.x -= alpha * qq.x; rr.y -= alpha * qq.y;
+    st_cg<NT>(r, i, rr);
+    s += rr.x * rr.x + rr.y * rr.y;
   }
   double vals[1] = {s};
-  block_partials<1>(vals, partials);
+  block_partials<1>(vals, pb);
 }
 
-// x += alpha p of the iteration just finished (cg.F90:97-98), then, unless the
-// solve has ended, p = r + beta p (sc_xpby, sc.F90:184-201); the same
-// arithmetic on the same values as updating x beside r
+// x += alpha p of the iteration just finished (cg.F90:97-98), the stop test
+// (cg.F90:111) and, unless the solve has ended, p = r + beta p (sc_xpby,
+// sc.F90:184-201)
+template <bool NT>
 __global__ __launch_bounds__(kBlock) void k_cg_pupdate(double2 *__restrict__ x, double2 *__restrict__ p,
-                                                       const double2 *__restrict__ r, int vh,
-                                                       const CgState *st) {
-  if (!st->xpend) return;
-  const double alpha = st->alpha, beta = st->beta;
-  const bool next = st->done == 0;
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
-#pragma unroll
-  HB_SITE_LOOP {
-    double2 pp = HB_AT(p, k), xx = HB_AT(x, k);
+                                                       const double2 *__restrict__ r, int n, CgState *st, int k,
+                                                       const double *pb, int nb) {
+  const CgSlot c = st->s[k & 1];
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (c.done) {
+    if (first) st->s[~k & 1] = c;
+    return;
+  }
+  const double rtr = partials_total(pb, nb);
+  const double alpha = c.rtr / st->pap, beta = rtr / c.rtr;
+  const int iter = c.iter + 1;
+  const int done = rtr <= st->rest ? 1 : iter >= st->maxiter ? 2 : 0;
+  if (first) st->s[~k & 1] = CgSlot{done ? c.rtr : rtr, rtr, iter, done};
+#pragma unroll 4
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    double2 pp = p[i], xx = x[i];
     xx.x += alpha * pp.x; xx.y += alpha * pp.y;
-    HB_ST(x, k, xx);
-    if (next) {
-      double2 rr = HB_AT(r, k);
-      HB_ST(p, k, make_double2(rr.x + beta * pp.x, rr.y + beta * pp.y));
+    st_cg<NT>(x, i, xx);
+    if (!done) {
+      double2 rr = r[i];
+      st_cg<NT>(p, i, make_double2(rr.x + beta * pp.x, rr.y + beta * pp.y));
     }
   }
 }
@@ -171,12 +178,6 @@ __global__ void k_copy(double2 *__restrict__ d, const double2 *__restrict__ s, s
   for (size_t k = i; k < n; k += (size_t)gridDim.x * blockDim.x) d[k] = s[k];
 }
 
-int reduce_grid(const Context *c, int n) {
-  int b = nblocks(n);
-  int cap = c->red_blocks;
-  return b < cap ? b : cap;
-}
-
 // every field of the CG state cleared, then the stopping bound and maxiter
 __global__ void k_cg_init(CgState *st, double rest, int maxiter) {
   if (threadIdx.x == 0) {
@@ -202,18 +203,28 @@ int cg_start(Context *c, double2 *r, double2 *p, const double2 *b, CgState *st, 
   return HB_OK;
 }
 
-int cg_update(Context *c, double2 *r, const double2 *q, CgState *st, double *red) {
-  const int vh = c->g.vh, grid = nblocks(vh);
-  if (!red) red = c->red;
-  k_cg_update<<<grid, kBlock, 0, c->stream>>>(r, q, vh, st, red);
-  k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(red, grid, nullptr, FinCgUpdate{st});
+int shorten_partials(Context *c, const double *&p, int &n, const int *skip) {
+  if (n <= kMaxParts) return HB_OK;
+  double *out = const_cast<double *>(p) + n;
+  k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(p, n, skip, FinStore1{out});
+  HB_HIP(hipGetLastError());
+  p = out;
+  n = 1;
+  return HB_OK;
+}
+
+int cg_update(Context *c, double2 *r, const double2 *q, CgState *st, int k, const double *pa, int na, double *pb) {
+  const int vh = c->g.vh;
+  const auto f = operator_policy<SF64, SF64R>(vh) == kNT ? k_cg_update<true> : k_cg_update<false>;
+  f<<<vector_grid(vh), kBlock, 0, c->stream>>>(r, q, 12 * vh, st, k, pa, na, pb);
   HB_HIP(hipGetLastError());
   return HB_OK;
 }
 
-int cg_pupdate(Context *c, double2 *x, double2 *p, const double2 *r, const CgState *st) {
+int cg_pupdate(Context *c, double2 *x, double2 *p, const double2 *r, CgState *st, int k, const double *pb) {
   const int vh = c->g.vh;
-  k_cg_pupdate<<<nblocks(vh), kBlock, 0, c->stream>>>(x, p, r, vh, st);
+  const auto f = operator_policy<SF64, SF64R>(vh) == kNT ? k_cg_pupdate<true> : k_cg_pupdate<false>;
+  f<<<vector_grid(vh), kBlock, 0, c->stream>>>(x, p, r, 12 * vh, st, k, pb, vector_grid(vh));
   HB_HIP(hipGetLastError());
   return HB_OK;
 }

@@ -25,12 +25,11 @@ DslashArgs<SF64> dslash_args64(Context *c, int out_parity, double2 *out, const d
 
 // half of M~ (or M~^+): t = A_oo^-1 D_oe in ; out = A_ee in - kappa^2 D_eo t + rho in
 // (m_tilde.F90:61-71 / :98-108 with w_mult.F90's sc_axpy folded in).  With
-// dot_out set, also Re<dotv, out> (sc_dot) in the same pass.  G = SF64 reads
+// dot set, also the partial sums of Re<dotv, out> (sc_dot) in the same pass.  G = SF64 reads
 // all 18 reals of each link, G = SF64R the two-row copy U (row 2 rebuilt).
 template <class G>
 int mtil_f64_g(Context *c, const typename G::ST *U, bool dag, double kappa, double rho, double2 *out,
-               const double2 *in, double2 *t, double *dot_out, const double2 *dotv, const int *skip,
-               double *red) {
+               const double2 *in, double2 *t, double *dot, const double2 *dotv, const int *skip) {
   const bool clov = use_clover(c);
   DslashArgs<SF64, G> a1{};
   a1.g = c->g;
@@ -51,10 +50,9 @@ int mtil_f64_g(Context *c, const typename G::ST *U, bool dag, double kappa, doub
   a2.mkappa2 = -kappa * kappa;
   a2.rho = rho;
   a2.skip = skip;
-  if (dot_out) {
+  if (dot) {
     a2.dotv = {const_cast<double2 *>(dotv), nullptr};
-    a2.dot_out = dot_out;
-    if (red) a2.partials = red;
+    a2.partials = dot;
     HB_TRY(launch_dslash(a2, dag, EPI_MTDOT, c->stream));
   } else {
     HB_TRY(launch_dslash(a2, dag, EPI_MTIL, c->stream));
@@ -63,10 +61,10 @@ int mtil_f64_g(Context *c, const typename G::ST *U, bool dag, double kappa, doub
 }
 
 int mtil_f64(Context *c, bool dag, double kappa, double rho, double2 *out, const double2 *in,
-             double2 *t, double *dot_out, const double2 *dotv, const int *skip, double *red, bool recon) {
+             double2 *t, double *dot, const double2 *dotv, const int *skip, bool recon) {
   if (recon)
-    return mtil_f64_g<SF64R>(c, c->gauge64r, dag, kappa, rho, out, in, t, dot_out, dotv, skip, red);
-  return mtil_f64_g<SF64>(c, c->gauge, dag, kappa, rho, out, in, t, dot_out, dotv, skip, red);
+    return mtil_f64_g<SF64R>(c, c->gauge64r, dag, kappa, rho, out, in, t, dot, dotv, skip);
+  return mtil_f64_g<SF64>(c, c->gauge, dag, kappa, rho, out, in, t, dot, dotv, skip);
 }
 
 // rows 0 and 1 of the FP64 links; the largest |row 2 - conj(row0 x row1)| of
@@ -126,17 +124,17 @@ int ensure_links_two_rows(Context *c, bool *use) {
 }
 
 int apply_f64(Context *c, int op, double kappa, double rho, double2 *out, const double2 *in,
-              double2 *t, double2 *y, double *dot_out, const int *skip, double *red, bool recon) {
+              double2 *t, double2 *y, double *dot, const int *skip, bool recon) {
   switch (op) {
-    case HB_OP_MTIL: return mtil_f64(c, false, kappa, 0.0, out, in, t, nullptr, nullptr, skip, nullptr, recon);
-    case HB_OP_MTIL_DAG: return mtil_f64(c, true, kappa, 0.0, out, in, t, nullptr, nullptr, skip, nullptr, recon);
-    case HB_OP_W: return mtil_f64(c, false, kappa, rho, out, in, t, nullptr, nullptr, skip, nullptr, recon);
-    case HB_OP_W_DAG: return mtil_f64(c, true, kappa, rho, out, in, t, nullptr, nullptr, skip, nullptr, recon);
+    case HB_OP_MTIL: return mtil_f64(c, false, kappa, 0.0, out, in, t, nullptr, nullptr, skip, recon);
+    case HB_OP_MTIL_DAG: return mtil_f64(c, true, kappa, 0.0, out, in, t, nullptr, nullptr, skip, recon);
+    case HB_OP_W: return mtil_f64(c, false, kappa, rho, out, in, t, nullptr, nullptr, skip, recon);
+    case HB_OP_W_DAG: return mtil_f64(c, true, kappa, rho, out, in, t, nullptr, nullptr, skip, recon);
     case HB_OP_MTDAGMT:
     case HB_OP_WDAGW: {
       double r = op == HB_OP_WDAGW ? rho : 0.0;
-      HB_TRY(mtil_f64(c, false, kappa, r, y, in, t, nullptr, nullptr, skip, nullptr, recon));
-      return mtil_f64(c, true, kappa, r, out, y, t, dot_out, in, skip, red, recon);
+      HB_TRY(mtil_f64(c, false, kappa, r, y, in, t, nullptr, nullptr, skip, recon));
+      return mtil_f64(c, true, kappa, r, out, y, t, dot, in, skip, recon);
     }
   }
   set_error("unknown operator %d", op);
@@ -167,34 +165,39 @@ int cg_f64_run(Context *c, const CgWork &w, int op, double kappa, double rho, do
   CgState *st = w.st, *hs = w.hs;
   HB_TRY(cg_init(c, st, (double)rest, maxiter));
   // r = A x; r = b - r; p = r; rtr_old = |r|^2
-  HB_TRY(apply_f64(c, op, kappa, rho, w.r, x, w.t, w.y, nullptr, nullptr, nullptr, w.recon));
+  HB_TRY(apply_f64(c, op, kappa, rho, w.r, x, w.t, w.y, nullptr, nullptr, w.recon));
   HB_TRY(cg_start(c, w.r, w.p, b, st, w.red));
-  int *skip = &st->done;
   int nmv = 1;
   if (maxiter == 0) {
     // the reference's loop body never runs: niter = 0, x unchanged
     HB_HIP(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
     HB_HIP(hipStreamSynchronize(c->stream));
   } else {
-    // iterations in chunks; every kernel returns immediately once done != 0, so
-    // the chunk length only sets how often the host looks at the state
+    // iterations in chunks (of even length, so that each ends in slot 0); every
+    // kernel returns immediately once done != 0, so the chunk length only sets
+    // how often the host looks at the state
+    const int na = w.recon ? dslash_grid<SF64, SF64R>(c->g.vh) : dslash_grid<SF64, SF64>(c->g.vh);
+    double *pa = w.red, *pb = w.red + na + 1;
     int chunk = 8;
     for (;;) {
       for (int k = 0; k < chunk; k++) {
-        HB_TRY(apply_f64(c, op, kappa, rho, w.q, w.p, w.t, w.y, &st->pap, skip, w.red, w.recon));
-        HB_TRY(cg_update(c, w.r, w.q, st, w.red));
-        HB_TRY(cg_pupdate(c, x, w.p, w.r, st));
+        HB_TRY(apply_f64(c, op, kappa, rho, w.q, w.p, w.t, w.y, pa, &st->s[k & 1].done, w.recon));
+        const double *sum = pa;
+        int nsum = na;
+        HB_TRY(shorten_partials(c, sum, nsum, &st->s[k & 1].done));
+        HB_TRY(cg_update(c, w.r, w.q, st, k, sum, nsum, pb));
+        HB_TRY(cg_pupdate(c, x, w.p, w.r, st, k, pb));
       }
       HB_HIP(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
       HB_HIP(hipStreamSynchronize(c->stream));
-      if (hs->done) break;
+      if (hs->s[0].done) break;
       if (chunk < 64) chunk *= 2;
     }
-    nmv += hs->iter;
+    nmv += hs->s[0].iter;
   }
-  const int niter = hs->iter;
-  const int done = hs->done;
-  const double rtr = hs->rtr;
+  const int niter = hs->s[0].iter;
+  const int done = hs->s[0].done;
+  const double rtr = hs->s[0].last;
   // true residual |b - A x|^2 in FP64 (invert_quda.F90:155-168), with all
   // 18 reals of each link
   HB_TRY(apply_f64(c, op, kappa, rho, w.q, x, w.t, w.y, nullptr, nullptr));

@@ -20,21 +20,21 @@ template <class S, class G = S> struct DslashArgs {
   SpinorPtr<S> dotv;         // MTDOT: Re<dotv, out>
   double mkappa2;            // -kappa^2
   double rho;
-  double *dot_out;           // MTDOT result (device)
-  double *partials;          // MTDOT per-block partial sums (gridDim doubles)
+  double *partials;          // MTDOT: per-workgroup partial sums (dslash_grid doubles)
   const int *skip;           // if non-null and *skip != 0 the launch does nothing
 };
 
 // Load policy of the links and clover words, which a kernel reads once: kept
-// in the caches while the operator and the vectors of a solve fit the 256 MB
-// last-level cache, streamed past them (so that the neighbour spinors stay)
-// when they do not.  CG iteration streamed / kept:
-//   FP64    12^3x24 (50 MB) 96.6 / 79.5 us, 16^3x32 (157 MB) 130 / 116 us,
-//           24^3x48 (796 MB) 605 / 666 us
-//   FP32    14x20x12x30 (63 MB) 88.1 / 77.5 us, 24^3x48 (414 MB) 363 / 373 us
-//   16-bit  24^3x48 (235 MB) 218 / 208 us, 32^3x64 (742 MB) 522 / 584 us
-//           two right-hand sides at 24^3x48 (353 MB) 340 / 352 us
-constexpr size_t kResidentBytes = (size_t)1 << 28;
+// in the caches while the operator and the vectors of a solve are up to half
+// as large again as the 256 MB last-level cache, streamed past them (so that
+// the neighbour spinors stay) beyond.  CG iteration streamed / kept:
+//   FP64    12^3x24 (62 MB) 96.6 / 79.5 us, 16^3x32 (195 MB) 130 / 116 us,
+//           24^3x48 (987 MB) 605 / 666 us
+//   FP32    14x20x12x30 (77 MB) 88.1 / 77.5 us, 24^3x48 (510 MB) 356 / 361 us
+//   16-bit  24^3x48 (288 MB) 219 / 200 us, 32^3x64 (910 MB) 522 / 584 us;
+//           two right-hand sides at 24^3x48 (406 MB) 340 / 352 us
+//   FP32 spinors, 16-bit links and clover: 24^3x48 (361 MB) 273 / 263 us
+constexpr size_t kResidentBytes = (size_t)360 << 20;
 template <class S, class G> constexpr size_t solve_bytes_per_site(int nr = 1) {
   const size_t link = std::is_same<G, SF16>::value ? 24 : G::kRecon ? 6 * G::kBytes : 9 * G::kBytes;
   const size_t clov = std::is_same<G, SF16>::value ? 2 * kClov16 : 36 * G::kBytes;
@@ -43,6 +43,27 @@ template <class S, class G> constexpr size_t solve_bytes_per_site(int nr = 1) {
 }
 template <class S, class G> inline int operator_policy(int vh, int nr = 1) {
   return solve_bytes_per_site<S, G>(nr) * (size_t)vh <= kResidentBytes ? 0 : kNT;
+}
+
+// Waves that share a site (1: k_dslash, else k_dslash_split), which sets the
+// number of workgroups of a launch and of the partial sums it leaves
+// (EPI_MTDOT).  us per CG iteration at 1 / 2 / 4 waves:
+//   FP64    8^4 (2 k sites per parity) 58.9 / 47.1 / 45.0, 12^3x24 (21 k)
+//           80.3 / 61.5 / 58.4, 16^4 (33 k) 85.4 / 69.0 / 69.2,
+//           16x16x18x18 (41 k) 91.3 / 79.4 / 89.8, 16^3x32 (66 k) 117 / 112 / 112;
+//           M~^+M~ with 18-real links 41 k 66.8 / 63.4 / 68.8, 50 k 74.2 / 80.2 / 82.1
+//   FP32    12^3x24 70.7 / 58.7 / 57.6, 16^4 69.5 / 61.5 / 59.4, 50 k 77.0 / 71.1 /
+//           72.2, 24^3x48 (332 k) 365 / 356 / 358, 32^3x64 1010 / 1056 / 1067
+//   16-bit  12^3x24 60.9 / 55.4 / 52.2, 50 k 62.9 / 58.7 / 60.6, 24^3x48
+//           207 / 200 / 214, 32^3x64 522 / 548 / 580
+// Eight waves (one hop each) were slower than four from 4 k sites on.
+template <class S, class G> inline int split_waves(int vh) {
+  if (vh <= (1 << 15)) return 4;
+  constexpr int two = !std::is_same<S, SF64>::value ? 1 << 19 : G::kRecon ? 1 << 16 : 3 << 14;
+  return vh <= two ? 2 : 1;
+}
+template <class S, class G> inline int dslash_grid(int vh) {
+  return nblocks(vh, split_waves<S, G>(vh) > 1 ? 64 : kBlock);
 }
 
 template <class S, class G> int launch_dslash(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st);

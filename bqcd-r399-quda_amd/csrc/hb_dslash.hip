@@ -12,7 +12,7 @@
 //   EPI_PLAIN  out = D in
 //   EPI_CLINV  out = A^-1 (D in)                      (clover_mult_ao on conf%i)
 //   EPI_MTIL   out = A x0 - kappa^2 (D in) + rho x0   (clover_mult_a + sc_xpby + sc_axpy)
-//   EPI_MTDOT  EPI_MTIL and a grid reduction of Re<v, out> (sc_dot), single pass
+//   EPI_MTDOT  EPI_MTIL and the partial sums of Re<v, out> (sc_dot) per workgroup
 #include "hb_dslash.h"
 #include "hb_hop.h"
 
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(64 * NW) void k_dslash_split(DslashArgs<S, G> a) {
 
 template <class S, class G, int NW, int POL>
 static void launch_split(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
-  dim3 grid(nblocks(a.g.vh, 64)), block(64 * NW);
+  dim3 grid(dslash_grid<S, G>(a.g.vh)), block(64 * NW);
 #define HB_DS(D, E) hipLaunchKernelGGL((k_dslash_split<S, G, D, E, NW, POL>), grid, block, 0, st, a)
   if (!dag) {
     switch (epi) {
@@ -221,7 +221,7 @@ static void launch_split(const DslashArgs<S, G> &a, bool dag, int epi, hipStream
 
 template <class S, class G, int POL>
 static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
-  dim3 grid(nblocks(a.g.vh)), block(kBlock);
+  dim3 grid(dslash_grid<S, G>(a.g.vh)), block(kBlock);
 #define HB_DS(D, E) hipLaunchKernelGGL((k_dslash<S, G, D, E, POL>), grid, block, 0, st, a)
   if (!dag) {
     switch (epi) {
@@ -241,22 +241,6 @@ static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t
 #undef HB_DS
 }
 
-// Waves that share a site (1: k_dslash).  us per CG iteration at 1 / 2 / 4:
-//   FP64    8^4 (2 k sites per parity) 58.9 / 47.1 / 45.0, 12^3x24 (21 k)
-//           80.3 / 61.5 / 58.4, 16^4 (33 k) 85.4 / 69.0 / 69.2,
-//           16x16x18x18 (41 k) 91.3 / 79.4 / 89.8, 16^3x32 (66 k) 117 / 112 / 112;
-//           M~^+M~ with 18-real links 41 k 66.8 / 63.4 / 68.8, 50 k 74.2 / 80.2 / 82.1
-//   FP32    12^3x24 70.7 / 58.7 / 57.6, 16^4 69.5 / 61.5 / 59.4, 50 k 77.0 / 71.1 /
-//           72.2, 24^3x48 (332 k) 365 / 356 / 358, 32^3x64 1010 / 1056 / 1067
-//   16-bit  12^3x24 60.9 / 55.4 / 52.2, 50 k 62.9 / 58.7 / 60.6, 24^3x48
-//           207 / 200 / 214, 32^3x64 522 / 548 / 580
-// Eight waves (one hop each) were slower than four from 4 k sites on.
-template <class S, class G> static int split_waves(int vh) {
-  if (vh <= (1 << 15)) return 4;
-  constexpr int two = !std::is_same<S, SF64>::value ? 1 << 19 : G::kRecon ? 1 << 16 : 3 << 14;
-  return vh <= two ? 2 : 1;
-}
-
 template <class S, class G>
 int launch_dslash(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
   const int nw = split_waves<S, G>(a.g.vh), pol = operator_policy<S, G>(a.g.vh);
@@ -269,9 +253,6 @@ int launch_dslash(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) 
     if (pol == kNT) launch_pol<S, G, kNT>(a, dag, epi, st);
     else launch_pol<S, G, 0>(a, dag, epi, st);
   }
-  if (epi == EPI_MTDOT)
-    k_finalize<1><<<1, kFinThreads, 0, st>>>(a.partials, nblocks(a.g.vh, nw > 1 ? 64 : kBlock), a.skip,
-                                             FinStore1{a.dot_out});
   HB_HIP(hipGetLastError());
   return HB_OK;
 }

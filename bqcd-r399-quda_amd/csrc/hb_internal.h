@@ -299,6 +299,29 @@ __device__ __forceinline__ void block_partials(const double (&v)[NV], double *pa
   }
 }
 
+// The sum of n partials, formed by every block of the kernel that needs it
+// (fixed order, the same in all blocks): at n <= kMaxParts this costs each
+// block about a microsecond of L2 reads and saves the one-block launch between
+// two kernels of an iteration.  Valid in all threads.
+constexpr int kMaxParts = 2048;
+__device__ __forceinline__ double partials_total(const double *__restrict__ p, int n) {
+  __shared__ double lds[16];
+  double a[4] = {0.0, 0.0, 0.0, 0.0};
+  int b = threadIdx.x;
+  const int step = blockDim.x;
+  for (; b + 3 * step < n; b += 4 * step) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) a[u] += p[b + u * step];
+  }
+  for (; b < n; b += step) a[0] += p[b];
+  const double s = wave_sum((a[0] + a[1]) + (a[2] + a[3]));
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
+  __syncthreads();
+  double t = 0.0;
+  for (int w = 0; w < ((int)blockDim.x + 63) >> 6; w++) t += lds[w];
+  return t;
+}
+
 // one block: sums nparts partials per value (fixed order) and calls f(sums)
 // from thread 0; `skip` gates it like the producing kernel.  1024 threads
 // with four independent loads in flight each: the partials come from L2, and

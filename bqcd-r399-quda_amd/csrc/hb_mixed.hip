@@ -16,14 +16,19 @@
 
 namespace hb {
 
+// The scalars of an iteration, in two slots as those of the FP64 CG (CgState).
+struct MixSlot {
+  double rtr, maxr;  // iterated |r|^2; largest |r| since the last reliable update
+  int iter, since;
+  int flag;          // 0 iterate, 1 reliable update due, 2 converged, 3 maxiter reached
+};
 struct MixState {
-  double rtr, rtr_new, pap, beta, maxr;
-  double alpha;  // of the last iteration, for the x_lo update
-  int xpend;     // the last launched iteration ran: its x_lo update is due
+  MixSlot s[2];
+  double pap;           // <p, A p> of the iteration, from the r update for the p update
+  double beta;          // of the restart after a reliable update
   double rp_re, rp_im;  // <r, p> / |r|^2 after a reliable update
   double rest, delta;
-  int iter, since, max_inner, maxiter;
-  int flag;      // 0 iterate, 1 reliable update due, 2 converged, 3 maxiter reached
+  int max_inner, maxiter;
   int n_reliable;
   double res[4];
 };
@@ -95,89 +100,114 @@ __global__ void k_spinor_to_f64(double2 *__restrict__ dst, SpinorPtr<S> src, int
 // inner solver).  The update x_lo += alpha p happens in the p update, which
 // reads p anyway.
 
-// alpha = rtr / pAp; r -= alpha q; rtr_new = |r|^2
-template <class S, class R>
-__global__ __launch_bounds__(kBlock) void k_mix_update(SpinorPtr<R> r, SpinorPtr<S> q, int vh,
-                                                       const MixState *st, double *partials) {
-  using V = typename S::V;
-  if (st->flag) return;
-  const float alpha = (float)(st->rtr / st->pap);
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double s = 0.0;
-  if (i < vh) {
-    V qv[12], rv[12];
-    load_spinor<S>(qv, q, i, vh);
-    load_spinor<R>(rv, r, i, vh);
-#pragma unroll
-    for (int k = 0; k < 12; k++) {
-      rv[k].x -= alpha * qv[k].x;
-      rv[k].y -= alpha * qv[k].y;
-      s += (double)rv[k].x * rv[k].x + (double)rv[k].y * rv[k].y;
-    }
-    store_spinor<R>(r, i, vh, rv);
-  }
-  double vals[1] = {s};
-  block_partials<1>(vals, partials);
+//
+// Fields without a scale per site are updated one complex number per thread,
+// 16-bit fields one site per thread; n counts what a thread works on.
+template <class S> constexpr bool kLinear = !S::kNorm;
+template <class S> inline int mix_count(int vh) { return kLinear<S> ? 12 * vh : vh; }
+template <class S> inline int mix_block(int vh) { return !kLinear<S> && vh <= (1 << 16) ? 64 : kBlock; }
+template <class S> inline int mix_grid(int vh) {
+  const int b = nblocks(mix_count<S>(vh), mix_block<S>(vh));
+  return b < 2048 ? b : 2048;
 }
 
-// iterated |r|^2 -> reliable-update decision or beta (cg.F90:109-115)
-// (launched unconditionally: after a skipped update it only clears xpend, so
-// that the p update of a skipped iteration adds nothing to x_lo)
-struct FinMixUpdate {
-  MixState *st;
-  __device__ void operator()(const double (&t)[1]) const {
-    if (st->flag) {
-      st->xpend = 0;
-      return;
-    }
-    st->alpha = st->rtr / st->pap;  // the alpha of k_mix_update
-    st->xpend = 1;
-    const double rn = t[0];
-    st->iter += 1;
-    st->since += 1;
-    st->rtr_new = rn;
-    const double rnorm = sqrt(rn);
-    if (rnorm > st->maxr) st->maxr = rnorm;
-    if (rn <= st->rest || rnorm < st->delta * st->maxr || st->since >= st->max_inner ||
-        st->iter >= st->maxiter) {
-      st->flag = 1;
-    } else {
-      st->beta = rn / st->rtr;
-      st->rtr = rn;
-    }
-  }
-};
-
-// x_lo += alpha p (every iteration that ran), then p = r + beta p (unless a
-// reliable update or the end is due)
-template <class S, class R>
-__global__ __launch_bounds__(kBlock) void k_mix_pupdate(SpinorPtr<S> p, SpinorPtr<R> r, float2 *__restrict__ xlo,
-                                                        int vh, const MixState *st) {
+// alpha = rtr / pAp; r -= alpha q; partial sums of |r|^2
+template <class S>
+__global__ __launch_bounds__(kBlock) void k_mix_update(SpinorPtr<S> r, SpinorPtr<S> q, int n, MixState *st, int k,
+                                                       const double *pa, int na, double *pb) {
   using V = typename S::V;
-  if (!st->xpend) return;
-  const float alpha = (float)st->alpha;
-  const float beta = (float)st->beta;
-  const bool next = st->flag == 0;
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
-  V pv[12];
-  load_spinor<S>(pv, p, i, vh);
+  const MixSlot c = st->s[k & 1];
+  if (c.flag) return;
+  const double pap = partials_total(pa, na);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->pap = pap;
+  const float alpha = (float)(c.rtr / pap);
+  double s = 0.0;
+#pragma unroll(kLinear<S> ? 4 : 1)
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    if constexpr (kLinear<S>) {
+      const V qv = S::ld(q.p, i);
+      V rv = S::ld(r.p, i);
+      rv.x -= alpha * qv.x;
+      rv.y -= alpha * qv.y;
+      s += (double)rv.x * rv.x + (double)rv.y * rv.y;
+      S::st(r.p, i, rv);
+    } else {
+      V qv[12], rv[12];
+      load_spinor<S>(qv, q, i, n);
+      load_spinor<S>(rv, r, i, n);
 #pragma unroll
-  for (int k = 0; k < 12; k++) {
-    float2 xv = xlo[(size_t)k * vh + i];
-    xv.x += alpha * pv[k].x;
-    xv.y += alpha * pv[k].y;
-    xlo[(size_t)k * vh + i] = xv;
-  }
-  if (next) {
-    V rv[12];
-    load_spinor<R>(rv, r, i, vh);
-#pragma unroll
-    for (int k = 0; k < 12; k++) {
-      pv[k].x = rv[k].x + beta * pv[k].x;
-      pv[k].y = rv[k].y + beta * pv[k].y;
+      for (int k = 0; k < 12; k++) {
+        rv[k].x -= alpha * qv[k].x;
+        rv[k].y -= alpha * qv[k].y;
+        s += (double)rv[k].x * rv[k].x + (double)rv[k].y * rv[k].y;
+      }
+      store_spinor<S>(r, i, n, rv);
     }
-    store_spinor<S>(p, i, vh, pv);
+  }
+  double vals[1] = {s};
+  block_partials<1>(vals, pb);
+}
+
+// iterated |r|^2 -> reliable-update decision or beta (cg.F90:109-115);
+// x_lo += alpha p, then p = r + beta p (unless a reliable update or the end is
+// due)
+template <class S>
+__global__ __launch_bounds__(kBlock) void k_mix_pupdate(SpinorPtr<S> p, SpinorPtr<S> r, float2 *__restrict__ xlo, int n,
+                                                        MixState *st, int k, const double *pb, int nb) {
+  using V = typename S::V;
+  const MixSlot c = st->s[k & 1];
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (c.flag) {
+    if (first) st->s[~k & 1] = c;
+    return;
+  }
+  const double rn = partials_total(pb, nb);
+  const double rnorm = sqrt(rn);
+  MixSlot d = c;
+  d.iter += 1;
+  d.since += 1;
+  if (rnorm > d.maxr) d.maxr = rnorm;
+  const bool next = !(rn <= st->rest || rnorm < st->delta * d.maxr || d.since >= st->max_inner || d.iter >= st->maxiter);
+  if (next) d.rtr = rn;
+  else d.flag = 1;
+  const float alpha = (float)(c.rtr / st->pap);
+  const float beta = (float)(rn / c.rtr);
+  if (first) st->s[~k & 1] = d;
+#pragma unroll(kLinear<S> ? 4 : 1)
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    if constexpr (kLinear<S>) {
+      V pv = S::ld(p.p, i);
+      float2 xv = xlo[i];
+      xv.x += alpha * pv.x;
+      xv.y += alpha * pv.y;
+      xlo[i] = xv;
+      if (next) {
+        const V rv = S::ld(r.p, i);
+        pv.x = rv.x + beta * pv.x;
+        pv.y = rv.y + beta * pv.y;
+        S::st(p.p, i, pv);
+      }
+    } else {
+      V pv[12];
+      load_spinor<S>(pv, p, i, n);
+#pragma unroll
+      for (int k = 0; k < 12; k++) {
+        float2 xv = xlo[(size_t)k * n + i];
+        xv.x += alpha * pv[k].x;
+        xv.y += alpha * pv[k].y;
+        xlo[(size_t)k * n + i] = xv;
+      }
+      if (next) {
+        V rv[12];
+        load_spinor<S>(rv, r, i, n);
+#pragma unroll
+        for (int k = 0; k < 12; k++) {
+          pv[k].x = rv[k].x + beta * pv[k].x;
+          pv[k].y = rv[k].y + beta * pv[k].y;
+        }
+        store_spinor<S>(p, i, n, pv);
+      }
+    }
   }
 }
 
@@ -194,10 +224,10 @@ __global__ void k_mix_accum(double2 *__restrict__ x, float2 *__restrict__ xlo, s
 }
 
 // r = b - Ax (in place in ax), |r|^2; then r_lo = r and the scalar bookkeeping
-template <class R>
+template <class S>
 __global__ __launch_bounds__(kBlock) void k_mix_true_residual(double2 *__restrict__ ax,
                                                               const double2 *__restrict__ b,
-                                                              SpinorPtr<R> rlo, int vh,
+                                                              SpinorPtr<S> rlo, int vh,
                                                               double *partials) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   double s = 0.0;
@@ -210,7 +240,7 @@ __global__ __launch_bounds__(kBlock) void k_mix_true_residual(double2 *__restric
       ax[(size_t)k * vh + i] = v[k];
       s += v[k].x * v[k].x + v[k].y * v[k].y;
     }
-    store_spinor<R>(rlo, i, vh, v);
+    store_spinor<S>(rlo, i, vh, v);
   }
   double vals[1] = {s};
   block_partials<1>(vals, partials);
@@ -222,19 +252,20 @@ struct FinMixTrue {
   int first;
   __device__ void operator()(const double (&t)[1]) const {
     const double rt = t[0];
+    MixSlot &c = st->s[0];
     st->res[0] = rt;
     if (!first) st->n_reliable += 1;
-    st->since = 0;
-    st->maxr = sqrt(rt);
+    c.since = 0;
+    c.maxr = sqrt(rt);
     if (rt <= st->rest) {
-      st->flag = 2;
-    } else if (st->iter >= st->maxiter) {
-      st->flag = 3;
+      c.flag = 2;
+    } else if (c.iter >= st->maxiter) {
+      c.flag = 3;
     } else {
       // the true residual replaces the iterated one; the search direction is kept
-      st->beta = first ? 0.0 : rt / st->rtr;
-      st->rtr = rt;
-      st->flag = 0;
+      st->beta = first ? 0.0 : rt / c.rtr;
+      c.rtr = rt;
+      c.flag = 0;
     }
   }
 };
@@ -247,17 +278,17 @@ struct FinMixTrue {
 #ifndef HB_MIX_REORTH
 #define HB_MIX_REORTH 1
 #endif
-template <class S, class R>
-__global__ __launch_bounds__(kBlock) void k_mix_rdotp(SpinorPtr<S> p, SpinorPtr<R> r, int vh, const MixState *st,
+template <class S>
+__global__ __launch_bounds__(kBlock) void k_mix_rdotp(SpinorPtr<S> p, SpinorPtr<S> r, int vh, const MixState *st,
                                                       double *partials) {
   using V = typename S::V;
-  if (st->flag) return;
+  if (st->s[0].flag) return;
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   double re = 0.0, im = 0.0;
   if (i < vh) {
     V pv[12], rv[12];
     load_spinor<S>(pv, p, i, vh);
-    load_spinor<R>(rv, r, i, vh);
+    load_spinor<S>(rv, r, i, vh);
 #pragma unroll
     for (int k = 0; k < 12; k++) {  // conj(r) p
       re += (double)rv[k].x * pv[k].x + (double)rv[k].y * pv[k].y;
@@ -271,24 +302,24 @@ __global__ __launch_bounds__(kBlock) void k_mix_rdotp(SpinorPtr<S> p, SpinorPtr<
 struct FinMixRdotp {
   MixState *st;
   __device__ void operator()(const double (&t)[2]) const {
-    st->rp_re = t[0] / st->rtr;
-    st->rp_im = t[1] / st->rtr;
+    st->rp_re = t[0] / st->s[0].rtr;
+    st->rp_im = t[1] / st->s[0].rtr;
   }
 };
 
 // p = r_lo + beta (p - rp r_lo) after a reliable update (rp = <r, p>/|r|^2, or
 // 0; beta = 0 at the start: p = r)
-template <class S, class R>
-__global__ __launch_bounds__(kBlock) void k_mix_prestart(SpinorPtr<S> p, SpinorPtr<R> r, int vh,
+template <class S>
+__global__ __launch_bounds__(kBlock) void k_mix_prestart(SpinorPtr<S> p, SpinorPtr<S> r, int vh,
                                                          const MixState *st) {
   using V = typename S::V;
-  if (st->flag) return;
+  if (st->s[0].flag) return;
   const float beta = (float)st->beta;
   const float cr = (float)st->rp_re, ci = (float)st->rp_im;
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= vh) return;
   V pv[12], rv[12];
-  load_spinor<R>(rv, r, i, vh);
+  load_spinor<S>(rv, r, i, vh);
   if (beta != 0.f) {
     load_spinor<S>(pv, p, i, vh);
   } else {
@@ -356,7 +387,7 @@ int ensure_lowprec(Context *c, int prec) {
 // half of M~ (or M~^+) with spinors in S and links/clover in G; see mtil_f64
 template <class S, class G>
 int mtil_lp(Context *c, bool dag, double kappa, double rho, SpinorPtr<S> out, SpinorPtr<S> in,
-            SpinorPtr<S> t, double *dot_out, SpinorPtr<S> dotv, const int *skip) {
+            SpinorPtr<S> t, double *dot, SpinorPtr<S> dotv, const int *skip) {
   const bool clov = use_clover(c);
   DslashArgs<S, G> a1{};
   a1.g = c->g;
@@ -380,10 +411,9 @@ int mtil_lp(Context *c, bool dag, double kappa, double rho, SpinorPtr<S> out, Sp
   a2.mkappa2 = -kappa * kappa;
   a2.rho = rho;
   a2.skip = skip;
-  a2.partials = c->red;
-  if (dot_out) {
+  if (dot) {
     a2.dotv = dotv;
-    a2.dot_out = dot_out;
+    a2.partials = dot;
     HB_TRY(launch_dslash(a2, dag, EPI_MTDOT, c->stream));
   } else {
     HB_TRY(launch_dslash(a2, dag, EPI_MTIL, c->stream));
@@ -402,7 +432,7 @@ template <class S> struct SpinorAlloc {
   }
 };
 
-template <class S, class G, class R = S>
+template <class S, class G>
 int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, const double2 *b,
                   float rest, int maxiter, int log, double delta, int max_inner, int *iters,
                   int *n_rel, double *true_rtr) {
@@ -416,7 +446,7 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
   float2 *xlo = static_cast<float2 *>(scratch(c, SLOT_MIX1, sizeof(float2) * 12 * (size_t)vh, &rc)); HB_TRY(rc);
   // low-precision fields (norm slots follow SLOT_LPN)
   SpinorPtr<S> p = SpinorAlloc<S>::get(c, SLOT_LP0, SLOT_LPN, &rc); HB_TRY(rc);
-  SpinorPtr<R> r = SpinorAlloc<R>::get(c, SLOT_LP1, SLOT_LPN1, &rc); HB_TRY(rc);
+  SpinorPtr<S> r = SpinorAlloc<S>::get(c, SLOT_LP1, SLOT_LPN1, &rc); HB_TRY(rc);
   SpinorPtr<S> q = SpinorAlloc<S>::get(c, SLOT_LP2, SLOT_LPN2, &rc); HB_TRY(rc);
   SpinorPtr<S> t = SpinorAlloc<S>::get(c, SLOT_LP3, SLOT_LPN3, &rc); HB_TRY(rc);
   SpinorPtr<S> y = SpinorAlloc<S>::get(c, SLOT_LP4, SLOT_LPN4, &rc); HB_TRY(rc);
@@ -444,40 +474,45 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
       HB_HIP(hipGetLastError());
     }
     HB_TRY(apply_f64(c, op, kappa, rho, ax, x, t64, y64, nullptr, nullptr));
-    k_mix_true_residual<R><<<nblocks(vh), kBlock, 0, c->stream>>>(ax, b, r, vh, c->red);
+    k_mix_true_residual<S><<<nblocks(vh), kBlock, 0, c->stream>>>(ax, b, r, vh, c->red);
     k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(c->red, nblocks(vh), nullptr, FinMixTrue{st, first});
     HB_HIP(hipGetLastError());
     if (!first && HB_MIX_REORTH) {
-      k_mix_rdotp<S, R><<<nblocks(vh), kBlock, 0, c->stream>>>(p, r, vh, st, c->red);
-      k_finalize<2><<<1, kFinThreads, 0, c->stream>>>(c->red, nblocks(vh), &st->flag, FinMixRdotp{st});
+      k_mix_rdotp<S><<<nblocks(vh), kBlock, 0, c->stream>>>(p, r, vh, st, c->red);
+      k_finalize<2><<<1, kFinThreads, 0, c->stream>>>(c->red, nblocks(vh), &st->s[0].flag, FinMixRdotp{st});
       HB_HIP(hipGetLastError());
     }
-    k_mix_prestart<S, R><<<nblocks(vh), kBlock, 0, c->stream>>>(p, r, vh, st);
+    k_mix_prestart<S><<<nblocks(vh), kBlock, 0, c->stream>>>(p, r, vh, st);
     HB_HIP(hipGetLastError());
     nmv++;
     return HB_OK;
   };
   HB_TRY(reliable(1));
-  const int *skip = &st->flag;
-  int chunk = 8;
+  // partials of <p, A p> and of |r|^2
+  const int na = dslash_grid<S, G>(vh), n = mix_count<S>(vh), grid = mix_grid<S>(vh), block = mix_block<S>(vh);
+  double *pa = c->red, *pb = c->red + na + 1;
+  int chunk = 8;  // iterations between looks at the state; even, so that each chunk ends in slot 0
   for (;;) {
     for (int k = 0; k < chunk; k++) {
+      const int *skip = &st->s[k & 1].flag;
       HB_TRY((mtil_lp<S, G>(c, false, kappa, r_op, y, p, t, nullptr, SpinorPtr<S>{}, skip)));
-      HB_TRY((mtil_lp<S, G>(c, true, kappa, r_op, q, y, t, &st->pap, p, skip)));
-      k_mix_update<S, R><<<nblocks(vh), kBlock, 0, c->stream>>>(r, q, vh, st, c->red);
-      k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(c->red, nblocks(vh), nullptr, FinMixUpdate{st});
+      HB_TRY((mtil_lp<S, G>(c, true, kappa, r_op, q, y, t, pa, p, skip)));
+      const double *sum = pa;
+      int nsum = na;
+      HB_TRY(shorten_partials(c, sum, nsum, skip));
+      k_mix_update<S><<<grid, block, 0, c->stream>>>(r, q, n, st, k, sum, nsum, pb);
       HB_HIP(hipGetLastError());
-      k_mix_pupdate<S, R><<<nblocks(vh), kBlock, 0, c->stream>>>(p, r, xlo, vh, st);
+      k_mix_pupdate<S><<<grid, block, 0, c->stream>>>(p, r, xlo, n, st, k, pb, grid);
       HB_HIP(hipGetLastError());
     }
     HB_HIP(hipMemcpyAsync(hs, st, sizeof(MixState), hipMemcpyDeviceToHost, c->stream));
     HB_HIP(hipStreamSynchronize(c->stream));
-    if (hs->flag == 2 || hs->flag == 3) break;
-    if (hs->flag == 1) {
+    if (hs->s[0].flag == 2 || hs->s[0].flag == 3) break;
+    if (hs->s[0].flag == 1) {
       HB_TRY(reliable(0));
       HB_HIP(hipMemcpyAsync(hs, st, sizeof(MixState), hipMemcpyDeviceToHost, c->stream));
       HB_HIP(hipStreamSynchronize(c->stream));
-      if (hs->flag == 2 || hs->flag == 3) break;
+      if (hs->s[0].flag == 2 || hs->s[0].flag == 3) break;
       // next chunk length: about the iterations one reliable interval took
       chunk = 8;
     } else if (chunk < 32) {
@@ -488,11 +523,11 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
   float ms = 0.f;
   HB_TRY(tm.elapsed(&ms));
   c->last_solve_ms = ms;
-  c->last_n_matvec = nmv + hs->iter;
-  if (iters) *iters = hs->iter;
+  c->last_n_matvec = nmv + hs->s[0].iter;
+  if (iters) *iters = hs->s[0].iter;
   if (n_rel) *n_rel = hs->n_reliable;
   if (true_rtr) *true_rtr = hs->res[0];
-  if (hs->flag != 2 && log != 2) {
+  if (hs->s[0].flag != 2 && log != 2) {
     set_error("cg_mixed(): no convergence; true rtr = %.17g", hs->res[0]);
     return HB_E_NOCONV;
   }

@@ -24,10 +24,10 @@ constexpr int kNoAllocMaxVolh = HB_NOALLOC_MAX_VOLH;         // e.g. a 16^3 x 32
 constexpr size_t kSpinorMax = 192ull * kNoAllocMaxVolh;      // one FP64 spinor field
 constexpr size_t kStateOff = 5 * kSpinorMax;                 // CgState
 constexpr size_t kRedOff = kStateOff + 256;                  // reduction partials
-constexpr size_t kRedDoubles = 4096;                         // >= nblocks(kNoAllocMaxVolh, 64)
+constexpr size_t kRedDoubles = 4096;                         // partials of CgWork::red
 constexpr size_t kScratchBytes = kRedOff + sizeof(double) * kRedDoubles;
 static_assert(sizeof(hb::CgState) <= 256, "CG state does not fit its slot");
-static_assert(kRedDoubles >= (kNoAllocMaxVolh + 63) / 64, "partials slot too small");
+static_assert(kRedDoubles >= (kNoAllocMaxVolh + 63) / 64 + 1 + 2048, "partials slot too small");
 static_assert(kStateOff % 256 == 0 && kRedOff % 256 == 0, "work fields must stay 256-byte aligned");
 
 constexpr int kMaxDevices = 64;

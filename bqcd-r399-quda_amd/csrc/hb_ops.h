@@ -77,19 +77,18 @@ int check_ready(const Context *c);
 size_t spinor_bytes(const Context *c);
 double2 *spinor_scratch(Context *c, int slot, int *rc);
 DslashArgs<SF64> dslash_args64(Context *c, int out_parity, double2 *out, const double2 *in);
-// `red` (optional): partials buffer of the fused dot product, else the context's;
+// `dot` (optional): also the partial sums of Re<dotv, out> (apply_f64: of
+// Re<in, out>), dslash_grid of them;
 // `recon`: iterate with the two-row copy of the links (ensure_links_two_rows)
 int mtil_f64(Context *c, bool dag, double kappa, double rho, double2 *out, const double2 *in,
-             double2 *t, double *dot_out, const double2 *dotv, const int *skip, double *red = nullptr,
-             bool recon = false);
+             double2 *t, double *dot, const double2 *dotv, const int *skip, bool recon = false);
 int apply_f64(Context *c, int op, double kappa, double rho, double2 *out, const double2 *in,
-              double2 *t, double2 *y, double *dot_out, const int *skip, double *red = nullptr,
-              bool recon = false);
+              double2 *t, double2 *y, double *dot, const int *skip, bool recon = false);
 int ensure_links_two_rows(Context *c, bool *use);
 
 // work fields of the FP64 CG: operator temporaries t (odd) and y (even), the
-// CG vectors r, p, q = A p, the device state, the reduction partials (at
-// least nblocks(vh) doubles) and host memory for reading the state back
+// CG vectors r, p, q = A p, the device state, the reduction partials
+// (nblocks(vh, 64) + 1 + vector_grid(vh) doubles) and host memory for reading the state back
 struct CgWork {
   double2 *t = nullptr, *y = nullptr, *r = nullptr, *p = nullptr, *q = nullptr;
   CgState *st = nullptr;
