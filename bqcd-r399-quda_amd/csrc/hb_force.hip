@@ -7,8 +7,6 @@
 // (mu, eo, i) and adds all terms of that link to its 8 momentum coordinates,
 // so no atomics are needed and the result is deterministic.  Momenta are
 // device SoA P[4 mu][2 eo][8][vh].
-#include <algorithm>
-
 #include "hb_ops.h"
 #include "hb_su3.h"
 
@@ -20,33 +18,6 @@ namespace hb {
 __device__ __forceinline__ void ld_spinor(double2 (&v)[12], const double2 *__restrict__ f, int i, int vh) {
 #pragma unroll
   for (int k = 0; k < 12; k++) v[k] = f[(size_t)k * vh + i];
-}
-
-// The force kernels' grid: a workgroup holds the four directions of 64
-// consecutive sites of one parity (one wave per direction), its neighbour in
-// the launch the other parity of the same sites.  All links of a neighbourhood
-// are then read at about the same time, instead of by eight passes over the
-// lattice, one per (direction, parity).  The XCDs share out every time slice
-// in contiguous runs of `run` workgroups, so that the slices t and t +- 1 that
-// all of them read stay in the last-level cache.  At 32^3x64 the gauge force
-// takes 3.39 ms in eight passes, 1.78 ms with one contiguous eighth of the
-// lattice per XCD, and 1.73 ms (1.54 ms in a single launch) with shared slices.
-constexpr int kLinkBlock = 256;
-struct LinkGrid {
-  int grid, run;
-  explicit LinkGrid(const Geom &g)
-      : grid(2 * nblocks(g.vh, 64)), run(std::max(1, nblocks(g.vh / g.L[3], 256))) {}
-};
-__device__ __forceinline__ bool link_slot(const Geom &g, int run, int &mu, int &e, int &i) {
-  int b = blockIdx.x;
-  if (b < (int)gridDim.x / (8 * run) * (8 * run)) {
-    const int x = b & 7, k = b >> 3;  // XCD (see xcd_block) and the workgroup's place in it
-    b = k / run * (8 * run) + x * run + k % run;
-  }
-  mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  e = b & 1;
-  i = (b >> 1) * 64 + ((int)threadIdx.x & 63);
-  return i < g.vh;
 }
 
 __device__ __forceinline__ double *mom(double *P, int mu, int eo, int vh) {
@@ -153,15 +124,7 @@ __global__ __launch_bounds__(kLinkBlock) void k_hop_force(double *P, const doubl
 // leaves (clover_d) once for each orientation of a leaf, as w and as w^+ on
 // the reversed path, so only the Hermitian H_k = s (w_k + w_k^+) is needed;
 // the scale s of the force is part of it.
-//
-// Field of one parity: nine real planes of vh sites per k, addressed as the
-// double2 planes H01, H02, H12, (H00, H11) and the double plane H22.
 // ---------------------------------------------------------------------------
-struct H3 {
-  double2 o[3];  // H01, H02, H12
-  double d[3];
-};
-
 // s (w + w^+) of a general w
 __device__ __forceinline__ H3 herm(const M3 &w, double s) {
   H3 h;
@@ -173,29 +136,6 @@ __device__ __forceinline__ H3 herm(const M3 &w, double s) {
   h.o[2] = cscale<double2>(s, cadd(w.m[5], cconj(w.m[7])));
   return h;
 }
-__device__ __forceinline__ void store_h(double *__restrict__ F, int k, int i, int vh, const H3 &h) {
-  double *b = F + (size_t)k * 9 * vh;
-  double2 *c = reinterpret_cast<double2 *>(b) + i;
-  c[0] = h.o[0];
-  c[vh] = h.o[1];
-  c[2 * (size_t)vh] = h.o[2];
-  c[3 * (size_t)vh] = make_double2(h.d[0], h.d[1]);
-  b[8 * (size_t)vh + i] = h.d[2];
-}
-__device__ __forceinline__ H3 load_h(const double *__restrict__ F, int k, int i, int vh) {
-  const uint32_t plane = (uint32_t)vh * 16u;
-  const rsrc_t r = make_rsrc(F + (size_t)k * 9 * vh, (uint32_t)vh * 72u);
-  const uint32_t vo = (uint32_t)i * 16u;
-  H3 h;
-#pragma unroll
-  for (int q = 0; q < 3; q++) h.o[q] = bld_f64x2(r, vo, plane * (uint32_t)q);
-  const double2 d = bld_f64x2(r, vo, plane * 3u);
-  h.d[0] = d.x;
-  h.d[1] = d.y;
-  h.d[2] = __builtin_bit_cast(double, bld_u32x2(r, (uint32_t)i * 8u, plane * 4u));
-  return h;
-}
-
 // w_k = sum over spins of (S_k a)_s (x) conj(b_s) (clover_bsa_12..34) from the
 // sixteen products T(s, s') = a_s' (x) conj(b_s): S_k has one entry per row,
 //   12: -00 +11 -22 +33    13: i (10 - 01 + 32 - 23)   23: -(01 + 10 + 23 + 32)
@@ -249,32 +189,6 @@ __global__ __launch_bounds__(kBlock) void k_h_spinors(double *__restrict__ F, co
     add(w, 0, 2, 1.0); add(w, 1, 3, -1.0); add(w, 2, 0, 1.0); add(w, 3, 1, -1.0);
     store_h(F, 5, i, vh, herm(w, s));
   }
-}
-
-// Z = (L D L^+)^-1 of one stored block (L unit lower triangular, D_k the
-// stored 1/2 * 1/d_k), upper triangle: M = L^-1, Z_rc = sum_k conj(M_kr) D_k M_kc
-__device__ __forceinline__ void ldl6_inverse(double2 (&Z)[6][6], const double2 (&w)[18]) {
-  double2 M[6][6];
-  const double d[6] = {w[15].x, w[15].y, w[16].x, w[16].y, w[17].x, w[17].y};
-#pragma unroll
-  for (int c = 0; c < 6; c++)
-#pragma unroll
-    for (int r = c + 1; r < 6; r++) {
-      double2 t = w[r * (r - 1) / 2 + c];
-#pragma unroll
-      for (int k = c + 1; k < r; k++) cfma3<false, false>(t, w[r * (r - 1) / 2 + k], M[k][c]);
-      M[r][c] = make_double2(-t.x, -t.y);
-    }
-#pragma unroll
-  for (int r = 0; r < 6; r++)
-#pragma unroll
-    for (int c = r; c < 6; c++) {
-      // k = c first: M_cc = 1
-      double2 t = r == c ? make_double2(d[c], 0.0) : cscale<double2>(d[c], cconj(M[c][r]));
-#pragma unroll
-      for (int k = c + 1; k < 6; k++) cfma3<true, false>(t, cscale<double2>(d[k], M[k][r]), M[k][c]);
-      Z[r][c] = t;
-    }
 }
 
 // H_k of T = A^-1 (clover_t_init, clover_ts) from the LDL^+ field of parity eo.
@@ -354,24 +268,6 @@ __device__ __forceinline__ void h_prod_acc(M3 &r, const H3 &h, const M3 &a) {
       }
     }
 }
-// an index the compiler cannot prove equal to its argument: a matrix loaded
-// again through it is a fresh load, not a register kept live since the first
-__device__ __forceinline__ int fresh(int i) {
-  asm volatile("" : "+v"(i));
-  return i;
-}
-
-// Ends a step of a kernel: the matrix is complete in registers here, and no
-// load of a later step is issued before.
-__device__ __forceinline__ void pin(M3 &m) {
-#pragma unroll
-  for (int k = 0; k < 9; k++) asm volatile("" : "+v"(m.m[k].x), "+v"(m.m[k].y));
-}
-__device__ __forceinline__ void step_end(M3 &m) {
-  pin(m);
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 // The four products of a leaf pair below.  The inner product is formed a row
 // or column at a time, so that no third matrix of temporaries is live.
 //   S += l (c b)^+
@@ -611,7 +507,7 @@ double *mom_scratch(Context *c, int *rc) {
   return static_cast<double *>(scratch(c, SLOT_MOM, sizeof(double) * 64 * (size_t)c->g.vh, rc));
 }
 
-// H field of one parity (k_h_spinors, k_h_inverse)
+// scratch for six Hermitian 3x3 matrices per site of one parity (H3)
 static double *h_scratch(Context *c, int slot, int *rc) {
   return static_cast<double *>(scratch(c, slot, sizeof(double) * 54 * (size_t)c->g.vh, rc));
 }

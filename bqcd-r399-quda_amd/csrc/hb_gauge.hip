@@ -10,38 +10,54 @@ namespace hb {
 // clover_f_mu_nu (clover/clover_f_mu_nu.F90:37-103): f = -i (Q - Q^+) with Q the
 // sum of the four plaquette leaves in plane (mu, nu) around x (parity e)
 // ---------------------------------------------------------------------------
-__device__ M3 f_mu_nu(const double2 *__restrict__ U, const Geom &g, int e, int i, const int (&x)[4],
-                      int mu, int nu) {
+// The leaves that share U_mu(x), or U_mu(x-mu), are added before they are
+// multiplied by it: with the two that run against it taken Hermitian conjugate,
+//   Q - Q^+ = X - X^+,  X = U_mu(x) (S1 - S4) + (S2 - S3) U_mu(x-mu)
+// ten matrix products where the four leaves take twelve.
+__device__ __forceinline__ H3 f_mu_nu(const double2 *__restrict__ U, const Geom &g, int e, int i, const int (&x)[4],
+                                      int mu, int nu) {
   const int o = 1 - e, vh = g.vh;
-  const int xp_ = nb(g, x[0], x[1], x[2], x[3], mu, 1);
-  const int xm_ = nb(g, x[0], x[1], x[2], x[3], mu, -1);
-  const int x_p = nb(g, x[0], x[1], x[2], x[3], nu, 1);
-  const int x_m = nb(g, x[0], x[1], x[2], x[3], nu, -1);
-  const int xmp = nb2(g, x[0], x[1], x[2], x[3], mu, -1, nu, 1);
-  const int xmm = nb2(g, x[0], x[1], x[2], x[3], mu, -1, nu, -1);
-  const int xpm = nb2(g, x[0], x[1], x[2], x[3], mu, 1, nu, -1);
-  const M3 umu_x = link(U, mu, e, i, vh);
-  const M3 unu_x = link(U, nu, e, i, vh);
-  const M3 umu_xm = link(U, mu, o, xm_, vh);
-  const M3 unu_xm = link(U, nu, o, x_m, vh);
-  // leaf 1: U_mu(x) U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
-  M3 q = m3_muld(m3_muld(m3_mul(umu_x, link(U, nu, o, xp_, vh)), link(U, mu, o, x_p, vh)), unu_x);
-  // leaf 2: U_nu(x) U_mu(x-mu+nu)^+ U_nu(x-mu)^+ U_mu(x-mu)
-  m3_acc(q, m3_mul(m3_muld(m3_muld(unu_x, link(U, mu, e, xmp, vh)), link(U, nu, o, xm_, vh)), umu_xm));
-  // leaf 3: U_mu(x-mu)^+ U_nu(x-mu-nu)^+ U_mu(x-mu-nu) U_nu(x-nu)
-  m3_acc(q, m3_mul(m3_dmul(m3_mul(link(U, nu, e, xmm, vh), umu_xm), link(U, mu, e, xmm, vh)), unu_xm));
-  // leaf 4: U_nu(x-nu)^+ U_mu(x-nu) U_nu(x+mu-nu) U_mu(x)^+
-  m3_acc(q, m3_muld(m3_mul(m3_dmul(unu_xm, link(U, mu, o, x_m, vh)), link(U, nu, e, xpm, vh)), umu_x));
-  M3 f;
+  M3 s, X;
+  {  // S1 = U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
+    const int xp = nb(g, x[0], x[1], x[2], x[3], mu, 1), yp = nb(g, x[0], x[1], x[2], x[3], nu, 1);
+    s = m3_muld(m3_muld(link_b(U, nu, o, xp, vh), link_b(U, mu, o, yp, vh)), link_b(U, nu, e, i, vh));
+  }
+  step_end(s);
+  {  // S4 = U_nu(x+mu-nu)^+ U_mu(x-nu)^+ U_nu(x-nu)
+    const int ym = nb(g, x[0], x[1], x[2], x[3], nu, -1);
+    const int xpym = nb2(g, x[0], x[1], x[2], x[3], mu, 1, nu, -1);
+    const M3 t = m3_dmul(m3_mul(link_b(U, mu, o, ym, vh), link_b(U, nu, e, xpym, vh)), link_b(U, nu, o, ym, vh));
 #pragma unroll
-  for (int a = 0; a < 3; a++)
+    for (int k = 0; k < 9; k++) s.m[k] = csub(s.m[k], t.m[k]);
+  }
+  step_end(s);
+  X = m3_mul(link_b(U, mu, e, i, vh), s);
+  step_end(X);
+  const int xm = nb(g, x[0], x[1], x[2], x[3], mu, -1);
+  {  // S2 = U_nu(x) U_mu(x-mu+nu)^+ U_nu(x-mu)^+
+    const int xmyp = nb2(g, x[0], x[1], x[2], x[3], mu, -1, nu, 1);
+    s = m3_muld(m3_muld(link_b(U, nu, e, i, vh), link_b(U, mu, e, xmyp, vh)), link_b(U, nu, o, xm, vh));
+  }
+  step_end(s);
+  {  // S3 = U_nu(x-nu)^+ U_mu(x-mu-nu)^+ U_nu(x-mu-nu)
+    const int ym = nb(g, x[0], x[1], x[2], x[3], nu, -1);
+    const int xmym = nb2(g, x[0], x[1], x[2], x[3], mu, -1, nu, -1);
+    const M3 t = m3_dmul(m3_mul(link_b(U, mu, e, xmym, vh), link_b(U, nu, o, ym, vh)), link_b(U, nu, e, xmym, vh));
 #pragma unroll
-    for (int b = 0; b < 3; b++) {
-      double2 d = csub(q.m[3 * a + b], cconj(q.m[3 * b + a]));
-      f.m[3 * a + b] = make_double2(d.y, -d.x);  // -i d
-    }
+    for (int k = 0; k < 9; k++) s.m[k] = csub(s.m[k], t.m[k]);
+  }
+  step_end(s);
+  m3_acc(X, m3_mul(s, link_b(U, mu, o, xm, vh)));
+  H3 f;  // -i (X - X^+)
 #pragma unroll
-  for (int a = 0; a < 3; a++) f.m[4 * a].y = 0.0;
+  for (int a = 0; a < 3; a++) f.d[a] = 2.0 * X.m[4 * a].y;
+  const auto off = [&X](int a, int b) {
+    const double2 d = csub(X.m[3 * a + b], cconj(X.m[3 * b + a]));
+    return make_double2(d.y, -d.x);
+  };
+  f.o[0] = off(0, 1);
+  f.o[1] = off(0, 2);
+  f.o[2] = off(1, 2);
   return f;
 }
 
@@ -68,13 +84,15 @@ __device__ void clover_block_store(double2 (&A)[6][6], double2 *__restrict__ Ca,
     d[r] = dr;
   }
   // B words: L_rc at r(r-1)/2 + c, then (1/(2 d)) pairs
+  double2 w[18];
 #pragma unroll
   for (int r = 1; r < 6; r++)
 #pragma unroll
-    for (int c = 0; c < r; c++) Cb[base + (size_t)(r * (r - 1) / 2 + c) * vh] = L[r][c];
-  Cb[base + (size_t)15 * vh] = make_double2(0.5 / d[0], 0.5 / d[1]);
-  Cb[base + (size_t)16 * vh] = make_double2(0.5 / d[2], 0.5 / d[3]);
-  Cb[base + (size_t)17 * vh] = make_double2(0.5 / d[4], 0.5 / d[5]);
+    for (int c = 0; c < r; c++) w[r * (r - 1) / 2 + c] = L[r][c];
+#pragma unroll
+  for (int k = 0; k < 3; k++) w[15 + k] = make_double2(0.5 / d[2 * k], 0.5 / d[2 * k + 1]);
+#pragma unroll
+  for (int k = 0; k < 18; k++) Cb[base + (size_t)k * vh] = w[k];
   // A/2 words
   Ca[base] = make_double2(0.5 * A[0][0].x, 0.5 * A[1][1].x);
   Ca[base + (size_t)10 * vh] = make_double2(0.5 * A[2][2].x, 0.5 * A[3][3].x);
@@ -83,96 +101,78 @@ __device__ void clover_block_store(double2 (&A)[6][6], double2 *__restrict__ Ca,
   for (int r = 0; r < 6; r++)
 #pragma unroll
     for (int c = r + 1; c < 6; c++) Ca[base + (size_t)a_off_word(r, c) * vh] = cscale<double2>(0.5, A[r][c]);
-  // inverse column by column: x = A^-1 e_col; row col of A^-1 = conj(x)
-  double2 Ainv[6][6];
-#pragma unroll
-  for (int col = 0; col < 6; col++) {
-    double2 y[6], x[6];
-#pragma unroll
-    for (int r = 0; r < 6; r++) {
-      double2 acc = make_double2(r == col ? 1.0 : 0.0, 0.0);
-#pragma unroll
-      for (int c = 0; c < r; c++) acc = csub(acc, cmul(L[r][c], y[c]));
-      y[r] = acc;
-    }
-#pragma unroll
-    for (int r = 5; r >= 0; r--) {
-      double2 acc = cscale<double2>(1.0 / d[r], y[r]);
-#pragma unroll
-      for (int c = r + 1; c < 6; c++) acc = csub(acc, cmulc(L[c][r], x[c]));
-      x[r] = acc;
-    }
-#pragma unroll
-    for (int r = 0; r < 6; r++) Ainv[col][r] = cconj(x[r]);
-  }
-  Ci[base] = make_double2(0.5 * Ainv[0][0].x, 0.5 * Ainv[1][1].x);
-  Ci[base + (size_t)10 * vh] = make_double2(0.5 * Ainv[2][2].x, 0.5 * Ainv[3][3].x);
-  Ci[base + (size_t)16 * vh] = make_double2(0.5 * Ainv[4][4].x, 0.5 * Ainv[5][5].x);
+  // A^-1/2 words
+  double2 Z[6][6];
+  ldl6_inverse(Z, w);
+  Ci[base] = make_double2(Z[0][0].x, Z[1][1].x);
+  Ci[base + (size_t)10 * vh] = make_double2(Z[2][2].x, Z[3][3].x);
+  Ci[base + (size_t)16 * vh] = make_double2(Z[4][4].x, Z[5][5].x);
 #pragma unroll
   for (int r = 0; r < 6; r++)
 #pragma unroll
-    for (int c = r + 1; c < 6; c++)
-      Ci[base + (size_t)a_off_word(r, c) * vh] = cscale<double2>(0.5, Ainv[r][c]);
+    for (int c = r + 1; c < 6; c++) Ci[base + (size_t)a_off_word(r, c) * vh] = Z[r][c];
 }
 
-// clover_init (clover/clover_init.F90:28-189): one thread per site of one parity
-__global__ __launch_bounds__(128) void k_clover_build(const double2 *__restrict__ U, Geom g, int e,
-                                                      double factor, double2 *__restrict__ Ca,
-                                                      double2 *__restrict__ Ci,
-                                                      double2 *__restrict__ Cb) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= g.vh) return;
-  int x[4];
-  site_coords(g, e, i, x[0], x[1], x[2], x[3]);
+// clover_init (clover/clover_init.F90:28-189): six waves compute the six f
+// fields of 64 sites of one parity, which meet in LDS, and two of them then
+// build and factor one chiral block each, from P = (f_21, f_32 + i f_31; .,
+// -f_21) and Q = (f_34, f_14 + i f_42; ., -f_34).
+constexpr int kPlaneBlock = 384;
+__global__ __launch_bounds__(kPlaneBlock, 3) void k_clover_build(const double2 *__restrict__ U, Geom g, int run,
+                                                                 double factor, double2 *__restrict__ Ca,
+                                                                 double2 *__restrict__ Ci, double2 *__restrict__ Cb) {
+  __shared__ double2 Fo[6][3][64];
+  __shared__ double Fd[6][3][64];
+  int k, e, i;
+  const bool active = link_slot(g, run, k, e, i);
+  const int lane = threadIdx.x & 63, vh = g.vh;
+  if (active) {
+    int x[4];
+    site_coords(g, e, i, x[0], x[1], x[2], x[3]);
+    const int mu = k == 0 ? 1 : k < 4 ? 2 : k == 4 ? 0 : 3;
+    const int nu = k == 0 || k == 2 ? 0 : k == 1 || k == 5 ? 1 : 3;
+    const H3 f = f_mu_nu(U, g, e, i, x, mu, nu);
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      Fo[k][q][lane] = f.o[q];
+      Fd[k][q][lane] = f.d[q];
+    }
+  }
+  __syncthreads();
+  const int J = k;
+  if (J > 1 || !active) return;
   double2 P[6][6], Q[6][6];
-  {
-    M3 f = f_mu_nu(U, g, e, i, x, 1, 0);  // f_21
+  const auto fill = [&](double2 (&M)[6][6], int k) {
+    const auto el = [&](int p, int a, int b) {
+      if (a == b) return make_double2(Fd[p][a][lane], 0.0);
+      const double2 z = Fo[p][a + b - 1][lane];
+      return a < b ? z : cconj(z);
+    };
 #pragma unroll
-    for (int r = 0; r < 3; r++)
+    for (int a = 0; a < 3; a++)
 #pragma unroll
-      for (int c = 0; c < 3; c++) {
-        P[r][c] = f.m[3 * r + c];
-        P[r + 3][c + 3] = make_double2(-f.m[3 * r + c].x, -f.m[3 * r + c].y);
+      for (int b = 0; b < 3; b++) {
+        if (a <= b) {
+          M[a][b] = el(k, a, b);
+          M[a + 3][b + 3] = make_double2(-M[a][b].x, -M[a][b].y);
+        }
+        M[a][b + 3] = cadd(el(k + 1, a, b), ci(el(k + 2, a, b)));
       }
-    M3 f32 = f_mu_nu(U, g, e, i, x, 2, 1);
-    M3 f31 = f_mu_nu(U, g, e, i, x, 2, 0);
-#pragma unroll
-    for (int r = 0; r < 3; r++)
-#pragma unroll
-      for (int c = 0; c < 3; c++) P[r][c + 3] = cadd(f32.m[3 * r + c], ci(f31.m[3 * r + c]));
-  }
-  {
-    M3 f = f_mu_nu(U, g, e, i, x, 2, 3);  // f_34
-#pragma unroll
-    for (int r = 0; r < 3; r++)
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        Q[r][c] = f.m[3 * r + c];
-        Q[r + 3][c + 3] = make_double2(-f.m[3 * r + c].x, -f.m[3 * r + c].y);
-      }
-    M3 f14 = f_mu_nu(U, g, e, i, x, 0, 3);
-    M3 f42 = f_mu_nu(U, g, e, i, x, 3, 1);
-#pragma unroll
-    for (int r = 0; r < 3; r++)
-#pragma unroll
-      for (int c = 0; c < 3; c++) Q[r][c + 3] = cadd(f14.m[3 * r + c], ci(f42.m[3 * r + c]));
-  }
+  };
+  fill(P, 0);
+  fill(Q, 3);
   // A_1 = 1 + s (P + Q), A_2 = 1 + s (P - Q) on the upper triangle
   double2 A[6][6];
+  const double sg = J == 0 ? 1.0 : -1.0;
 #pragma unroll
-  for (int J = 0; J < 2; J++) {
-    const double sg = J == 0 ? 1.0 : -1.0;
+  for (int r = 0; r < 6; r++)
 #pragma unroll
-    for (int r = 0; r < 6; r++)
-#pragma unroll
-      for (int c = r; c < 6; c++) {
-        double2 v = cscale<double2>(factor, make_double2(P[r][c].x + sg * Q[r][c].x, P[r][c].y + sg * Q[r][c].y));
-        if (r == c) v = make_double2(v.x + 1.0, 0.0);
-        A[r][c] = v;
-      }
-    const size_t base = (size_t)(e * 36 + J * 18) * g.vh + i;
-    clover_block_store(A, Ca, Ci, Cb, base, g.vh);
-  }
+    for (int c = r; c < 6; c++) {
+      double2 v = cscale<double2>(factor, make_double2(P[r][c].x + sg * Q[r][c].x, P[r][c].y + sg * Q[r][c].y));
+      if (r == c) v = make_double2(v.x + 1.0, 0.0);
+      A[r][c] = v;
+    }
+  clover_block_store(A, Ca, Ci, Cb, (size_t)(e * 36 + J * 18) * vh + i, vh);
 }
 
 // ---------------------------------------------------------------------------
@@ -258,11 +258,9 @@ __global__ __launch_bounds__(128) void k_ape(double2 *__restrict__ Unew, const d
 }
 
 int build_clover_into(Context *c, double csw_kappa, double2 *Ca, double2 *Ci, double2 *Cb) {
-  for (int e = 0; e < 2; e++) {
-    k_clover_build<<<nblocks(c->g.vh, 128), 128, 0, c->stream>>>(c->gauge, c->g, e, -csw_kappa / 8.0,
-                                                                 Ca, Ci, Cb);
-    HB_HIP(hipGetLastError());
-  }
+  const LinkGrid lg(c->g);
+  k_clover_build<<<lg.grid, kPlaneBlock, 0, c->stream>>>(c->gauge, c->g, lg.run, -csw_kappa / 8.0, Ca, Ci, Cb);
+  HB_HIP(hipGetLastError());
   return HB_OK;
 }
 
