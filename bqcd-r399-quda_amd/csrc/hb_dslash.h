@@ -5,7 +5,7 @@
 
 namespace hb {
 
-enum { EPI_PLAIN = 0, EPI_CLINV = 1, EPI_MTIL = 2, EPI_MTDOT = 3 };
+enum { EPI_PLAIN = 0, EPI_CLINV = 1, EPI_MTIL = 2, EPI_MTDOT = 3, EPI_SOLVE = 4 };
 
 // S: spinor storage; G: link and clover storage (same arithmetic type as S)
 template <class S, class G = S> struct DslashArgs {
@@ -14,7 +14,7 @@ template <class S, class G = S> struct DslashArgs {
   SpinorPtr<S> out;
   SpinorPtr<S> in;
   const typename G::ST *U;   // links [4][2][9][vh]
-  const typename G::ST *C;   // clover field for the epilogue (A^-1 for CLINV, A for MTIL), or null
+  const typename G::ST *C;   // clover field for the epilogue (A^-1 for CLINV, A for MTIL, LDL^+ for SOLVE), or null
   const float *Cn;           // 16-bit clover: (scale, diagonal offset) per site and block
   SpinorPtr<S> x0;           // MTIL: the vector the clover term acts on
   SpinorPtr<S> dotv;         // MTDOT: Re<dotv, out>

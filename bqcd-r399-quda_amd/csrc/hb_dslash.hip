@@ -11,6 +11,7 @@
 // Epilogues fuse the operator algebra of m_tilde.F90:43-114 into the write:
 //   EPI_PLAIN  out = D in
 //   EPI_CLINV  out = A^-1 (D in)                      (clover_mult_ao on conf%i)
+//   EPI_SOLVE  the same by LDL^+ substitution             (clover_mult_b on conf%b; FP64)
 //   EPI_MTIL   out = A x0 - kappa^2 (D in) + rho x0   (clover_mult_a + sc_xpby + sc_axpy)
 //   EPI_MTDOT  EPI_MTIL and the partial sums of Re<v, out> (sc_dot) per workgroup
 #include "hb_dslash.h"
@@ -47,11 +48,11 @@ __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<S, G> a) {
 
   if constexpr (EPI == EPI_PLAIN) {
     if (active) store_spinor<S>(a.out, i, vh, acc);
-  } else if constexpr (EPI == EPI_CLINV) {
+  } else if constexpr (EPI == EPI_CLINV || EPI == EPI_SOLVE) {
     if (active) {
       if (a.C) {
         V r[12];
-        clover_apply<G, 0, POL>(r, acc, a.C, a.Cn, e, i, vh);
+        clover_apply<G, EPI == EPI_SOLVE, POL>(r, acc, a.C, a.Cn, e, i, vh);
         store_spinor<S>(a.out, i, vh, r);
       } else {
         store_spinor<S>(a.out, i, vh, acc);
@@ -108,7 +109,7 @@ __global__ __launch_bounds__(64 * NW) void k_dslash_split(DslashArgs<S, G> a) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int i = xcd_block(blockIdx.x, gridDim.x) * 64 + lane;
   const bool active = i < vh;
-  constexpr bool kClovSum = EPI == EPI_CLINV, kClovX0 = EPI == EPI_MTIL || EPI == EPI_MTDOT;
+  constexpr bool kClovSum = EPI == EPI_CLINV || EPI == EPI_SOLVE, kClovX0 = EPI == EPI_MTIL || EPI == EPI_MTDOT;
   V acc[12], x0[12], y[6], dv[12];
 #pragma unroll
   for (int k = 0; k < 12; k++) acc[k] = cmk<V>((A)0, (A)0);
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(64 * NW) void k_dslash_split(DslashArgs<S, G> a) {
       V xp[6];
 #pragma unroll
       for (int m = 0; m < 6; m++) xp[m] = w == 0 ? cadd(acc[m], acc[m + 6]) : csub(acc[m], acc[m + 6]);
-      clover_block_apply<G, 0, POL>(y, xp, a.C, a.Cn, e, w, i, vh);
+      clover_block_apply<G, EPI == EPI_SOLVE, POL>(y, xp, a.C, a.Cn, e, w, i, vh);
       if (w == 1) {
 #pragma unroll
         for (int m = 0; m < 6; m++) y1s[m][lane] = y[m];
@@ -206,6 +207,9 @@ static void launch_split(const DslashArgs<S, G> &a, bool dag, int epi, hipStream
       case EPI_PLAIN: HB_DS(false, EPI_PLAIN); break;
       case EPI_CLINV: HB_DS(false, EPI_CLINV); break;
       case EPI_MTIL: HB_DS(false, EPI_MTIL); break;
+      case EPI_SOLVE:
+        if constexpr (std::is_same<G, SF64>::value) HB_DS(false, EPI_SOLVE);
+        break;
       default: HB_DS(false, EPI_MTDOT); break;
     }
   } else {
@@ -213,6 +217,9 @@ static void launch_split(const DslashArgs<S, G> &a, bool dag, int epi, hipStream
       case EPI_PLAIN: HB_DS(true, EPI_PLAIN); break;
       case EPI_CLINV: HB_DS(true, EPI_CLINV); break;
       case EPI_MTIL: HB_DS(true, EPI_MTIL); break;
+      case EPI_SOLVE:
+        if constexpr (std::is_same<G, SF64>::value) HB_DS(true, EPI_SOLVE);
+        break;
       default: HB_DS(true, EPI_MTDOT); break;
     }
   }
@@ -228,6 +235,9 @@ static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t
       case EPI_PLAIN: HB_DS(false, EPI_PLAIN); break;
       case EPI_CLINV: HB_DS(false, EPI_CLINV); break;
       case EPI_MTIL: HB_DS(false, EPI_MTIL); break;
+      case EPI_SOLVE:
+        if constexpr (std::is_same<G, SF64>::value) HB_DS(false, EPI_SOLVE);
+        break;
       default: HB_DS(false, EPI_MTDOT); break;
     }
   } else {
@@ -235,6 +245,9 @@ static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t
       case EPI_PLAIN: HB_DS(true, EPI_PLAIN); break;
       case EPI_CLINV: HB_DS(true, EPI_CLINV); break;
       case EPI_MTIL: HB_DS(true, EPI_MTIL); break;
+      case EPI_SOLVE:
+        if constexpr (std::is_same<G, SF64>::value) HB_DS(true, EPI_SOLVE);
+        break;
       default: HB_DS(true, EPI_MTDOT); break;
     }
   }

@@ -99,23 +99,22 @@ __device__ void hop_force_link(double (&q)[8], const double2 *__restrict__ U, co
   im_tr_j_outer(q, h, w, sg);
 }
 
-__global__ __launch_bounds__(kLinkBlock) void k_hop_force(double *P, const double2 *__restrict__ U, Geom g, int run,
-                                                          const double2 *a, const double2 *b, const double2 *at,
-                                                          const double2 *bt, double s) {
-  int mu, e, i;
-  if (!link_slot(g, run, mu, e, i)) return;
-  int x[4];
-  site_coords(g, e, i, x[0], x[1], x[2], x[3]);
-  const double2 *Bi = e == 0 ? b : bt, *Aj = e == 0 ? at : a;
-  const double2 *Ai = e == 0 ? a : at, *Bj = e == 0 ? bt : b;
-  double q[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+// spinors of the hopping force: a, b on the even sites, at = A~, bt = B~ on the
+// odd ones; s = 0: no hopping force
+struct HopForce {
+  const double2 *a, *b, *at, *bt;
+  double s;
+};
+__device__ __forceinline__ void hop_force(double (&q)[8], const double2 *__restrict__ U, const Geom &g, int mu, int e,
+                                          int i, const int (&x)[4], const HopForce &h) {
+  const double2 *Bi = e == 0 ? h.b : h.bt, *Aj = e == 0 ? h.at : h.a;
+  const double2 *Ai = e == 0 ? h.a : h.at, *Bj = e == 0 ? h.bt : h.b;
   switch (mu) {
-    case 0: hop_force_link<0>(q, U, g, e, i, x, Bi, Aj, Ai, Bj, s); break;
-    case 1: hop_force_link<1>(q, U, g, e, i, x, Bi, Aj, Ai, Bj, s); break;
-    case 2: hop_force_link<2>(q, U, g, e, i, x, Bi, Aj, Ai, Bj, s); break;
-    default: hop_force_link<3>(q, U, g, e, i, x, Bi, Aj, Ai, Bj, s); break;
+    case 0: hop_force_link<0>(q, U, g, e, i, x, Bi, Aj, Ai, Bj, h.s); break;
+    case 1: hop_force_link<1>(q, U, g, e, i, x, Bi, Aj, Ai, Bj, h.s); break;
+    case 2: hop_force_link<2>(q, U, g, e, i, x, Bi, Aj, Ai, Bj, h.s); break;
+    default: hop_force_link<3>(q, U, g, e, i, x, Bi, Aj, Ai, Bj, h.s); break;
   }
-  mom_add(P, mu, e, i, g.vh, q);
 }
 
 // ---------------------------------------------------------------------------
@@ -140,10 +139,19 @@ __device__ __forceinline__ H3 herm(const M3 &w, double s) {
 // sixteen products T(s, s') = a_s' (x) conj(b_s): S_k has one entry per row,
 //   12: -00 +11 -22 +33    13: i (10 - 01 + 32 - 23)   23: -(01 + 10 + 23 + 32)
 //   14: 03 + 12 + 21 + 30  24: i (12 - 03 + 30 - 21)   34: 02 - 13 + 20 - 31
-__global__ __launch_bounds__(kBlock) void k_h_spinors(double *__restrict__ F, const double2 *__restrict__ b,
-                                                      const double2 *__restrict__ a, int vh, double s) {
+// (blockIdx.y: one of up to two fields)
+struct HSpinors {
+  double *F;
+  const double2 *b, *a;
+  double s;
+};
+__global__ __launch_bounds__(kBlock) void k_h_spinors(HSpinors h0, HSpinors h1, int vh) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= vh) return;
+  const HSpinors h = blockIdx.y == 0 ? h0 : h1;
+  double *F = h.F;
+  const double2 *b = h.b, *a = h.a;
+  const double s = h.s;
   double2 av[12], bv[12];
   ld_spinor(av, a, i, vh);
   ld_spinor(bv, b, i, vh);
@@ -418,19 +426,26 @@ __device__ __forceinline__ void clover_leaves(M3 &S, const double2 *__restrict__
   }
 }
 
+// the clover force of one link and, for the fermion force, its hopping force
+// (HOP; the spinors of hop): in a kernel of its own the hopping force reads the
+// links and updates the momenta once more
+template <bool HOP>
 __global__ __launch_bounds__(kLinkBlock, 2) void k_clover_force(double *P, const double2 *__restrict__ U, Geom g, int run,
-                                                             const double *H0, const double *H1) {
+                                                                const double *H0, const double *H1, HopForce hop) {
   int mu, e, i;
   if (!link_slot(g, run, mu, e, i)) return;
   const double *He = e == 0 ? H0 : H1, *Ho = e == 0 ? H1 : H0;
   int x[4];
   site_coords(g, e, i, x[0], x[1], x[2], x[3]);
-  M3 S = m3_zero();
-  if (He && Ho) clover_leaves<true, true>(S, U, g, mu, e, i, x, He, Ho);
-  else if (He) clover_leaves<true, false>(S, U, g, mu, e, i, x, He, Ho);
-  else clover_leaves<false, true>(S, U, g, mu, e, i, x, He, Ho);
   double q[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  re_tr_j_prod<0>(q, link_b(U, mu, e, i, g.vh), S, 1.0);
+  if (He || Ho) {
+    M3 S = m3_zero();
+    if (He && Ho) clover_leaves<true, true>(S, U, g, mu, e, i, x, He, Ho);
+    else if (He) clover_leaves<true, false>(S, U, g, mu, e, i, x, He, Ho);
+    else clover_leaves<false, true>(S, U, g, mu, e, i, x, He, Ho);
+    re_tr_j_prod<0>(q, link_b(U, mu, e, i, g.vh), S, 1.0);
+  }
+  if (HOP && hop.s != 0.0) hop_force(q, U, g, mu, e, i, x, hop);
   mom_add(P, mu, e, i, g.vh, q);
 }
 
@@ -521,45 +536,40 @@ int dsf_dev(Context *c, double *P, double step, double kappa, double csw_kappa, 
   double2 *bt = spinor_scratch(c, SLOT_FORCE1, &rc); HB_TRY(rc);
   double *H0 = h_scratch(c, SLOT_FORCE2, &rc); HB_TRY(rc);
   double *H1 = h_scratch(c, SLOT_FORCE3, &rc); HB_TRY(rc);
-  double2 *tmp = spinor_scratch(c, SLOT_FORCE4, &rc); HB_TRY(rc);
   const bool clov = csw_kappa != 0.0;
   if (clov) HB_CHECK(c->have_clover[HB_CLOVER_B], HB_E_STATE, "dsf: clover B field not present");
   if (kappa != 0.0) {
     // A~ = D_oe a, B~ = D_eo^+ b (dsf.F90:56-57), then A_oo^-1 by LDL^+ (clover_mult_b)
-    DslashArgs<SF64> d1 = dslash_args64(c, 1, clov ? tmp : at, a);
-    HB_TRY(launch_dslash(d1, false, EPI_PLAIN, c->stream));
-    if (clov) HB_TRY(clover_mult_f64(c, HB_CLOVER_B, 1, at, tmp));
-    DslashArgs<SF64> d2 = dslash_args64(c, 1, clov ? tmp : bt, b);
-    HB_TRY(launch_dslash(d2, true, EPI_PLAIN, c->stream));
-    if (clov) HB_TRY(clover_mult_f64(c, HB_CLOVER_B, 1, bt, tmp));
+    DslashArgs<SF64> d1 = dslash_args64(c, 1, at, a);
+    if (clov) d1.C = c->clov[HB_CLOVER_B];
+    HB_TRY(launch_dslash(d1, false, clov ? EPI_SOLVE : EPI_PLAIN, c->stream));
+    DslashArgs<SF64> d2 = dslash_args64(c, 1, bt, b);
+    d2.C = d1.C;
+    HB_TRY(launch_dslash(d2, true, clov ? EPI_SOLVE : EPI_PLAIN, c->stream));
   } else {
     HB_TRY(zero_f64(c, at, 12 * (size_t)vh));
     HB_TRY(zero_f64(c, bt, 12 * (size_t)vh));
   }
-  const double s = -step * 2.0 * kappa * kappa;
   const LinkGrid lg(c->g);
-  if (s != 0.0) {
-    k_hop_force<<<lg.grid, kLinkBlock, 0, c->stream>>>(P, c->gauge, c->g, lg.run, a, b, at, bt, s);
-    HB_HIP(hipGetLastError());
-  }
+  const HopForce hop{a, b, at, bt, -step * 2.0 * kappa * kappa};
   // clover part (dsf.F90:103-109) on physical links
   const double s1 = -step * 2.0 * (csw_kappa / 8.0);
   const double s2 = s1 * kappa * kappa;
-  if (s1 != 0.0 || s2 != 0.0) {
-    if (s1 != 0.0) k_h_spinors<<<nblocks(vh), kBlock, 0, c->stream>>>(H0, b, a, vh, s1);
-    if (s2 != 0.0) k_h_spinors<<<nblocks(vh), kBlock, 0, c->stream>>>(H1, bt, at, vh, s2);
-    k_clover_force<<<lg.grid, kLinkBlock, 0, c->stream>>>(P, c->gauge, c->g, lg.run, s1 != 0.0 ? H0 : nullptr,
-                                                          s2 != 0.0 ? H1 : nullptr);
-    HB_HIP(hipGetLastError());
-  }
+  if (s1 != 0.0)
+    k_h_spinors<<<dim3(nblocks(vh), s2 != 0.0 ? 2 : 1), kBlock, 0, c->stream>>>(HSpinors{H0, b, a, s1},
+                                                                               HSpinors{H1, bt, at, s2}, vh);
+  if (hop.s != 0.0 || s1 != 0.0)
+    k_clover_force<true><<<lg.grid, kLinkBlock, 0, c->stream>>>(P, c->gauge, c->g, lg.run, s1 != 0.0 ? H0 : nullptr,
+                                                                s2 != 0.0 ? H1 : nullptr, hop);
+  HB_HIP(hipGetLastError());
   return HB_OK;
 }
 
 // the clover force of one parity's H field
 static int clover_force_one(Context *c, double *P, int eo, const double *H) {
   const LinkGrid lg(c->g);
-  k_clover_force<<<lg.grid, kLinkBlock, 0, c->stream>>>(P, c->gauge, c->g, lg.run, eo == 0 ? H : nullptr,
-                                                        eo == 0 ? nullptr : H);
+  k_clover_force<false><<<lg.grid, kLinkBlock, 0, c->stream>>>(P, c->gauge, c->g, lg.run, eo == 0 ? H : nullptr,
+                                                               eo == 0 ? nullptr : H, HopForce{});
   HB_HIP(hipGetLastError());
   return HB_OK;
 }
@@ -570,7 +580,8 @@ int clover_dsf_dev(Context *c, double *P, int eo, const double2 *b, const double
   if (s == 0.0) return HB_OK;
   int rc = 0;
   double *H = h_scratch(c, SLOT_FORCE2, &rc); HB_TRY(rc);
-  k_h_spinors<<<nblocks(c->g.vh), kBlock, 0, c->stream>>>(H, b, a, c->g.vh, s);
+  const HSpinors h{H, b, a, s};
+  k_h_spinors<<<nblocks(c->g.vh), kBlock, 0, c->stream>>>(h, h, c->g.vh);
   return clover_force_one(c, P, eo, H);
 }
 

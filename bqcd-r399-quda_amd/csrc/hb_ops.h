@@ -34,7 +34,6 @@ enum {
   SLOT_FORCE1,
   SLOT_FORCE2,
   SLOT_FORCE3,
-  SLOT_FORCE4,
   SLOT_MOM,
   SLOT_SINGLE_END
 };
