@@ -199,6 +199,32 @@ __global__ __launch_bounds__(kBlock) void k_h_spinors(HSpinors h0, HSpinors h1, 
   }
 }
 
+// Z = (L D L^+)^-1 of one stored block (L unit lower triangular, D_k the
+// stored 1/2 * 1/d_k), upper triangle: M = L^-1, Z_rc = sum_k conj(M_kr) D_k M_kc
+__device__ __forceinline__ void ldl6_inverse(double2 (&Z)[6][6], const double2 (&w)[18]) {
+  double2 M[6][6];
+  const double d[6] = {w[15].x, w[15].y, w[16].x, w[16].y, w[17].x, w[17].y};
+#pragma unroll
+  for (int c = 0; c < 6; c++)
+#pragma unroll
+    for (int r = c + 1; r < 6; r++) {
+      double2 t = w[r * (r - 1) / 2 + c];
+#pragma unroll
+      for (int k = c + 1; k < r; k++) cfma3<false, false>(t, w[r * (r - 1) / 2 + k], M[k][c]);
+      M[r][c] = make_double2(-t.x, -t.y);
+    }
+#pragma unroll
+  for (int r = 0; r < 6; r++)
+#pragma unroll
+    for (int c = r; c < 6; c++) {
+      // k = c first: M_cc = 1
+      double2 t = r == c ? make_double2(d[c], 0.0) : cscale<double2>(d[c], cconj(M[c][r]));
+#pragma unroll
+      for (int k = c + 1; k < 6; k++) cfma3<true, false>(t, cscale<double2>(d[k], M[k][r]), M[k][c]);
+      Z[r][c] = t;
+    }
+}
+
 // H_k of T = A^-1 (clover_t_init, clover_ts) from the LDL^+ field of parity eo.
 // T's spin blocks are T_uu = T_ll = Z_1 + Z_2 and T_ul = T_lu = Z_1 - Z_2 with
 // the inverses Z of the two chiral blocks, so that with P = Z_1 + Z_2 and

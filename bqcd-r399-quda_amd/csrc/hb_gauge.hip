@@ -10,49 +10,42 @@ namespace hb {
 // clover_f_mu_nu (clover/clover_f_mu_nu.F90:37-103): f = -i (Q - Q^+) with Q the
 // sum of the four plaquette leaves in plane (mu, nu) around x (parity e)
 // ---------------------------------------------------------------------------
-// The leaves that share U_mu(x), or U_mu(x-mu), are added before they are
-// multiplied by it: with the two that run against it taken Hermitian conjugate,
-//   Q - Q^+ = X - X^+,  X = U_mu(x) (S1 - S4) + (S2 - S3) U_mu(x-mu)
-// ten matrix products where the four leaves take twelve.
 __device__ __forceinline__ H3 f_mu_nu(const double2 *__restrict__ U, const Geom &g, int e, int i, const int (&x)[4],
                                       int mu, int nu) {
   const int o = 1 - e, vh = g.vh;
-  M3 s, X;
-  {  // S1 = U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
-    const int xp = nb(g, x[0], x[1], x[2], x[3], mu, 1), yp = nb(g, x[0], x[1], x[2], x[3], nu, 1);
-    s = m3_muld(m3_muld(link_b(U, nu, o, xp, vh), link_b(U, mu, o, yp, vh)), link_b(U, nu, e, i, vh));
+  const int xm_ = nb(g, x[0], x[1], x[2], x[3], mu, -1), x_m = nb(g, x[0], x[1], x[2], x[3], nu, -1);
+  M3 q;
+  {  // leaf 1: U_mu(x) U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
+    const int xp_ = nb(g, x[0], x[1], x[2], x[3], mu, 1), x_p = nb(g, x[0], x[1], x[2], x[3], nu, 1);
+    q = m3_muld(m3_muld(m3_mul(link_b(U, mu, e, i, vh), link_b(U, nu, o, xp_, vh)), link_b(U, mu, o, x_p, vh)),
+                link_b(U, nu, e, i, vh));
   }
-  step_end(s);
-  {  // S4 = U_nu(x+mu-nu)^+ U_mu(x-nu)^+ U_nu(x-nu)
-    const int ym = nb(g, x[0], x[1], x[2], x[3], nu, -1);
-    const int xpym = nb2(g, x[0], x[1], x[2], x[3], mu, 1, nu, -1);
-    const M3 t = m3_dmul(m3_mul(link_b(U, mu, o, ym, vh), link_b(U, nu, e, xpym, vh)), link_b(U, nu, o, ym, vh));
+  step_end(q);
+  {  // leaf 2: U_nu(x) U_mu(x-mu+nu)^+ U_nu(x-mu)^+ U_mu(x-mu)
+    const int xmp = nb2(g, x[0], x[1], x[2], x[3], mu, -1, nu, 1);
+    m3_acc(q, m3_mul(m3_muld(m3_muld(link_b(U, nu, e, fresh(i), vh), link_b(U, mu, e, xmp, vh)),
+                             link_b(U, nu, o, xm_, vh)),
+                     link_b(U, mu, o, xm_, vh)));
+  }
+  step_end(q);
+  {  // leaf 3: U_mu(x-mu)^+ U_nu(x-mu-nu)^+ U_mu(x-mu-nu) U_nu(x-nu)
+    const int xmm = nb2(g, x[0], x[1], x[2], x[3], mu, -1, nu, -1);
+    m3_acc(q, m3_mul(m3_dmul(m3_mul(link_b(U, nu, e, xmm, vh), link_b(U, mu, o, fresh(xm_), vh)),
+                             link_b(U, mu, e, xmm, vh)),
+                     link_b(U, nu, o, x_m, vh)));
+  }
+  step_end(q);
+  {  // leaf 4: U_nu(x-nu)^+ U_mu(x-nu) U_nu(x+mu-nu) U_mu(x)^+
+    const int xpm = nb2(g, x[0], x[1], x[2], x[3], mu, 1, nu, -1);
+    m3_acc(q, m3_muld(m3_mul(m3_dmul(link_b(U, nu, o, fresh(x_m), vh), link_b(U, mu, o, x_m, vh)),
+                             link_b(U, nu, e, xpm, vh)),
+                      link_b(U, mu, e, fresh(i), vh)));
+  }
+  H3 f;  // -i (Q - Q^+)
 #pragma unroll
-    for (int k = 0; k < 9; k++) s.m[k] = csub(s.m[k], t.m[k]);
-  }
-  step_end(s);
-  X = m3_mul(link_b(U, mu, e, i, vh), s);
-  step_end(X);
-  const int xm = nb(g, x[0], x[1], x[2], x[3], mu, -1);
-  {  // S2 = U_nu(x) U_mu(x-mu+nu)^+ U_nu(x-mu)^+
-    const int xmyp = nb2(g, x[0], x[1], x[2], x[3], mu, -1, nu, 1);
-    s = m3_muld(m3_muld(link_b(U, nu, e, i, vh), link_b(U, mu, e, xmyp, vh)), link_b(U, nu, o, xm, vh));
-  }
-  step_end(s);
-  {  // S3 = U_nu(x-nu)^+ U_mu(x-mu-nu)^+ U_nu(x-mu-nu)
-    const int ym = nb(g, x[0], x[1], x[2], x[3], nu, -1);
-    const int xmym = nb2(g, x[0], x[1], x[2], x[3], mu, -1, nu, -1);
-    const M3 t = m3_dmul(m3_mul(link_b(U, mu, e, xmym, vh), link_b(U, nu, o, ym, vh)), link_b(U, nu, e, xmym, vh));
-#pragma unroll
-    for (int k = 0; k < 9; k++) s.m[k] = csub(s.m[k], t.m[k]);
-  }
-  step_end(s);
-  m3_acc(X, m3_mul(s, link_b(U, mu, o, xm, vh)));
-  H3 f;  // -i (X - X^+)
-#pragma unroll
-  for (int a = 0; a < 3; a++) f.d[a] = 2.0 * X.m[4 * a].y;
-  const auto off = [&X](int a, int b) {
-    const double2 d = csub(X.m[3 * a + b], cconj(X.m[3 * b + a]));
+  for (int a = 0; a < 3; a++) f.d[a] = csub(q.m[4 * a], cconj(q.m[4 * a])).y;
+  const auto off = [&q](int a, int b) {
+    const double2 d = csub(q.m[3 * a + b], cconj(q.m[3 * b + a]));
     return make_double2(d.y, -d.x);
   };
   f.o[0] = off(0, 1);
@@ -84,15 +77,13 @@ __device__ void clover_block_store(double2 (&A)[6][6], double2 *__restrict__ Ca,
     d[r] = dr;
   }
   // B words: L_rc at r(r-1)/2 + c, then (1/(2 d)) pairs
-  double2 w[18];
 #pragma unroll
   for (int r = 1; r < 6; r++)
 #pragma unroll
-    for (int c = 0; c < r; c++) w[r * (r - 1) / 2 + c] = L[r][c];
-#pragma unroll
-  for (int k = 0; k < 3; k++) w[15 + k] = make_double2(0.5 / d[2 * k], 0.5 / d[2 * k + 1]);
-#pragma unroll
-  for (int k = 0; k < 18; k++) Cb[base + (size_t)k * vh] = w[k];
+    for (int c = 0; c < r; c++) Cb[base + (size_t)(r * (r - 1) / 2 + c) * vh] = L[r][c];
+  Cb[base + (size_t)15 * vh] = make_double2(0.5 / d[0], 0.5 / d[1]);
+  Cb[base + (size_t)16 * vh] = make_double2(0.5 / d[2], 0.5 / d[3]);
+  Cb[base + (size_t)17 * vh] = make_double2(0.5 / d[4], 0.5 / d[5]);
   // A/2 words
   Ca[base] = make_double2(0.5 * A[0][0].x, 0.5 * A[1][1].x);
   Ca[base + (size_t)10 * vh] = make_double2(0.5 * A[2][2].x, 0.5 * A[3][3].x);
@@ -101,22 +92,46 @@ __device__ void clover_block_store(double2 (&A)[6][6], double2 *__restrict__ Ca,
   for (int r = 0; r < 6; r++)
 #pragma unroll
     for (int c = r + 1; c < 6; c++) Ca[base + (size_t)a_off_word(r, c) * vh] = cscale<double2>(0.5, A[r][c]);
-  // A^-1/2 words
-  double2 Z[6][6];
-  ldl6_inverse(Z, w);
-  Ci[base] = make_double2(Z[0][0].x, Z[1][1].x);
-  Ci[base + (size_t)10 * vh] = make_double2(Z[2][2].x, Z[3][3].x);
-  Ci[base + (size_t)16 * vh] = make_double2(Z[4][4].x, Z[5][5].x);
+  // inverse column by column: x = A^-1 e_col; row col of A^-1 = conj(x)
+  double2 Ainv[6][6];
+#pragma unroll
+  for (int col = 0; col < 6; col++) {
+    double2 y[6], x[6];
+#pragma unroll
+    for (int r = 0; r < 6; r++) {
+      double2 acc = make_double2(r == col ? 1.0 : 0.0, 0.0);
+#pragma unroll
+      for (int c = 0; c < r; c++) acc = csub(acc, cmul(L[r][c], y[c]));
+      y[r] = acc;
+    }
+#pragma unroll
+    for (int r = 5; r >= 0; r--) {
+      double2 acc = cscale<double2>(1.0 / d[r], y[r]);
+#pragma unroll
+      for (int c = r + 1; c < 6; c++) acc = csub(acc, cmulc(L[c][r], x[c]));
+      x[r] = acc;
+    }
+#pragma unroll
+    for (int r = 0; r < 6; r++) Ainv[col][r] = cconj(x[r]);
+  }
+  Ci[base] = make_double2(0.5 * Ainv[0][0].x, 0.5 * Ainv[1][1].x);
+  Ci[base + (size_t)10 * vh] = make_double2(0.5 * Ainv[2][2].x, 0.5 * Ainv[3][3].x);
+  Ci[base + (size_t)16 * vh] = make_double2(0.5 * Ainv[4][4].x, 0.5 * Ainv[5][5].x);
 #pragma unroll
   for (int r = 0; r < 6; r++)
 #pragma unroll
-    for (int c = r + 1; c < 6; c++) Ci[base + (size_t)a_off_word(r, c) * vh] = Z[r][c];
+    for (int c = r + 1; c < 6; c++)
+      Ci[base + (size_t)a_off_word(r, c) * vh] = cscale<double2>(0.5, Ainv[r][c]);
 }
 
 // clover_init (clover/clover_init.F90:28-189): six waves compute the six f
 // fields of 64 sites of one parity, which meet in LDS, and two of them then
 // build and factor one chiral block each, from P = (f_21, f_32 + i f_31; .,
-// -f_21) and Q = (f_34, f_14 + i f_42; ., -f_34).
+// -f_21) and Q = (f_34, f_14 + i f_42; ., -f_34).  One thread per site, the
+// planes one after the other, needs 512 registers, one wave per SIMD.  Both
+// parities, that way / this way: 8^3x16 68 / 19 us, 16^3x32 147 / 125,
+// 24x20x12x36 262 / 208, 32^3x64 2.27 / 2.29 ms (there the links, read 14 times
+// a plane, come from beyond L2).
 constexpr int kPlaneBlock = 384;
 __global__ __launch_bounds__(kPlaneBlock, 3) void k_clover_build(const double2 *__restrict__ U, Geom g, int run,
                                                                  double factor, double2 *__restrict__ Ca,

@@ -702,11 +702,11 @@ __device__ __forceinline__ float2 clover_block_word(double2 v, int k, float2 mc)
 }
 
 // loads block J of the FP64 / FP32 clover field of parity eo at site i (16-bit
-// fields are site-packed, see load_clover_block_raw)
+// fields are site-packed, see CloverFetch<SF16>)
 template <class S, int POL = kNT>
 __device__ __forceinline__ void load_clover_block(typename S::V (&w)[18], const typename S::ST *C,
                                                   const float *Cn, int eo, int J, int i, int vh) {
-  static_assert(!S::kNorm, "16-bit clover blocks are read with load_clover_block_raw");
+  static_assert(!S::kNorm, "16-bit clover blocks are read with CloverFetch");
   const uint32_t plane = (uint32_t)vh * S::kBytes;
   rsrc_t r = make_rsrc(C + (size_t)(eo * 36 + J * 18) * vh, plane * 18u);
   const uint32_t vo = (uint32_t)i * S::kBytes;
@@ -722,13 +722,15 @@ constexpr uint32_t kClov16 = 80;  // bytes of one block of one element
 constexpr int kClov16Words = 20;  // the same in short2 units
 
 // block of element e of a slab (buffer r, plane = 16 * elements per slab
-// bytes): Q as stored (the integers as floats) and the block's factors: the
-// block is c 1 + (m / 32767) Q_int; returns (m / 32767, c)
+// bytes) as stored
 template <int POL = kNT>
-__device__ __forceinline__ float2 load_clover_rec16(float2 (&w)[18], rsrc_t r, uint32_t e, uint32_t plane) {
-  u32x4 q[5];
+__device__ __forceinline__ void fetch_clover_rec16(u32x4 (&q)[5], rsrc_t r, uint32_t e, uint32_t plane) {
 #pragma unroll
   for (int k = 0; k < 5; k++) q[k] = bld_u32x4<POL>(r, e * 16u, plane * k);
+}
+// its Q (the integers as floats) and factors: the block is c 1 + (m / 32767)
+// Q_int; returns (m / 32767, c)
+__device__ __forceinline__ float2 decode_clover_rec16(float2 (&w)[18], const u32x4 (&q)[5]) {
 #pragma unroll
   for (int k = 0; k < 18; k++) {
     const uint32_t x = q[k >> 2][k & 3];
@@ -736,6 +738,12 @@ __device__ __forceinline__ float2 load_clover_rec16(float2 (&w)[18], rsrc_t r, u
   }
   const uint32_t m = q[4][2], c = q[4][3];
   return make_float2(as_float(m) * SF16::kInv, as_float(c));
+}
+template <int POL = kNT>
+__device__ __forceinline__ float2 load_clover_rec16(float2 (&w)[18], rsrc_t r, uint32_t e, uint32_t plane) {
+  u32x4 q[5];
+  fetch_clover_rec16<POL>(q, r, e, plane);
+  return decode_clover_rec16(w, q);
 }
 
 // block J of the 16-bit clover field of parity eo at site i (Cn is unused: the
@@ -797,23 +805,40 @@ __device__ __forceinline__ void clover_raw_finish(V (&y)[6], const V (&x)[6], fl
   }
 }
 
-// y = A_J x for chiral block J of the clover field C: mode 0 = Hermitian
-// product, 1 = LDL^+ solve
-template <class SG, int MODE, int POL = kNT, class V>
-__device__ __forceinline__ void clover_block_apply(V (&y)[6], const V (&x)[6], const typename SG::ST *C,
-                                                   const float *Cn, int eo, int J, int i, int vh) {
-  constexpr bool kRaw = std::is_same<SG, SF16>::value;
-  static_assert(!kRaw || MODE == 0, "16-bit clover blocks hold A/2 or A^-1/2, not LDL factors");
+// Chiral block J of the clover field C at one site, fetched as stored (so that
+// the loads can be issued ahead of their use) and applied: y = A_J x, mode 0 =
+// Hermitian product, 1 = LDL^+ solve
+template <class SG> struct CloverFetch {
   typename SG::V w[18];
-  float2 mc;
-  if constexpr (kRaw) mc = load_clover_block_raw<POL>(w, C, Cn, eo, J, i, vh);
-  else load_clover_block<SG, POL>(w, C, Cn, eo, J, i, vh);
-  V ww[18];
+  template <int POL = kNT>
+  __device__ __forceinline__ void load(const typename SG::ST *C, int eo, int J, int i, int vh) {
+    load_clover_block<SG, POL>(w, C, nullptr, eo, J, i, vh);
+  }
+  template <int MODE, class V> __device__ __forceinline__ void apply(V (&y)[6], const V (&x)[6]) const {
+    V ww[18];
 #pragma unroll
-  for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);
-  if constexpr (MODE == 0) herm6(y, ww, x); else ldl6(y, ww, x);
-  if constexpr (kRaw) clover_raw_finish(y, x, mc);
-}
+    for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);
+    if constexpr (MODE == 0) herm6(y, ww, x); else ldl6(y, ww, x);
+  }
+};
+template <> struct CloverFetch<SF16> {
+  u32x4 q[5];
+  template <int POL = kNT>
+  __device__ __forceinline__ void load(const SF16::ST *C, int eo, int J, int i, int vh) {
+    const rsrc_t r = make_rsrc(C + (size_t)((eo * 2 + J) * kClov16Words) * vh, (uint32_t)vh * kClov16);
+    fetch_clover_rec16<POL>(q, r, (uint32_t)i, (uint32_t)vh * 16u);
+  }
+  template <int MODE, class V> __device__ __forceinline__ void apply(V (&y)[6], const V (&x)[6]) const {
+    static_assert(MODE == 0, "16-bit clover blocks hold A/2 or A^-1/2, not LDL factors");
+    float2 w[18];
+    const float2 mc = decode_clover_rec16(w, q);
+    V ww[18];
+#pragma unroll
+    for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);
+    herm6(y, ww, x);
+    clover_raw_finish(y, x, mc);
+  }
+};
 
 // out = A in (Dirac basis) with A stored as two chiral blocks of A/2
 // (clover_mult_a.F90:44-95); mode 0 = Hermitian product, 1 = LDL^+ solve.
@@ -823,16 +848,38 @@ __device__ __forceinline__ void clover_apply(V (&out)[12], const V (&in)[12],
                                              const typename SG::ST *C, const float *Cn, int eo,
                                              int i, int vh) {
   V xp[6], y1[6], y2[6];
+  constexpr bool kRaw = std::is_same<SG, SF16>::value;
+  static_assert(!kRaw || MODE == 0, "16-bit clover blocks hold A/2 or A^-1/2, not LDL factors");
 #pragma unroll
   for (int m = 0; m < 6; m++) xp[m] = cadd(in[m], in[m + 6]);
-  clover_block_apply<SG, MODE, POL>(y1, xp, C, Cn, eo, 0, i, vh);
+  {
+    typename SG::V w[18];
+    float2 mc;
+    if constexpr (kRaw) mc = load_clover_block_raw<POL>(w, C, Cn, eo, 0, i, vh);
+    else load_clover_block<SG, POL>(w, C, Cn, eo, 0, i, vh);
+    V ww[18];
+#pragma unroll
+    for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);
+    if constexpr (MODE == 0) herm6(y1, ww, xp); else ldl6(y1, ww, xp);
+    if constexpr (kRaw) clover_raw_finish(y1, xp, mc);
+  }
   // finish block 0 before loading block 1 (bounds live registers)
 #pragma unroll
   for (int m = 0; m < 6; m++) asm volatile("" : "+v"(y1[m].x), "+v"(y1[m].y));
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int m = 0; m < 6; m++) xp[m] = csub(in[m], in[m + 6]);
-  clover_block_apply<SG, MODE, POL>(y2, xp, C, Cn, eo, 1, i, vh);
+  {
+    typename SG::V w[18];
+    float2 mc;
+    if constexpr (kRaw) mc = load_clover_block_raw<POL>(w, C, Cn, eo, 1, i, vh);
+    else load_clover_block<SG, POL>(w, C, Cn, eo, 1, i, vh);
+    V ww[18];
+#pragma unroll
+    for (int k = 0; k < 18; k++) ww[k] = cmk<V>(w[k].x, w[k].y);
+    if constexpr (MODE == 0) herm6(y2, ww, xp); else ldl6(y2, ww, xp);
+    if constexpr (kRaw) clover_raw_finish(y2, xp, mc);
+  }
 #pragma unroll
   for (int m = 0; m < 6; m++) {
     out[m] = cadd(y1[m], y2[m]);
