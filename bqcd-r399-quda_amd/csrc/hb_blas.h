@@ -19,6 +19,7 @@ struct CgSlot {
 struct CgState {
   CgSlot s[2];
   double pap;      // <p, A p> of the iteration, from the r update for the p update
+  double alpha[4]; // of the iterations whose x updates are pending (CgRing)
   double rest;     // stopping bound on |r|^2 (cg_para%rest, promoted to FP64)
   int maxiter;
   double res[4];   // scratch results (true residual etc.)
@@ -50,13 +51,20 @@ inline int vector_grid(int vh) {
 // doubles); null selects the context's own buffer
 int cg_init(Context *c, CgState *st, double rest, int maxiter);
 int cg_start(Context *c, double2 *r, double2 *p, const double2 *b, CgState *st, double *red = nullptr);
-// more than kMaxParts partials (skip: as the kernel that left them) become one,
+// more than `most` partials (skip: as the kernel that left them) become one,
 // at p + n; otherwise nothing happens
-int shorten_partials(Context *c, const double *&p, int &n, const int *skip);
+int shorten_partials(Context *c, const double *&p, int &n, const int *skip, int most = kMaxParts);
 // the vector updates of iteration k: from the partials of <p, A p>
 // (pa, na of them) to those of |r|^2 (pb, vector_grid(vh) doubles), and on
 int cg_update(Context *c, double2 *r, const double2 *q, CgState *st, int k, const double *pa, int na, double *pb);
-int cg_pupdate(Context *c, double2 *x, double2 *p, const double2 *r, CgState *st, int k, const double *pb);
+// Search directions: p of iteration k is p[k & 3].  Four buffers on lattices
+// that are bound by the bytes of the updates: x then takes up four directions
+// at a time, in the order and with the sums of one at a time.  One (all four
+// the same) elsewhere.
+struct CgRing {
+  double2 *p[4];
+};
+int cg_pupdate(Context *c, double2 *x, const CgRing &ring, const double2 *r, CgState *st, int k, const double *pb);
 int residual(Context *c, double2 *out, const double2 *b, double *res_d, double *red = nullptr);
 int dot_norm(Context *c, const double2 *x, const double2 *y, double *res_d);
 int zero_f64(Context *c, double2 *p, size_t n);

@@ -85,16 +85,25 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(double2 *__restrict__ r, c
                                                       CgState *st, int k, const double *pa, int na, double *pb) {
   const CgSlot c = st->s[k & 1];
   if (c.done) return;
+  // the first operands are on their way while the partials are summed
+  const int step = gridDim.x * blockDim.x;
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  double2 qq = i < n ? q[i] : double2{}, rr = i < n ? r[i] : double2{};
+  asm volatile("" ::: "memory");
   const double pap = partials_total(pa, na);
   if (blockIdx.x == 0 && threadIdx.x == 0) st->pap = pap;
   const double alpha = c.rtr / pap;
   double s = 0.0;
-#pragma unroll 4
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    double2 qq = q[i], rr = r[i];
-    rr.x -= alpha * qq.x; rr.y -= alpha * qq.y;
-    st_cg<NT>(r, i, rr);
-    s += rr.x * rr.x + rr.y * rr.y;
+  while (i < n) {
+    const double2 v = make_double2(rr.x - alpha * qq.x, rr.y - alpha * qq.y);
+    s += v.x * v.x + v.y * v.y;
+    const int j = i + step;
+    if (j < n) {
+      qq = q[j];
+      rr = r[j];
+    }
+    st_cg<NT>(r, i, v);
+    i = j;
   }
   double vals[1] = {s};
   block_partials<1>(vals, pb);
@@ -113,19 +122,71 @@ __global__ __launch_bounds__(kBlock) void k_cg_pupdate(double2 *__restrict__ x, 
     if (first) st->s[~k & 1] = c;
     return;
   }
+  const int step = gridDim.x * blockDim.x;
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  double2 pp = i < n ? p[i] : double2{}, xx = i < n ? x[i] : double2{}, rr = i < n ? r[i] : double2{};
+  asm volatile("" ::: "memory");
   const double rtr = partials_total(pb, nb);
   const double alpha = c.rtr / st->pap, beta = rtr / c.rtr;
   const int iter = c.iter + 1;
   const int done = rtr <= st->rest ? 1 : iter >= st->maxiter ? 2 : 0;
   if (first) st->s[~k & 1] = CgSlot{done ? c.rtr : rtr, rtr, iter, done};
-#pragma unroll 4
+  while (i < n) {
+    const double2 xv = make_double2(xx.x + alpha * pp.x, xx.y + alpha * pp.y);
+    const double2 pv = make_double2(rr.x + beta * pp.x, rr.y + beta * pp.y);
+    const int j = i + step;
+    if (j < n) {
+      pp = p[j];
+      xx = x[j];
+      rr = r[j];
+    }
+    st_cg<NT>(x, i, xv);
+    if (!done) st_cg<NT>(p, i, pv);
+    i = j;
+  }
+}
+
+// the same with the search directions in a ring (CgRing): 24^3x48 44.7 us
+// against 49.3
+__global__ __launch_bounds__(kBlock) void k_cg_pupdate_ring(double2 *__restrict__ x, CgRing ring,
+                                                            const double2 *__restrict__ r, int n, CgState *st, int k,
+                                                            const double *pb, int nb) {
+  const CgSlot c = st->s[k & 1];
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (c.done) {
+    if (first) st->s[~k & 1] = c;
+    return;
+  }
+  const int slot = k & 3;
+  const double *alphas = st->alpha;
+  const double rtr = partials_total(pb, nb);
+  const double alpha = c.rtr / st->pap, beta = rtr / c.rtr;
+  const int iter = c.iter + 1;
+  const int done = rtr <= st->rest ? 1 : iter >= st->maxiter ? 2 : 0;
+  if (first) {
+    st->s[~k & 1] = CgSlot{done ? c.rtr : rtr, rtr, iter, done};
+    st->alpha[slot] = alpha;
+  }
+  const bool take = slot == 3 || done;
+  const double2 *p = ring.p[slot];
+  double2 *pn = ring.p[(k + 1) & 3];
+  double al[3];
+  for (int q = 0; q < 3; q++) al[q] = q < slot ? alphas[q] : 0.0;
+#pragma unroll 2
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    double2 pp = p[i], xx = x[i];
-    xx.x += alpha * pp.x; xx.y += alpha * pp.y;
-    st_cg<NT>(x, i, xx);
+    const double2 pp = p[i];
+    if (take) {
+      double2 xx = x[i];
+      for (int q = 0; q < slot; q++) {
+        const double2 v = ring.p[q][i];
+        xx.x += al[q] * v.x; xx.y += al[q] * v.y;
+      }
+      xx.x += alpha * pp.x; xx.y += alpha * pp.y;
+      SF64::st_nt(x, i, xx);
+    }
     if (!done) {
-      double2 rr = r[i];
-      st_cg<NT>(p, i, make_double2(rr.x + beta * pp.x, rr.y + beta * pp.y));
+      const double2 rr = r[i];
+      SF64::st_nt(pn, i, make_double2(rr.x + beta * pp.x, rr.y + beta * pp.y));
     }
   }
 }
@@ -203,8 +264,8 @@ int cg_start(Context *c, double2 *r, double2 *p, const double2 *b, CgState *st, 
   return HB_OK;
 }
 
-int shorten_partials(Context *c, const double *&p, int &n, const int *skip) {
-  if (n <= kMaxParts) return HB_OK;
+int shorten_partials(Context *c, const double *&p, int &n, const int *skip, int most) {
+  if (n <= most) return HB_OK;
   double *out = const_cast<double *>(p) + n;
   k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(p, n, skip, FinStore1{out});
   HB_HIP(hipGetLastError());
@@ -221,10 +282,14 @@ int cg_update(Context *c, double2 *r, const double2 *q, CgState *st, int k, cons
   return HB_OK;
 }
 
-int cg_pupdate(Context *c, double2 *x, double2 *p, const double2 *r, CgState *st, int k, const double *pb) {
+int cg_pupdate(Context *c, double2 *x, const CgRing &ring, const double2 *r, CgState *st, int k, const double *pb) {
   const int vh = c->g.vh;
-  const auto f = operator_policy<SF64, SF64R>(vh) == kNT ? k_cg_pupdate<true> : k_cg_pupdate<false>;
-  f<<<vector_grid(vh), kBlock, 0, c->stream>>>(x, p, r, 12 * vh, st, k, pb, vector_grid(vh));
+  if (ring.p[1] != ring.p[0]) {
+    k_cg_pupdate_ring<<<vector_grid(vh), kBlock, 0, c->stream>>>(x, ring, r, 12 * vh, st, k, pb, vector_grid(vh));
+  } else {
+    const auto f = operator_policy<SF64, SF64R>(vh) == kNT ? k_cg_pupdate<true> : k_cg_pupdate<false>;
+    f<<<vector_grid(vh), kBlock, 0, c->stream>>>(x, ring.p[0], r, 12 * vh, st, k, pb, vector_grid(vh));
+  }
   HB_HIP(hipGetLastError());
   return HB_OK;
 }

@@ -166,14 +166,14 @@ int cg_f64_run(Context *c, const CgWork &w, int op, double kappa, double rho, do
   HB_TRY(cg_init(c, st, (double)rest, maxiter));
   // r = A x; r = b - r; p = r; rtr_old = |r|^2
   HB_TRY(apply_f64(c, op, kappa, rho, w.r, x, w.t, w.y, nullptr, nullptr, w.recon));
-  HB_TRY(cg_start(c, w.r, w.p, b, st, w.red));
+  HB_TRY(cg_start(c, w.r, w.p.p[0], b, st, w.red));
   int nmv = 1;
   if (maxiter == 0) {
     // the reference's loop body never runs: niter = 0, x unchanged
     HB_HIP(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
     HB_HIP(hipStreamSynchronize(c->stream));
   } else {
-    // iterations in chunks (of even length, so that each ends in slot 0); every
+    // iterations in chunks (a multiple of four, so that each ends in slot 0); every
     // kernel returns immediately once done != 0, so the chunk length only sets
     // how often the host looks at the state
     const int na = w.recon ? dslash_grid<SF64, SF64R>(c->g.vh) : dslash_grid<SF64, SF64>(c->g.vh);
@@ -181,7 +181,7 @@ int cg_f64_run(Context *c, const CgWork &w, int op, double kappa, double rho, do
     int chunk = 8;
     for (;;) {
       for (int k = 0; k < chunk; k++) {
-        HB_TRY(apply_f64(c, op, kappa, rho, w.q, w.p, w.t, w.y, pa, &st->s[k & 1].done, w.recon));
+        HB_TRY(apply_f64(c, op, kappa, rho, w.q, w.p.p[k & 3], w.t, w.y, pa, &st->s[k & 1].done, w.recon));
         const double *sum = pa;
         int nsum = na;
         HB_TRY(shorten_partials(c, sum, nsum, &st->s[k & 1].done));
@@ -222,7 +222,11 @@ int cg_f64(Context *c, int op, double kappa, double rho, double2 *x, const doubl
   w.t = spinor_scratch(c, SLOT_T, &rc); HB_TRY(rc);
   w.y = spinor_scratch(c, SLOT_Y, &rc); HB_TRY(rc);
   w.r = spinor_scratch(c, SLOT_R, &rc); HB_TRY(rc);
-  w.p = spinor_scratch(c, SLOT_P, &rc); HB_TRY(rc);
+  const bool ring = operator_policy<SF64, SF64R>(c->g.vh) == kNT;
+  for (int q = 0; q < 4; q++) {
+    w.p.p[q] = spinor_scratch(c, ring && q > 0 ? SLOT_P1 + q - 1 : SLOT_P, &rc);
+    HB_TRY(rc);
+  }
   w.q = spinor_scratch(c, SLOT_Q, &rc); HB_TRY(rc);
   w.st = static_cast<CgState *>(scratch(c, SLOT_STATE, sizeof(CgState), &rc)); HB_TRY(rc);
   w.red = c->red;

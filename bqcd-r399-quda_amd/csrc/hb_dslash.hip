@@ -110,6 +110,7 @@ __global__ __launch_bounds__(64 * NW) void k_dslash_split(DslashArgs<S, G> a) {
   const int i = xcd_block(blockIdx.x, gridDim.x) * 64 + lane;
   const bool active = i < vh;
   constexpr bool kClovSum = EPI == EPI_CLINV || EPI == EPI_SOLVE, kClovX0 = EPI == EPI_MTIL || EPI == EPI_MTDOT;
+  CloverFetch<G> cf;
   V acc[12], x0[12], y[6], dv[12];
 #pragma unroll
   for (int k = 0; k < 12; k++) acc[k] = cmk<V>((A)0, (A)0);
@@ -123,21 +124,20 @@ __global__ __launch_bounds__(64 * NW) void k_dslash_split(DslashArgs<S, G> a) {
     }
 #undef HB_PART
     if constexpr (kClovX0) {
-      if (w < 2) {
-        load_spinor<S>(x0, a.x0, i, vh);
-        if (a.C) {
-          V xp[6];
+      if (w < 2) load_spinor<S>(x0, a.x0, i, vh);
+      if (w < 2 && a.C) {
+        cf.template load<POL>(a.C, e, w, i, vh);
+        V xp[6];
 #pragma unroll
-          for (int m = 0; m < 6; m++) xp[m] = w == 0 ? cadd(x0[m], x0[m + 6]) : csub(x0[m], x0[m + 6]);
-          clover_block_apply<G, 0, POL>(y, xp, a.C, a.Cn, e, w, i, vh);
-          if (w == 1) {
+        for (int m = 0; m < 6; m++) xp[m] = w == 0 ? cadd(x0[m], x0[m + 6]) : csub(x0[m], x0[m + 6]);
+        cf.template apply<0>(y, xp);
+        if (w == 1) {
 #pragma unroll
-            for (int m = 0; m < 6; m++) y1s[m][lane] = y[m];
-          }
+          for (int m = 0; m < 6; m++) y1s[m][lane] = y[m];
         }
-        if (EPI == EPI_MTDOT && w == 0) load_spinor<S>(dv, a.dotv, i, vh);
       }
     }
+    if (EPI == EPI_MTDOT && w == 0) load_spinor<S>(dv, a.dotv, i, vh);
 #pragma unroll
     for (int k = 0; k < 12; k++) part[w][k][lane] = acc[k];
   }
@@ -152,10 +152,11 @@ __global__ __launch_bounds__(64 * NW) void k_dslash_split(DslashArgs<S, G> a) {
       HB_SCHED_FENCE();  // one part's reads in flight at a time (registers)
     }
     if (kClovSum && a.C) {
+      cf.template load<POL>(a.C, e, w, i, vh);
       V xp[6];
 #pragma unroll
       for (int m = 0; m < 6; m++) xp[m] = w == 0 ? cadd(acc[m], acc[m + 6]) : csub(acc[m], acc[m + 6]);
-      clover_block_apply<G, EPI == EPI_SOLVE, POL>(y, xp, a.C, a.Cn, e, w, i, vh);
+      cf.template apply<EPI == EPI_SOLVE>(y, xp);
       if (w == 1) {
 #pragma unroll
         for (int m = 0; m < 6; m++) y1s[m][lane] = y[m];

@@ -25,7 +25,10 @@ struct MixSlot {
 struct MixState {
   MixSlot s[2];
   double pap;           // <p, A p> of the iteration, from the r update for the p update
-  double beta;          // of the restart after a reliable update
+  double alpha[4];      // of the iterations whose x_lo updates are pending (MixRing)
+  double beta;          // of the p update or of the restart after a reliable update
+  int go;               // the iteration ran: its p update is due
+  int cur;              // slot of the ring that holds the search direction at a reliable update
   double rp_re, rp_im;  // <r, p> / |r|^2 after a reliable update
   double rest, delta;
   int max_inner, maxiter;
@@ -106,51 +109,96 @@ __global__ void k_spinor_to_f64(double2 *__restrict__ dst, SpinorPtr<S> src, int
 template <class S> constexpr bool kLinear = !S::kNorm;
 template <class S> inline int mix_count(int vh) { return kLinear<S> ? 12 * vh : vh; }
 template <class S> inline int mix_block(int vh) { return !kLinear<S> && vh <= (1 << 16) ? 64 : kBlock; }
+// (linear fields in at most 2048 blocks that go round)
 template <class S> inline int mix_grid(int vh) {
   const int b = nblocks(mix_count<S>(vh), mix_block<S>(vh));
-  return b < 2048 ? b : 2048;
+  return kLinear<S> && b > 2048 ? 2048 : b;
+}
+
+// The blocks sum the partials of a reduction themselves while their first
+// operands are on their way (SUM), except in the site kernels of large
+// lattices, which hold a whole site's operands in registers meanwhile and wait
+// at the barrier: 16-bit updates at 32^3x64 74 us, with a finalize launch for
+// each sum 64 + 8 us; at 12^3x24 7.2 against 6.3 + 5 us.
+template <class S> inline bool mix_sum(int vh) { return kLinear<S> || vh <= (1 << 18); }
+template <bool SUM> __device__ __forceinline__ double mix_total(const double *p, int n) {
+  if constexpr (SUM) return partials_total(p, n);
+  else return *p;
+}
+
+// what a thread works on: one number, or a site's twelve
+template <class S> constexpr int kNums = kLinear<S> ? 1 : 12;
+template <class S>
+__device__ __forceinline__ void load_nums(typename S::V (&v)[kNums<S>], const SpinorPtr<S> &f, int i, int n) {
+  if constexpr (kLinear<S>) v[0] = S::ld(f.p, i);
+  else load_spinor<S>(v, f, i, n);
+}
+template <class S>
+__device__ __forceinline__ void store_nums(const SpinorPtr<S> &f, int i, int n, const typename S::V (&v)[kNums<S>]) {
+  if constexpr (kLinear<S>) S::st(f.p, i, v[0]);
+  else store_spinor<S>(f, i, n, v);
 }
 
 // alpha = rtr / pAp; r -= alpha q; partial sums of |r|^2
-template <class S>
+template <class S, bool SUM>
 __global__ __launch_bounds__(kBlock) void k_mix_update(SpinorPtr<S> r, SpinorPtr<S> q, int n, MixState *st, int k,
                                                        const double *pa, int na, double *pb) {
   using V = typename S::V;
   const MixSlot c = st->s[k & 1];
   if (c.flag) return;
-  const double pap = partials_total(pa, na);
+  // the first operands are on their way while the partials are summed
+  const int step = gridDim.x * blockDim.x;
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  V qv[kNums<S>], rv[kNums<S>];
+  if (SUM && i < n) {
+    load_nums<S>(qv, q, i, n);
+    load_nums<S>(rv, r, i, n);
+    asm volatile("" ::: "memory");
+  }
+  const double pap = mix_total<SUM>(pa, na);
   if (blockIdx.x == 0 && threadIdx.x == 0) st->pap = pap;
   const float alpha = (float)(c.rtr / pap);
   double s = 0.0;
-#pragma unroll(kLinear<S> ? 4 : 1)
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    if constexpr (kLinear<S>) {
-      const V qv = S::ld(q.p, i);
-      V rv = S::ld(r.p, i);
-      rv.x -= alpha * qv.x;
-      rv.y -= alpha * qv.y;
-      s += (double)rv.x * rv.x + (double)rv.y * rv.y;
-      S::st(r.p, i, rv);
-    } else {
-      V qv[12], rv[12];
-      load_spinor<S>(qv, q, i, n);
-      load_spinor<S>(rv, r, i, n);
+  if (!SUM && i < n) {
+    load_nums<S>(qv, q, i, n);
+    load_nums<S>(rv, r, i, n);
+  }
+  while (i < n) {
+    V v[kNums<S>];
 #pragma unroll
-      for (int k = 0; k < 12; k++) {
-        rv[k].x -= alpha * qv[k].x;
-        rv[k].y -= alpha * qv[k].y;
-        s += (double)rv[k].x * rv[k].x + (double)rv[k].y * rv[k].y;
-      }
-      store_spinor<S>(r, i, n, rv);
+    for (int m = 0; m < kNums<S>; m++) {
+      v[m].x = rv[m].x - alpha * qv[m].x;
+      v[m].y = rv[m].y - alpha * qv[m].y;
+      s += (double)v[m].x * v[m].x + (double)v[m].y * v[m].y;
     }
+    const int j = i + step;
+    if (kLinear<S> && j < n) {
+      load_nums<S>(qv, q, j, n);
+      load_nums<S>(rv, r, j, n);
+    }
+    store_nums<S>(r, i, n, v);
+    i = kLinear<S> ? j : n;
   }
   double vals[1] = {s};
   block_partials<1>(vals, pb);
 }
 
-// iterated |r|^2 -> reliable-update decision or beta (cg.F90:109-115);
-// x_lo += alpha p, then p = r + beta p (unless a reliable update or the end is
-// due)
+// iterated |r|^2 -> reliable-update decision or beta (cg.F90:109-115): the slot
+// of the next iteration; returns whether it goes on
+__device__ __forceinline__ bool mix_decide(MixSlot &d, const MixSlot &c, const MixState *st, double rn) {
+  const double rnorm = sqrt(rn);
+  d = c;
+  d.iter += 1;
+  d.since += 1;
+  if (rnorm > d.maxr) d.maxr = rnorm;
+  const bool next = !(rn <= st->rest || rnorm < st->delta * d.maxr || d.since >= st->max_inner || d.iter >= st->maxiter);
+  if (next) d.rtr = rn;
+  else d.flag = 1;
+  return next;
+}
+
+// small lattices: x_lo += alpha p, then p = r + beta p (unless a reliable
+// update or the end is due)
 template <class S>
 __global__ __launch_bounds__(kBlock) void k_mix_pupdate(SpinorPtr<S> p, SpinorPtr<S> r, float2 *__restrict__ xlo, int n,
                                                         MixState *st, int k, const double *pb, int nb) {
@@ -161,54 +209,100 @@ __global__ __launch_bounds__(kBlock) void k_mix_pupdate(SpinorPtr<S> p, SpinorPt
     if (first) st->s[~k & 1] = c;
     return;
   }
+  const int step = gridDim.x * blockDim.x;
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  V pv[kNums<S>], rv[kNums<S>];
+  float2 xv[kNums<S>];
+  const auto load = [&](int j) {
+    load_nums<S>(pv, p, j, n);
+    load_nums<S>(rv, r, j, n);
+#pragma unroll
+    for (int m = 0; m < kNums<S>; m++) xv[m] = xlo[(size_t)m * n + j];
+  };
+  if (i < n) load(i);
+  asm volatile("" ::: "memory");
   const double rn = partials_total(pb, nb);
-  const double rnorm = sqrt(rn);
-  MixSlot d = c;
-  d.iter += 1;
-  d.since += 1;
-  if (rnorm > d.maxr) d.maxr = rnorm;
-  const bool next = !(rn <= st->rest || rnorm < st->delta * d.maxr || d.since >= st->max_inner || d.iter >= st->maxiter);
-  if (next) d.rtr = rn;
-  else d.flag = 1;
+  MixSlot d;
+  const bool next = mix_decide(d, c, st, rn);
   const float alpha = (float)(c.rtr / st->pap);
   const float beta = (float)(rn / c.rtr);
   if (first) st->s[~k & 1] = d;
-#pragma unroll(kLinear<S> ? 4 : 1)
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    if constexpr (kLinear<S>) {
-      V pv = S::ld(p.p, i);
-      float2 xv = xlo[i];
-      xv.x += alpha * pv.x;
-      xv.y += alpha * pv.y;
-      xlo[i] = xv;
-      if (next) {
-        const V rv = S::ld(r.p, i);
-        pv.x = rv.x + beta * pv.x;
-        pv.y = rv.y + beta * pv.y;
-        S::st(p.p, i, pv);
-      }
-    } else {
-      V pv[12];
-      load_spinor<S>(pv, p, i, n);
+  while (i < n) {
+    V v[kNums<S>];
 #pragma unroll
-      for (int k = 0; k < 12; k++) {
-        float2 xv = xlo[(size_t)k * n + i];
-        xv.x += alpha * pv[k].x;
-        xv.y += alpha * pv[k].y;
-        xlo[(size_t)k * n + i] = xv;
-      }
-      if (next) {
-        V rv[12];
-        load_spinor<S>(rv, r, i, n);
+    for (int m = 0; m < kNums<S>; m++) {
+      xlo[(size_t)m * n + i] = make_float2(xv[m].x + alpha * pv[m].x, xv[m].y + alpha * pv[m].y);
+      v[m].x = rv[m].x + beta * pv[m].x;
+      v[m].y = rv[m].y + beta * pv[m].y;
+    }
+    if (next) store_nums<S>(p, i, n, v);
+    i = kLinear<S> ? i + step : n;
+    if (kLinear<S> && i < n) load(i);
+  }
+}
+
+// Large lattices are bound by the bytes of the vector updates, half of them
+// x_lo's.  Their search directions go round four buffers, p of iteration k in
+// slot k & 3, and x_lo takes up four of them at a time (or those there are,
+// when a reliable update is due): the same sums in the same order.  16-bit
+// storage at 32^3x64: 34.9 us a launch against 43.0, an iteration 474 against 493.
+template <class S> struct MixRing {
+  SpinorPtr<S> p[4];
+};
+struct FinMixStep {
+  MixState *st;
+  int k;
+  __device__ void operator()(const double (&t)[1]) const {
+    const MixSlot c = st->s[k & 1];
+    MixSlot d = c;
+    st->go = c.flag == 0;
+    if (c.flag == 0) {
+      mix_decide(d, c, st, t[0]);
+      st->alpha[k & 3] = c.rtr / st->pap;
+      st->beta = t[0] / c.rtr;
+      st->cur = k & 3;
+    }
+    st->s[~k & 1] = d;
+  }
+};
+template <class S>
+__global__ __launch_bounds__(kBlock) void k_mix_pupdate_ring(MixRing<S> ring, SpinorPtr<S> r, float2 *__restrict__ xlo,
+                                                             int n, const MixState *st, int k) {
+  using V = typename S::V;
+  if (!st->go) return;
+  const bool next = st->s[~k & 1].flag == 0;
+  const int slot = k & 3;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  V pv[12];
+  if (slot == 3 || !next) {
+    float2 x[12];
 #pragma unroll
-        for (int k = 0; k < 12; k++) {
-          pv[k].x = rv[k].x + beta * pv[k].x;
-          pv[k].y = rv[k].y + beta * pv[k].y;
-        }
-        store_spinor<S>(p, i, n, pv);
+    for (int m = 0; m < 12; m++) x[m] = xlo[(size_t)m * n + i];
+    for (int q = 0; q <= slot; q++) {
+      const float alpha = (float)st->alpha[q];
+      load_spinor<S>(pv, ring.p[q], i, n);
+#pragma unroll
+      for (int m = 0; m < 12; m++) {
+        x[m].x += alpha * pv[m].x;
+        x[m].y += alpha * pv[m].y;
       }
     }
+#pragma unroll
+    for (int m = 0; m < 12; m++) xlo[(size_t)m * n + i] = x[m];
+  } else {
+    load_spinor<S>(pv, ring.p[slot], i, n);
   }
+  if (!next) return;
+  const float beta = (float)st->beta;
+  V rv[12];
+  load_spinor<S>(rv, r, i, n);
+#pragma unroll
+  for (int m = 0; m < 12; m++) {
+    pv[m].x = rv[m].x + beta * pv[m].x;
+    pv[m].y = rv[m].y + beta * pv[m].y;
+  }
+  store_spinor<S>(ring.p[(k + 1) & 3], i, n, pv);
 }
 
 // ---- reliable update kernels ------------------------------------------------------
@@ -279,7 +373,7 @@ struct FinMixTrue {
 #define HB_MIX_REORTH 1
 #endif
 template <class S>
-__global__ __launch_bounds__(kBlock) void k_mix_rdotp(SpinorPtr<S> p, SpinorPtr<S> r, int vh, const MixState *st,
+__global__ __launch_bounds__(kBlock) void k_mix_rdotp(MixRing<S> ring, SpinorPtr<S> r, int vh, const MixState *st,
                                                       double *partials) {
   using V = typename S::V;
   if (st->s[0].flag) return;
@@ -287,7 +381,7 @@ __global__ __launch_bounds__(kBlock) void k_mix_rdotp(SpinorPtr<S> p, SpinorPtr<
   double re = 0.0, im = 0.0;
   if (i < vh) {
     V pv[12], rv[12];
-    load_spinor<S>(pv, p, i, vh);
+    load_spinor<S>(pv, ring.p[st->cur], i, vh);
     load_spinor<S>(rv, r, i, vh);
 #pragma unroll
     for (int k = 0; k < 12; k++) {  // conj(r) p
@@ -310,7 +404,7 @@ struct FinMixRdotp {
 // p = r_lo + beta (p - rp r_lo) after a reliable update (rp = <r, p>/|r|^2, or
 // 0; beta = 0 at the start: p = r)
 template <class S>
-__global__ __launch_bounds__(kBlock) void k_mix_prestart(SpinorPtr<S> p, SpinorPtr<S> r, int vh,
+__global__ __launch_bounds__(kBlock) void k_mix_prestart(MixRing<S> ring, SpinorPtr<S> r, int vh,
                                                          const MixState *st) {
   using V = typename S::V;
   if (st->s[0].flag) return;
@@ -321,7 +415,7 @@ __global__ __launch_bounds__(kBlock) void k_mix_prestart(SpinorPtr<S> p, SpinorP
   V pv[12], rv[12];
   load_spinor<S>(rv, r, i, vh);
   if (beta != 0.f) {
-    load_spinor<S>(pv, p, i, vh);
+    load_spinor<S>(pv, ring.p[st->cur], i, vh);
   } else {
 #pragma unroll
     for (int k = 0; k < 12; k++) pv[k] = cmk<V>(0.f, 0.f);
@@ -333,7 +427,7 @@ __global__ __launch_bounds__(kBlock) void k_mix_prestart(SpinorPtr<S> p, SpinorP
     pv[k].x = rv[k].x + beta * ux;
     pv[k].y = rv[k].y + beta * uy;
   }
-  store_spinor<S>(p, i, vh, pv);
+  store_spinor<S>(ring.p[0], i, vh, pv);
 }
 
 // ---- low-precision copies of links and clover ------------------------------------
@@ -446,6 +540,13 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
   float2 *xlo = static_cast<float2 *>(scratch(c, SLOT_MIX1, sizeof(float2) * 12 * (size_t)vh, &rc)); HB_TRY(rc);
   // low-precision fields (norm slots follow SLOT_LPN)
   SpinorPtr<S> p = SpinorAlloc<S>::get(c, SLOT_LP0, SLOT_LPN, &rc); HB_TRY(rc);
+  const bool sums = mix_sum<S>(vh);
+  MixRing<S> ring{{p, p, p, p}};
+  if (!sums)
+    for (int q = 1; q < 4; q++) {
+      ring.p[q] = SpinorAlloc<S>::get(c, SLOT_LPR + 2 * q, SLOT_LPR + 2 * q + 1, &rc);
+      HB_TRY(rc);
+    }
   SpinorPtr<S> r = SpinorAlloc<S>::get(c, SLOT_LP1, SLOT_LPN1, &rc); HB_TRY(rc);
   SpinorPtr<S> q = SpinorAlloc<S>::get(c, SLOT_LP2, SLOT_LPN2, &rc); HB_TRY(rc);
   SpinorPtr<S> t = SpinorAlloc<S>::get(c, SLOT_LP3, SLOT_LPN3, &rc); HB_TRY(rc);
@@ -478,11 +579,11 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
     k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(c->red, nblocks(vh), nullptr, FinMixTrue{st, first});
     HB_HIP(hipGetLastError());
     if (!first && HB_MIX_REORTH) {
-      k_mix_rdotp<S><<<nblocks(vh), kBlock, 0, c->stream>>>(p, r, vh, st, c->red);
+      k_mix_rdotp<S><<<nblocks(vh), kBlock, 0, c->stream>>>(ring, r, vh, st, c->red);
       k_finalize<2><<<1, kFinThreads, 0, c->stream>>>(c->red, nblocks(vh), &st->s[0].flag, FinMixRdotp{st});
       HB_HIP(hipGetLastError());
     }
-    k_mix_prestart<S><<<nblocks(vh), kBlock, 0, c->stream>>>(p, r, vh, st);
+    k_mix_prestart<S><<<nblocks(vh), kBlock, 0, c->stream>>>(ring, r, vh, st);
     HB_HIP(hipGetLastError());
     nmv++;
     return HB_OK;
@@ -491,18 +592,24 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
   // partials of <p, A p> and of |r|^2
   const int na = dslash_grid<S, G>(vh), n = mix_count<S>(vh), grid = mix_grid<S>(vh), block = mix_block<S>(vh);
   double *pa = c->red, *pb = c->red + na + 1;
-  int chunk = 8;  // iterations between looks at the state; even, so that each chunk ends in slot 0
+  int chunk = 8;  // iterations between looks at the state; a multiple of four, so that each chunk ends in slot 0
   for (;;) {
     for (int k = 0; k < chunk; k++) {
       const int *skip = &st->s[k & 1].flag;
-      HB_TRY((mtil_lp<S, G>(c, false, kappa, r_op, y, p, t, nullptr, SpinorPtr<S>{}, skip)));
-      HB_TRY((mtil_lp<S, G>(c, true, kappa, r_op, q, y, t, pa, p, skip)));
+      const SpinorPtr<S> pk = ring.p[k & 3];
+      HB_TRY((mtil_lp<S, G>(c, false, kappa, r_op, y, pk, t, nullptr, SpinorPtr<S>{}, skip)));
+      HB_TRY((mtil_lp<S, G>(c, true, kappa, r_op, q, y, t, pa, pk, skip)));
       const double *sum = pa;
       int nsum = na;
-      HB_TRY(shorten_partials(c, sum, nsum, skip));
-      k_mix_update<S><<<grid, block, 0, c->stream>>>(r, q, n, st, k, sum, nsum, pb);
-      HB_HIP(hipGetLastError());
-      k_mix_pupdate<S><<<grid, block, 0, c->stream>>>(p, r, xlo, n, st, k, pb, grid);
+      HB_TRY(shorten_partials(c, sum, nsum, skip, sums ? kMaxParts : 1));
+      if (sums) {
+        k_mix_update<S, true><<<grid, block, 0, c->stream>>>(r, q, n, st, k, sum, nsum, pb);
+        k_mix_pupdate<S><<<grid, block, 0, c->stream>>>(p, r, xlo, n, st, k, pb, grid);
+      } else {
+        k_mix_update<S, false><<<grid, block, 0, c->stream>>>(r, q, n, st, k, sum, nsum, pb);
+        k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(pb, grid, nullptr, FinMixStep{st, k});
+        if constexpr (!kLinear<S>) k_mix_pupdate_ring<S><<<grid, block, 0, c->stream>>>(ring, r, xlo, n, st, k);
+      }
       HB_HIP(hipGetLastError());
     }
     HB_HIP(hipMemcpyAsync(hs, st, sizeof(MixState), hipMemcpyDeviceToHost, c->stream));

@@ -27,8 +27,9 @@ double *multi_partials(Context *c, int NR, int *rc);
 
 struct MultiState {
   double rtr[16], pap[16], beta[16], maxr[16], rest[16], res[16];
-  double alpha[16];  // of each RHS's last iteration, for its x_lo update
-  int xpend[16];     // that iteration ran: its x_lo update is due
+  double alpha[4][16];  // of each RHS's last iterations, for its x_lo update (MultiRing)
+  int xpend[16];        // the iteration ran: its p update is due
+  int cur[16];          // slot of the ring that holds its search direction at a reliable update
   int flag[16];   // 0 iterate, 1 reliable update due, 2 converged, 3 maxiter, 4 unused lane
   int iter[16], since[16], nrel[16];
   double delta;
@@ -196,40 +197,67 @@ __global__ __launch_bounds__(kBlock) void k_dslash_multi(MultiArgs<S, G> a) {
   }
 }
 
-// per-RHS finalize functors ------------------------------------------------------
-template <int NR> struct FinMultiStore {
+// per-RHS sums ---------------------------------------------------------------------
+// as k_finalize, with each RHS's sum formed by waves of its own and taken to
+// f(k, sum) by a thread of its own: one after the other the NR sums, and the
+// divisions on the systems' scalars after them, are NR chains of L2 latencies
+// (4 RHS at 24^3x48: 7.7 and 6.1 us, 10.9 and 7.0 one after the other)
+template <int NR, class F>
+__global__ __launch_bounds__(kFinThreads) void k_finalize_each(const double *__restrict__ partials, int nparts, F f) {
+  constexpr int W = kFinThreads / 64 / NR, U = 8;  // waves per RHS, loads in flight
+  __shared__ double lds[NR][W];
+  const int lane = threadIdx.x & 63, k = ((int)threadIdx.x >> 6) / W, w = ((int)threadIdx.x >> 6) % W;
+  if (k < NR) {
+    const double *p = partials + (size_t)k * nparts;
+    double a[U] = {};
+    int b = w * 64 + lane;
+    for (; b + (U - 1) * W * 64 < nparts; b += U * W * 64) {
+#pragma unroll
+      for (int u = 0; u < U; u++) a[u] += p[b + u * W * 64];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (b + u * W * 64 < nparts) a[u] += p[b + u * W * 64];
+    const double s = wave_sum(((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7])));
+    if (lane == 0) lds[k][w] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x < NR) {
+    double s = 0.0;
+    for (int q = 0; q < W; q++) s += lds[threadIdx.x][q];
+    f(threadIdx.x, s);
+  }
+}
+
+struct FinMultiStore {
   double *out;
   const int *flag;
-  __device__ void operator()(const double (&t)[NR]) const {
-#pragma unroll
-    for (int k = 0; k < NR; k++)
-      if (flag[k] == 0) out[k] = t[k];
+  __device__ void operator()(int k, double t) const {
+    if (flag[k] == 0) out[k] = t;
   }
 };
 
-template <int NR> struct FinMultiUpdate {
+struct FinMultiUpdate {
   MultiState *st;
-  __device__ void operator()(const double (&t)[NR]) const {
-#pragma unroll
-    for (int k = 0; k < NR; k++) {
-      if (st->flag[k] != 0) {
-        st->xpend[k] = 0;  // the p update of a skipped iteration adds nothing to x_lo
-        continue;
-      }
-      st->alpha[k] = st->rtr[k] / st->pap[k];  // the alpha of k_multi_update
-      st->xpend[k] = 1;
-      const double rn = t[k];
-      st->iter[k] += 1;
-      st->since[k] += 1;
-      const double rnorm = sqrt(rn);
-      if (rnorm > st->maxr[k]) st->maxr[k] = rnorm;
-      if (rn <= st->rest[k] || rnorm < st->delta * st->maxr[k] || st->since[k] >= st->max_inner ||
-          st->iter[k] >= st->maxiter) {
-        st->flag[k] = 1;
-      } else {
-        st->beta[k] = rn / st->rtr[k];
-        st->rtr[k] = rn;
-      }
+  int slot;  // of the iteration in the ring
+  __device__ void operator()(int k, double rn) const {
+    if (st->flag[k] != 0) {
+      st->xpend[k] = 0;  // the p update of a skipped iteration adds nothing to x_lo
+      return;
+    }
+    st->alpha[slot][k] = st->rtr[k] / st->pap[k];  // the alpha of k_multi_update
+    st->xpend[k] = 1;
+    st->cur[k] = slot;
+    st->iter[k] += 1;
+    st->since[k] += 1;
+    const double rnorm = sqrt(rn);
+    if (rnorm > st->maxr[k]) st->maxr[k] = rnorm;
+    if (rn <= st->rest[k] || rnorm < st->delta * st->maxr[k] || st->since[k] >= st->max_inner ||
+        st->iter[k] >= st->maxiter) {
+      st->flag[k] = 1;
+    } else {
+      st->beta[k] = rn / st->rtr[k];
+      st->rtr[k] = rn;
     }
   }
 };
@@ -267,27 +295,43 @@ __global__ __launch_bounds__(kBlock) void k_multi_update(SpinorPtr<S> r, SpinorP
   block_partials<NR>(vals, partials);
 }
 
-// x_lo += alpha p for every RHS whose iteration ran, then p = r + beta p for
-// those that go on
+// p = r + beta p for every RHS that goes on.  Search directions go round four
+// buffers, and x_lo takes up four of them at a time, or those there are when a
+// reliable update of the RHS is due (the same sums in the same order): half of
+// the bytes of this kernel were x_lo's.  4 RHS at 24^3x48: 70 -> 57 us
+template <class S> struct MultiRing {
+  SpinorPtr<S> p[4];
+};
 template <class S, int NR>
-__global__ __launch_bounds__(kBlock) void k_multi_pupdate(SpinorPtr<S> p, SpinorPtr<S> r, float2 *__restrict__ xlo,
-                                                          int vh, const MultiState *st) {
+__global__ __launch_bounds__(kBlock) void k_multi_pupdate(MultiRing<S> ring, SpinorPtr<S> r, float2 *__restrict__ xlo,
+                                                          int vh, const MultiState *st, int slot) {
   using V = typename S::V;
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
   const int site = tid / NR, k0 = tid - site * NR;
   if (site >= vh || !st->xpend[k0]) return;
   const int vhe = vh * NR;
-  const float alpha = (float)st->alpha[k0], beta = (float)st->beta[k0];
+  const bool next = st->flag[k0] == 0;
   V pv[12];
-  load_spinor<S>(pv, p, tid, vhe);
+  if (slot == 3 || !next) {
+    float2 x[12];
 #pragma unroll
-  for (int k = 0; k < 12; k++) {
-    float2 xv = xlo[(size_t)k * vhe + tid];
-    xv.x += alpha * pv[k].x;
-    xv.y += alpha * pv[k].y;
-    xlo[(size_t)k * vhe + tid] = xv;
+    for (int k = 0; k < 12; k++) x[k] = xlo[(size_t)k * vhe + tid];
+    for (int q = 0; q <= slot; q++) {
+      const float alpha = (float)st->alpha[q][k0];
+      load_spinor<S>(pv, ring.p[q], tid, vhe);
+#pragma unroll
+      for (int k = 0; k < 12; k++) {
+        x[k].x += alpha * pv[k].x;
+        x[k].y += alpha * pv[k].y;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 12; k++) xlo[(size_t)k * vhe + tid] = x[k];
+  } else {
+    load_spinor<S>(pv, ring.p[slot], tid, vhe);
   }
-  if (st->flag[k0] != 0) return;
+  if (!next) return;
+  const float beta = (float)st->beta[k0];
   V rv[12];
   load_spinor<S>(rv, r, tid, vhe);
 #pragma unroll
@@ -295,7 +339,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_pupdate(SpinorPtr<S> p, Spinor
     pv[k].x = rv[k].x + beta * pv[k].x;
     pv[k].y = rv[k].y + beta * pv[k].y;
   }
-  store_spinor<S>(p, tid, vhe, pv);
+  store_spinor<S>(ring.p[(slot + 1) & 3], tid, vhe, pv);
 }
 
 // reliable update of RHS k0: x += x_lo[k0]; x_lo[k0] = 0
@@ -357,7 +401,7 @@ struct FinMultiTrue {
 };
 
 template <class S, int NR>
-__global__ __launch_bounds__(kBlock) void k_multi_prestart(SpinorPtr<S> p, SpinorPtr<S> r, int vh,
+__global__ __launch_bounds__(kBlock) void k_multi_prestart(MultiRing<S> ring, SpinorPtr<S> r, int vh,
                                                            int k0, const MultiState *st) {
   using V = typename S::V;
   if (st->flag[k0] != 0) return;
@@ -367,7 +411,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_prestart(SpinorPtr<S> p, Spino
   const float beta = (float)st->beta[k0];
   V pv[12], rv[12];
   load_spinor<S>(rv, r, ie, vhe);
-  if (beta != 0.f) load_spinor<S>(pv, p, ie, vhe);
+  if (beta != 0.f) load_spinor<S>(pv, ring.p[st->cur[k0]], ie, vhe);
   else {
 #pragma unroll
     for (int k = 0; k < 12; k++) pv[k] = cmk<V>(0.f, 0.f);
@@ -377,7 +421,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_prestart(SpinorPtr<S> p, Spino
     pv[k].x = rv[k].x + beta * pv[k].x;
     pv[k].y = rv[k].y + beta * pv[k].y;
   }
-  store_spinor<S>(p, ie, vhe, pv);
+  store_spinor<S>(ring.p[0], ie, vhe, pv);
 }
 
 // conversions of the per-group clover fields --------------------------------------
@@ -465,8 +509,7 @@ int launch_multi_dslash(Context *c, const MultiArgs<S, G> &a, bool dag, int epi)
   if (operator_policy<S, G>(c->g.vh, NR) == kNT) launch_multi_pol<S, G, NR, kNT>(c, a, dag, epi);
   else launch_multi_pol<S, G, NR, 0>(c, a, dag, epi);
   if (epi == EPI_MTDOT)
-    k_finalize<NR><<<1, kFinThreads, 0, c->stream>>>(a.partials, grid, nullptr,
-                                            FinMultiStore<NR>{a.dot_out, a.flag});
+    k_finalize_each<NR><<<1, kFinThreads, 0, c->stream>>>(a.partials, grid, FinMultiStore{a.dot_out, a.flag});
   HB_HIP(hipGetLastError());
   return HB_OK;
 }
@@ -572,6 +615,11 @@ int cg_multi_block(Context *c, const MultiPlan &plan, const MultiFields<S, G> &f
   const int vh = c->g.vh, nb = (int)idx.size();
   int rc = 0;
   SpinorPtr<S> p = block_field<S>(c, SLOT_MULTI + 0, SLOT_MULTI + 10, NR, &rc); HB_TRY(rc);
+  MultiRing<S> ring{{p, p, p, p}};
+  for (int q = 1; q < 4; q++) {
+    ring.p[q] = block_field<S>(c, SLOT_MULTI_RING + 2 * q - 2, SLOT_MULTI_RING + 2 * q - 1, NR, &rc);
+    HB_TRY(rc);
+  }
   SpinorPtr<S> r = block_field<S>(c, SLOT_MULTI + 1, SLOT_MULTI + 11, NR, &rc); HB_TRY(rc);
   SpinorPtr<S> q = block_field<S>(c, SLOT_MULTI + 2, SLOT_MULTI + 12, NR, &rc); HB_TRY(rc);
   SpinorPtr<S> t = block_field<S>(c, SLOT_MULTI + 3, SLOT_MULTI + 13, NR, &rc); HB_TRY(rc);
@@ -630,24 +678,24 @@ int cg_multi_block(Context *c, const MultiPlan &plan, const MultiFields<S, G> &f
     HB_TRY(rr);
     k_multi_true_residual<S, NR><<<nblocks(vh), kBlock, 0, c->stream>>>(ax, b[idx[k]], r, vh, k, c->red);
     k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(c->red, nblocks(vh), nullptr, FinMultiTrue{st, k, first});
-    k_multi_prestart<S, NR><<<nblocks(vh), kBlock, 0, c->stream>>>(p, r, vh, k, st);
+    k_multi_prestart<S, NR><<<nblocks(vh), kBlock, 0, c->stream>>>(ring, r, vh, k, st);
     HB_HIP(hipGetLastError());
     return HB_OK;
   };
   for (int k = 0; k < nb; k++) HB_TRY(reliable(k, 1));
 
   // one batched iteration; captured once into a graph and replayed
-  auto iteration = [&]() -> int {
-    HB_TRY((multi_apply<S, G, NR>(c, f, plan.ngroups, grp, kap, rh, q, p, t, y, st, plan.clover)));
+  auto iteration = [&](int slot) -> int {
+    HB_TRY((multi_apply<S, G, NR>(c, f, plan.ngroups, grp, kap, rh, q, ring.p[slot], t, y, st, plan.clover)));
     const int tile = c->multi_tile;
     const int grid = nblocks(vh * NR, tile);
     k_multi_update<S, NR><<<grid, tile, 0, c->stream>>>(r, q, vh, st, part);
-    k_finalize<NR><<<1, kFinThreads, 0, c->stream>>>(part, grid, nullptr, FinMultiUpdate<NR>{st});
-    k_multi_pupdate<S, NR><<<grid, tile, 0, c->stream>>>(p, r, xlo, vh, st);
+    k_finalize_each<NR><<<1, kFinThreads, 0, c->stream>>>(part, grid, FinMultiUpdate{st, slot});
+    k_multi_pupdate<S, NR><<<grid, tile, 0, c->stream>>>(ring, r, xlo, vh, st, slot);
     HB_HIP(hipGetLastError());
     return HB_OK;
   };
-  const int chunk = 8;
+  const int chunk = 8;  // a multiple of the ring's four slots
   // the captured chunk and its executable, destroyed on every return path
   struct Graph {
     hipGraph_t graph = nullptr;
@@ -659,7 +707,7 @@ int cg_multi_block(Context *c, const MultiPlan &plan, const MultiFields<S, G> &f
   } gr;
   HB_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   int crc = HB_OK;
-  for (int k = 0; k < chunk && crc == HB_OK; k++) crc = iteration();
+  for (int k = 0; k < chunk && crc == HB_OK; k++) crc = iteration(k & 3);
   hipError_t ce = hipStreamEndCapture(c->stream, &gr.graph);
   HB_TRY(crc);
   if (ce != hipSuccess) {

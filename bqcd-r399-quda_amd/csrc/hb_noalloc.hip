@@ -84,7 +84,7 @@ int hb_cg_d_noalloc(hb_context *ctx, int op, double kappa, double rho, double *x
   w.t = reinterpret_cast<double2 *>(b + 0 * kSpinorMax);
   w.y = reinterpret_cast<double2 *>(b + 1 * kSpinorMax);
   w.r = reinterpret_cast<double2 *>(b + 2 * kSpinorMax);
-  w.p = reinterpret_cast<double2 *>(b + 3 * kSpinorMax);
+  for (double2 *&p : w.p.p) p = reinterpret_cast<double2 *>(b + 3 * kSpinorMax);
   w.q = reinterpret_cast<double2 *>(b + 4 * kSpinorMax);
   w.st = reinterpret_cast<hb::CgState *>(b + kStateOff);
   w.red = reinterpret_cast<double *>(b + kRedOff);

@@ -18,6 +18,9 @@ enum {
   SLOT_IN,
   SLOT_OUT,
   SLOT_STATE,      // CgState
+  SLOT_P1,         // further search directions (CgRing)
+  SLOT_P2,
+  SLOT_P3,
   SLOT_LP0,        // low-precision fields of the mixed solver
   SLOT_LP1,
   SLOT_LP2,
@@ -28,6 +31,8 @@ enum {
   SLOT_LPN2,
   SLOT_LPN3,
   SLOT_LPN4,
+  SLOT_LPR,        // search directions of the mixed solver's ring and their norms: +2 .. +7
+  SLOT_LPR_LAST = SLOT_LPR + 7,
   SLOT_MIX0,       // FP64 fields of the mixed solver
   SLOT_MIX1,
   SLOT_FORCE0,     // force temporaries
@@ -56,7 +61,8 @@ enum {
   SLOT_HMC_MV = SLOT_HMC + 24,                      // kMaxMre products M v_i
   SLOT_HMC_MRE = SLOT_HMC_MV + kMaxMre,             // 2 bases of kMaxMre vectors
   SLOT_PLUGIN = SLOT_HMC_MRE + 2 * kMaxMre,         // staging of the plugin entry points (hb_plugin.hip), 6 slots
-  SLOT_END = SLOT_PLUGIN + 6
+  SLOT_MULTI_RING = SLOT_PLUGIN + 6,                // search directions of the multi-RHS ring and their norms, 6 slots
+  SLOT_END = SLOT_MULTI_RING + 6
 };
 static_assert(SLOT_SINGLE_END <= SLOT_MULTI, "single-RHS slots overlap the multi-RHS range");
 static_assert(SLOT_MULTI_LAST < SLOT_MULTI_CLOVER_B, "multi-RHS fields overlap the clover scratch");
@@ -89,7 +95,8 @@ int ensure_links_two_rows(Context *c, bool *use);
 // CG vectors r, p, q = A p, the device state, the reduction partials
 // (nblocks(vh, 64) + 1 + vector_grid(vh) doubles) and host memory for reading the state back
 struct CgWork {
-  double2 *t = nullptr, *y = nullptr, *r = nullptr, *p = nullptr, *q = nullptr;
+  double2 *t = nullptr, *y = nullptr, *r = nullptr, *q = nullptr;
+  CgRing p{};
   CgState *st = nullptr;
   double *red = nullptr;
   CgState *hs = nullptr;
