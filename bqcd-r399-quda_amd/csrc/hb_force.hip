@@ -478,27 +478,84 @@ __global__ __launch_bounds__(kLinkBlock, 2) void k_clover_force(double *P, const
 // ---------------------------------------------------------------------------
 // gauge force (dsg.F90:28-63) with the staple of staple.F90:28-76
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kLinkBlock) void k_gauge_force(double *P, const double2 *__restrict__ U, Geom g, int run, double s) {
-  int mu, e, i;
-  if (!link_slot(g, run, mu, e, i)) return;
-  const int vh = g.vh, o = 1 - e;
-  int x[4];
-  site_coords(g, e, i, x[0], x[1], x[2], x[3]);
-  M3 st = m3_zero();
-  for (int nu = 0; nu < 4; nu++) {
-    if (nu == mu) continue;
-    const int j1 = nb(g, x[0], x[1], x[2], x[3], mu, 1), j2 = nb(g, x[0], x[1], x[2], x[3], nu, 1);
-    const int j3 = nb(g, x[0], x[1], x[2], x[3], nu, -1);
-    const int j4 = nb2(g, x[0], x[1], x[2], x[3], nu, -1, mu, 1);
-    // U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+  +  U_nu(x+mu-nu)^+ U_mu(x-nu)^+ U_nu(x-nu)
-    m3_acc(st, m3_muld(m3_muld(link_b(U, nu, o, j1, vh), link_b(U, mu, o, j2, vh)), link_b(U, nu, e, i, vh)));
-    __builtin_amdgcn_sched_barrier(0);
-    m3_acc(st, m3_dmul(m3_mul(link_b(U, mu, o, j3, vh), link_b(U, nu, e, j4, vh)), link_b(U, nu, o, j3, vh)));
-    __builtin_amdgcn_sched_barrier(0);
+// One wave per plane (mu, nu) of 64 sites.  The plaquette at x is the staple
+// above for both of its links (v for U_mu(x), v^+ for U_nu(x)), which leaves
+// ten links and nine products per plane, where the two links' staples taken
+// apart read fourteen; the sites' own links, which every plane needs, are
+// shared through LDS, and so are the six waves' shares of the four forces.
+// Bound by the addresser of the vector memory path (busy 77 % with the links
+// in memory, 60 % here, FP64 issue 36 %): 32^3x64 1.30 ms, one wave per
+// direction 1.54 ms; 16^3x32 118 -> 87 us.  Registers for one link fetched
+// ahead spill (1.37 ms); two waves per SIMD with both own links held: 1.67 ms.
+constexpr int kPlaneBlock = 384;
+__global__ __launch_bounds__(kPlaneBlock, 3) void k_gauge_force(double *P, const double2 *__restrict__ U, Geom g, int run,
+                                                                double s) {
+  __shared__ union {
+    double2 own[4][9][64];
+    double part[6][2][8][64];
+  } lds;
+  int k, e, i;
+  const bool active = link_slot(g, run, k, e, i);
+  const int mu = k < 3 ? 0 : k < 5 ? 1 : 2, nu = k < 3 ? k + 1 : k < 5 ? k - 1 : 3;
+  const int vh = g.vh, o = 1 - e, lane = threadIdx.x & 63;
+  int x[4] = {0, 0, 0, 0};
+  M3 t = m3_zero();
+  if (active) {
+    if (k < 4) {
+      const M3 u = link_b(U, k, e, i, vh);
+#pragma unroll
+      for (int m = 0; m < 9; m++) lds.own[k][m][lane] = u.m[m];
+    }
+    site_coords(g, e, i, x[0], x[1], x[2], x[3]);
+    const int xp = nb(g, x[0], x[1], x[2], x[3], mu, 1), yp = nb(g, x[0], x[1], x[2], x[3], nu, 1);
+    t = m3_muld(link_b(U, nu, o, xp, vh), link_b(U, mu, o, yp, vh));
   }
-  double q[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  im_tr_j(q, m3_mul(link_b(U, mu, e, i, vh), st), s);
-  mom_add(P, mu, e, i, vh, q);
+  __syncthreads();
+  double q[8] = {0, 0, 0, 0, 0, 0, 0, 0}, r[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (active) {
+    const auto own = [&](int d) {
+      M3 u;
+#pragma unroll
+      for (int m = 0; m < 9; m++) u.m[m] = lds.own[d][m][lane];
+      return u;
+    };
+    const int xm = nb(g, x[0], x[1], x[2], x[3], mu, -1), ym = nb(g, x[0], x[1], x[2], x[3], nu, -1);
+    const int xpym = nb2(g, x[0], x[1], x[2], x[3], mu, 1, nu, -1);
+    const int xmyp = nb2(g, x[0], x[1], x[2], x[3], mu, -1, nu, 1);
+    t = m3_muld(t, own(nu));
+    step_end(t);
+    im_tr_j(q, m3_mul(own(mu), t), s);
+#pragma unroll
+    for (int j = 0; j < 8; j++) r[j] = -q[j];
+    t = m3_mul(link_b(U, mu, o, ym, vh), link_b(U, nu, e, xpym, vh));
+    step_end(t);
+    t = m3_dmul(t, link_b(U, nu, o, ym, vh));
+    step_end(t);
+    im_tr_j(q, m3_mul(own(mu), t), s);
+    t = m3_mul(link_b(U, nu, o, xm, vh), link_b(U, mu, e, xmyp, vh));
+    step_end(t);
+    t = m3_dmul(t, link_b(U, mu, o, xm, vh));
+    step_end(t);
+    im_tr_j(r, m3_mul(own(nu), t), s);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    lds.part[k][0][j][lane] = q[j];
+    lds.part[k][1][j][lane] = r[j];
+  }
+  __syncthreads();
+  if (k > 3 || !active) return;
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    // planes 01 02 03 12 13 23; 0: the first direction's share, 1: the second's
+    const auto part = [&](int p, int d) { return lds.part[p][d][j][lane]; };
+    q[j] = k == 0 ? part(0, 0) + part(1, 0) + part(2, 0)
+         : k == 1 ? part(0, 1) + part(3, 0) + part(4, 0)
+         : k == 2 ? part(1, 1) + part(3, 1) + part(5, 0)
+                  : part(2, 1) + part(4, 1) + part(5, 1);
+  }
+  mom_add(P, k, e, i, vh, q);
 }
 
 // ---------------------------------------------------------------------------
@@ -641,7 +698,7 @@ int clover_action_parity_dev(Context *c, const double2 *Cb, int eo, double *res_
 int dsg_dev(Context *c, double *P, double step, double beta) {
   if (beta == 0.0) return HB_OK;
   const LinkGrid lg(c->g);
-  k_gauge_force<<<lg.grid, kLinkBlock, 0, c->stream>>>(P, c->gauge, c->g, lg.run, -step * beta / 3.0);
+  k_gauge_force<<<lg.grid, kPlaneBlock, 0, c->stream>>>(P, c->gauge, c->g, lg.run, -step * beta / 3.0);
   HB_HIP(hipGetLastError());
   return HB_OK;
 }
