@@ -10,20 +10,21 @@ namespace hb {
 // clover_f_mu_nu (clover/clover_f_mu_nu.F90:37-103): f = -i (Q - Q^+) with Q the
 // sum of the four plaquette leaves in plane (mu, nu) around x (parity e)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ H3 f_mu_nu(const double2 *__restrict__ U, const Geom &g, int e, int i, const int (&x)[4],
-                                      int mu, int nu) {
+// own(d): U_d(x)
+template <class F>
+__device__ __forceinline__ H3 f_mu_nu(const double2 *__restrict__ U, const Geom &g, int e, const int (&x)[4], int mu,
+                                      int nu, F own) {
   const int o = 1 - e, vh = g.vh;
   const int xm_ = nb(g, x[0], x[1], x[2], x[3], mu, -1), x_m = nb(g, x[0], x[1], x[2], x[3], nu, -1);
   M3 q;
   {  // leaf 1: U_mu(x) U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
     const int xp_ = nb(g, x[0], x[1], x[2], x[3], mu, 1), x_p = nb(g, x[0], x[1], x[2], x[3], nu, 1);
-    q = m3_muld(m3_muld(m3_mul(link_b(U, mu, e, i, vh), link_b(U, nu, o, xp_, vh)), link_b(U, mu, o, x_p, vh)),
-                link_b(U, nu, e, i, vh));
+    q = m3_muld(m3_muld(m3_mul(own(mu), link_b(U, nu, o, xp_, vh)), link_b(U, mu, o, x_p, vh)), own(nu));
   }
   step_end(q);
   {  // leaf 2: U_nu(x) U_mu(x-mu+nu)^+ U_nu(x-mu)^+ U_mu(x-mu)
     const int xmp = nb2(g, x[0], x[1], x[2], x[3], mu, -1, nu, 1);
-    m3_acc(q, m3_mul(m3_muld(m3_muld(link_b(U, nu, e, fresh(i), vh), link_b(U, mu, e, xmp, vh)),
+    m3_acc(q, m3_mul(m3_muld(m3_muld(own(nu), link_b(U, mu, e, xmp, vh)),
                              link_b(U, nu, o, xm_, vh)),
                      link_b(U, mu, o, xm_, vh)));
   }
@@ -39,7 +40,7 @@ __device__ __forceinline__ H3 f_mu_nu(const double2 *__restrict__ U, const Geom 
     const int xpm = nb2(g, x[0], x[1], x[2], x[3], mu, 1, nu, -1);
     m3_acc(q, m3_muld(m3_mul(m3_dmul(link_b(U, nu, o, fresh(x_m), vh), link_b(U, mu, o, x_m, vh)),
                              link_b(U, nu, e, xpm, vh)),
-                      link_b(U, mu, e, fresh(i), vh)));
+                      own(mu)));
   }
   H3 f;  // -i (Q - Q^+)
 #pragma unroll
@@ -128,25 +129,38 @@ __device__ void clover_block_store(double2 (&A)[6][6], double2 *__restrict__ Ca,
 // fields of 64 sites of one parity, which meet in LDS, and two of them then
 // build and factor one chiral block each, from P = (f_21, f_32 + i f_31; .,
 // -f_21) and Q = (f_34, f_14 + i f_42; ., -f_34).  One thread per site, the
-// planes one after the other, needs 512 registers, one wave per SIMD.  Both
-// parities, that way / this way: 8^3x16 68 / 19 us, 16^3x32 147 / 125,
-// 24x20x12x36 262 / 208, 32^3x64 2.27 / 2.29 ms (there the links, read 14 times
-// a plane, come from beyond L2).
+// planes one after the other, needs 512 registers, one wave per SIMD.  The
+// sites' own links, four of a plane's sixteen link reads, are read once.  Both
+// parities, one thread per site / six waves / own links in LDS: 8^3x16 68 / 19 /
+// 19 us, 16^3x32 147 / 125 / 115, 24x20x12x36 262 / 208 / 193, 32^3x64 2.27 / 2.29 /
+// 2.02 ms.
 constexpr int kPlaneBlock = 384;
 __global__ __launch_bounds__(kPlaneBlock, 3) void k_clover_build(const double2 *__restrict__ U, Geom g, int run,
                                                                  double factor, double2 *__restrict__ Ca,
                                                                  double2 *__restrict__ Ci, double2 *__restrict__ Cb) {
+  __shared__ double2 links[4][9][64];
   __shared__ double2 Fo[6][3][64];
   __shared__ double Fd[6][3][64];
   int k, e, i;
   const bool active = link_slot(g, run, k, e, i);
   const int lane = threadIdx.x & 63, vh = g.vh;
+  if (active && k < 4) {
+    const M3 u = link_b(U, k, e, i, vh);
+#pragma unroll
+    for (int m = 0; m < 9; m++) links[k][m][lane] = u.m[m];
+  }
+  __syncthreads();
   if (active) {
     int x[4];
     site_coords(g, e, i, x[0], x[1], x[2], x[3]);
     const int mu = k == 0 ? 1 : k < 4 ? 2 : k == 4 ? 0 : 3;
     const int nu = k == 0 || k == 2 ? 0 : k == 1 || k == 5 ? 1 : 3;
-    const H3 f = f_mu_nu(U, g, e, i, x, mu, nu);
+    const H3 f = f_mu_nu(U, g, e, x, mu, nu, [&](int d) {
+      M3 u;
+#pragma unroll
+      for (int m = 0; m < 9; m++) u.m[m] = links[d][m][lane];
+      return u;
+    });
 #pragma unroll
     for (int q = 0; q < 3; q++) {
       Fo[k][q][lane] = f.o[q];
