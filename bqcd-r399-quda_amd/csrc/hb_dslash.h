@@ -45,12 +45,13 @@ template <class S, class G> inline int operator_policy(int vh, int nr = 1) {
   return solve_bytes_per_site<S, G>(nr) * (size_t)vh <= kResidentBytes ? 0 : kNT;
 }
 
-// Waves that share a site (1: k_dslash, else k_dslash_split), which sets the
-// number of workgroups of a launch and of the partial sums it leaves
-// (EPI_MTDOT).  us per CG iteration at 1 / 2 / 4 waves:
+// Waves that share a site (1: k_dslash, else k_dslash_split).  us per CG
+// iteration at 1 / 2 / 4 waves:
 //   FP64    8^4 (2 k sites per parity) 58.9 / 47.1 / 45.0, 12^3x24 (21 k)
 //           80.3 / 61.5 / 58.4, 16^4 (33 k) 85.4 / 69.0 / 69.2,
-//           16x16x18x18 (41 k) 91.3 / 79.4 / 89.8, 16^3x32 (66 k) 117 / 112 / 112;
+//           16x16x18x18 (41 k) 91.3 / 79.4 / 89.8, 16^3x32 (66 k) 117 / 112 / 112,
+//           24x20x12x36 (104 k) 184 / 178, 20^3x40 (160 k) 273 / 274, 24^3x48
+//           (332 k) 570 / 580 (the one wave in workgroups of 64 sites);
 //           M~^+M~ with 18-real links 41 k 66.8 / 63.4 / 68.8, 50 k 74.2 / 80.2 / 82.1
 //   FP32    12^3x24 70.7 / 58.7 / 57.6, 16^4 69.5 / 61.5 / 59.4, 50 k 77.0 / 71.1 /
 //           72.2, 24^3x48 (332 k) 365 / 356 / 358, 32^3x64 1010 / 1056 / 1067
@@ -59,11 +60,25 @@ template <class S, class G> inline int operator_policy(int vh, int nr = 1) {
 // Eight waves (one hop each) were slower than four from 4 k sites on.
 template <class S, class G> inline int split_waves(int vh) {
   if (vh <= (1 << 15)) return 4;
-  constexpr int two = !std::is_same<S, SF64>::value ? 1 << 19 : G::kRecon ? 1 << 16 : 3 << 14;
+  constexpr int two = !std::is_same<S, SF64>::value ? 1 << 19 : G::kRecon ? 1 << 17 : 3 << 14;
   return vh <= two ? 2 : 1;
 }
+
+// Sites per workgroup.  One wave per site in FP64 runs two workgroups of 256
+// per CU: where that is a few rounds of the chip, workgroups of one wave leave
+// less of it idle in the last one.  256 / 64 sites, us, FP64 CG iteration and
+// M~^+M~ with 18-real links: 24x20x12x36 (104 k sites per parity, one round) 184 /
+// 183 and 170 / 176, 20^3x40 (160 k) 288 / 276 and 265 / 257, 24^3x48 (332 k) 592 /
+// 574 and 569 / 545, 32^3x64 (1049 k) 1693 / 1699 and 1621 / 1624.  FP32 and 16-bit
+// fields, at higher occupancy: 354 / 352 and 196 / 194 at 24^3x48, 998 / 1023 and
+// 503 / 507 at 32^3x64.
+template <class S, class G> inline int dslash_tile(int vh) {
+  if (split_waves<S, G>(vh) > 1) return 64;
+  return std::is_same<S, SF64>::value && vh > (1 << 17) && vh <= (1 << 19) ? 64 : kBlock;
+}
+// workgroups of a launch, each of which leaves one partial sum (EPI_MTDOT)
 template <class S, class G> inline int dslash_grid(int vh) {
-  return nblocks(vh, split_waves<S, G>(vh) > 1 ? 64 : kBlock);
+  return nblocks(vh, dslash_tile<S, G>(vh));
 }
 
 template <class S, class G> int launch_dslash(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st);

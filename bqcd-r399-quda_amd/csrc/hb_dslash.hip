@@ -229,7 +229,7 @@ static void launch_split(const DslashArgs<S, G> &a, bool dag, int epi, hipStream
 
 template <class S, class G, int POL>
 static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
-  dim3 grid(dslash_grid<S, G>(a.g.vh)), block(kBlock);
+  dim3 grid(dslash_grid<S, G>(a.g.vh)), block(dslash_tile<S, G>(a.g.vh));
 #define HB_DS(D, E) hipLaunchKernelGGL((k_dslash<S, G, D, E, POL>), grid, block, 0, st, a)
   if (!dag) {
     switch (epi) {

@@ -17,8 +17,9 @@ pytestmark = pytest.mark.gpu
 KAPPA, CSW, RHO = 0.125, 1.0, 0.07
 
 # sites per parity: 35640 (two waves), 50400 (18-real links: one, kept; two-row: two),
-# 146016 (one, streamed)
-FP64 = [(10, 18, 22, 18), (14, 20, 12, 30), (26, 18, 24, 26)]
+# 131040 (18-real: one; two-row: two; both streamed), 146016 (one, streamed, in
+# workgroups of one wave)
+FP64 = [(10, 18, 22, 18), (14, 20, 12, 30), (26, 18, 20, 28), (26, 18, 24, 26)]
 # 35640, 121680 (two waves, kept), 262080 (FP32: two, streamed), 554880 (one, streamed)
 REDUCED = [(10, 18, 22, 18), (26, 18, 20, 26), (30, 26, 28, 24), (34, 30, 32, 34)]
 TOL = {"f16": (1e-4, 3e-4), "f16g": (5e-5, 1e-4), "f32": (1e-6, 2e-6)}
