@@ -115,11 +115,14 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(double2 *__restrict__ r, c
 template <bool NT>
 __global__ __launch_bounds__(kBlock) void k_cg_pupdate(double2 *__restrict__ x, double2 *__restrict__ p,
                                                        const double2 *__restrict__ r, int n, CgState *st, int k,
-                                                       const double *pb, int nb) {
+                                                       const double *pb, int nb, Note note) {
   const CgSlot c = st->s[k & 1];
   const bool first = blockIdx.x == 0 && threadIdx.x == 0;
   if (c.done) {
-    if (first) st->s[~k & 1] = c;
+    if (first) {
+      st->s[~k & 1] = c;
+      note.tell(c.done);
+    }
     return;
   }
   const int step = gridDim.x * blockDim.x;
@@ -130,7 +133,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_pupdate(double2 *__restrict__ x, 
   const double alpha = c.rtr / st->pap, beta = rtr / c.rtr;
   const int iter = c.iter + 1;
   const int done = rtr <= st->rest ? 1 : iter >= st->maxiter ? 2 : 0;
-  if (first) st->s[~k & 1] = CgSlot{done ? c.rtr : rtr, rtr, iter, done};
+  if (first) {
+    st->s[~k & 1] = CgSlot{done ? c.rtr : rtr, rtr, iter, done};
+    note.tell(done);
+  }
   while (i < n) {
     const double2 xv = make_double2(xx.x + alpha * pp.x, xx.y + alpha * pp.y);
     const double2 pv = make_double2(rr.x + beta * pp.x, rr.y + beta * pp.y);
@@ -150,11 +156,14 @@ __global__ __launch_bounds__(kBlock) void k_cg_pupdate(double2 *__restrict__ x, 
 // against 49.3
 __global__ __launch_bounds__(kBlock) void k_cg_pupdate_ring(double2 *__restrict__ x, CgRing ring,
                                                             const double2 *__restrict__ r, int n, CgState *st, int k,
-                                                            const double *pb, int nb) {
+                                                            const double *pb, int nb, Note note) {
   const CgSlot c = st->s[k & 1];
   const bool first = blockIdx.x == 0 && threadIdx.x == 0;
   if (c.done) {
-    if (first) st->s[~k & 1] = c;
+    if (first) {
+      st->s[~k & 1] = c;
+      note.tell(c.done);
+    }
     return;
   }
   const int slot = k & 3;
@@ -166,6 +175,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_pupdate_ring(double2 *__restrict_
   if (first) {
     st->s[~k & 1] = CgSlot{done ? c.rtr : rtr, rtr, iter, done};
     st->alpha[slot] = alpha;
+    note.tell(done);
   }
   const bool take = slot == 3 || done;
   const double2 *p = ring.p[slot];
@@ -285,10 +295,11 @@ int cg_update(Context *c, double2 *r, const double2 *q, CgState *st, int k, cons
 int cg_pupdate(Context *c, double2 *x, const CgRing &ring, const double2 *r, CgState *st, int k, const double *pb) {
   const int vh = c->g.vh;
   if (ring.p[1] != ring.p[0]) {
-    k_cg_pupdate_ring<<<vector_grid(vh), kBlock, 0, c->stream>>>(x, ring, r, 12 * vh, st, k, pb, vector_grid(vh));
+    k_cg_pupdate_ring<<<vector_grid(vh), kBlock, 0, c->stream>>>(x, ring, r, 12 * vh, st, k, pb, vector_grid(vh),
+                                                               next_note(c));
   } else {
     const auto f = operator_policy<SF64, SF64R>(vh) == kNT ? k_cg_pupdate<true> : k_cg_pupdate<false>;
-    f<<<vector_grid(vh), kBlock, 0, c->stream>>>(x, ring.p[0], r, 12 * vh, st, k, pb, vector_grid(vh));
+    f<<<vector_grid(vh), kBlock, 0, c->stream>>>(x, ring.p[0], r, 12 * vh, st, k, pb, vector_grid(vh), next_note(c));
   }
   HB_HIP(hipGetLastError());
   return HB_OK;

@@ -173,26 +173,20 @@ int cg_f64_run(Context *c, const CgWork &w, int op, double kappa, double rho, do
     HB_HIP(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
     HB_HIP(hipStreamSynchronize(c->stream));
   } else {
-    // iterations in chunks (a multiple of four, so that each ends in slot 0); every
-    // kernel returns immediately once done != 0, so the chunk length only sets
-    // how often the host looks at the state
     const int na = w.recon ? dslash_grid<SF64, SF64R>(c->g.vh) : dslash_grid<SF64, SF64>(c->g.vh);
     double *pa = w.red, *pb = w.red + na + 1;
-    int chunk = 8;
-    for (;;) {
-      for (int k = 0; k < chunk; k++) {
-        HB_TRY(apply_f64(c, op, kappa, rho, w.q, w.p.p[k & 3], w.t, w.y, pa, &st->s[k & 1].done, w.recon));
-        const double *sum = pa;
-        int nsum = na;
-        HB_TRY(shorten_partials(c, sum, nsum, &st->s[k & 1].done));
-        HB_TRY(cg_update(c, w.r, w.q, st, k, sum, nsum, pb));
-        HB_TRY(cg_pupdate(c, x, w.p, w.r, st, k, pb));
-      }
-      HB_HIP(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
-      HB_HIP(hipStreamSynchronize(c->stream));
-      if (hs->s[0].done) break;
-      if (chunk < 64) chunk *= 2;
+    Watch watch(c);
+    for (int k = 0, done = 0; !done; k++) {
+      HB_TRY(apply_f64(c, op, kappa, rho, w.q, w.p.p[k & 3], w.t, w.y, pa, &st->s[k & 1].done, w.recon));
+      const double *sum = pa;
+      int nsum = na;
+      HB_TRY(shorten_partials(c, sum, nsum, &st->s[k & 1].done));
+      HB_TRY(cg_update(c, w.r, w.q, st, k, sum, nsum, pb));
+      HB_TRY(cg_pupdate(c, x, w.p, w.r, st, k, pb));
+      if (k > 0) HB_TRY(watch.look(&done));
     }
+    HB_HIP(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
+    HB_HIP(hipStreamSynchronize(c->stream));
     nmv += hs->s[0].iter;
   }
   const int niter = hs->s[0].iter;

@@ -36,6 +36,32 @@ int ensure_host_stage(Context *c, size_t bytes) {
   return HB_OK;
 }
 
+int Watch::look(int *flag) {
+  const uint64_t last = c_->note_seq;
+  uint64_t v;
+  for (unsigned spin = 1;; spin++) {
+    v = __atomic_load_n(c_->note, __ATOMIC_ACQUIRE);
+    if ((v >> 2) + 1 >= last) break;
+    __builtin_ia32_pause();
+    if (spin % 4096) continue;
+    // every report has been written once the stream is empty: the wait ends
+    // there also when a kernel failed
+    const hipError_t e = hipStreamQuery(c_->stream);
+    if (e == hipErrorNotReady) {
+      (void)hipGetLastError();
+      continue;
+    }
+    HB_HIP(e);
+    v = __atomic_load_n(c_->note, __ATOMIC_ACQUIRE);
+    HB_CHECK((v >> 2) + 1 >= last, HB_E_HIP, "a solve's progress was not reported");
+    break;
+  }
+  const bool set = (v & 3) != 0, follows = (v >> 2) < last || set_;
+  set_ = set && !follows;
+  *flag = set && follows ? (int)(v & 3) : 0;
+  return HB_OK;
+}
+
 // Scratch slots grow on demand and are kept for the life of the context.
 void *scratch(Context *c, int slot, size_t bytes, int *rc) {
   *rc = HB_OK;
@@ -109,11 +135,13 @@ int hb_init(const int L[4], const int bc[4], int device, hb_context **out) {
   // reduction partials: up to 16 values per block of a site-parallel grid
   c->red_blocks = nblocks(2 * c->g.vh) + 64;
   e = hipMalloc(&c->red, sizeof(double) * 16 * (size_t)c->red_blocks);
+  if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&c->note), 64, hipHostMallocDefault);
   if (e != hipSuccess) {
     set_error("hb_init: %s", hipGetErrorString(e));
     hb_finalize(reinterpret_cast<hb_context *>(c));
     return HB_E_HIP;
   }
+  *c->note = 0;
   *out = reinterpret_cast<hb_context *>(c);
   return HB_OK;
 }
@@ -135,6 +163,7 @@ int hb_finalize(hb_context *ctx) {
   (void)hipFree(c->red);
   (void)hipFree(c->dev_stage);
   if (c->host_stage) (void)hipHostFree(c->host_stage);
+  if (c->note) (void)hipHostFree(c->note);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   delete c;
   return HB_OK;

@@ -201,12 +201,15 @@ __device__ __forceinline__ bool mix_decide(MixSlot &d, const MixSlot &c, const M
 // update or the end is due)
 template <class S>
 __global__ __launch_bounds__(kBlock) void k_mix_pupdate(SpinorPtr<S> p, SpinorPtr<S> r, float2 *__restrict__ xlo, int n,
-                                                        MixState *st, int k, const double *pb, int nb) {
+                                                        MixState *st, int k, const double *pb, int nb, Note note) {
   using V = typename S::V;
   const MixSlot c = st->s[k & 1];
   const bool first = blockIdx.x == 0 && threadIdx.x == 0;
   if (c.flag) {
-    if (first) st->s[~k & 1] = c;
+    if (first) {
+      st->s[~k & 1] = c;
+      note.tell(c.flag);
+    }
     return;
   }
   const int step = gridDim.x * blockDim.x;
@@ -226,7 +229,10 @@ __global__ __launch_bounds__(kBlock) void k_mix_pupdate(SpinorPtr<S> p, SpinorPt
   const bool next = mix_decide(d, c, st, rn);
   const float alpha = (float)(c.rtr / st->pap);
   const float beta = (float)(rn / c.rtr);
-  if (first) st->s[~k & 1] = d;
+  if (first) {
+    st->s[~k & 1] = d;
+    note.tell(d.flag);
+  }
   while (i < n) {
     V v[kNums<S>];
 #pragma unroll
@@ -252,6 +258,7 @@ template <class S> struct MixRing {
 struct FinMixStep {
   MixState *st;
   int k;
+  Note note;
   __device__ void operator()(const double (&t)[1]) const {
     const MixSlot c = st->s[k & 1];
     MixSlot d = c;
@@ -263,6 +270,7 @@ struct FinMixStep {
       st->cur = k & 3;
     }
     st->s[~k & 1] = d;
+    note.tell(d.flag);
   }
 };
 template <class S>
@@ -344,6 +352,7 @@ __global__ __launch_bounds__(kBlock) void k_mix_true_residual(double2 *__restric
 struct FinMixTrue {
   MixState *st;
   int first;
+  Note note;
   __device__ void operator()(const double (&t)[1]) const {
     const double rt = t[0];
     MixSlot &c = st->s[0];
@@ -361,6 +370,7 @@ struct FinMixTrue {
       c.rtr = rt;
       c.flag = 0;
     }
+    note.tell(c.flag);
   }
 };
 
@@ -576,7 +586,7 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
     }
     HB_TRY(apply_f64(c, op, kappa, rho, ax, x, t64, y64, nullptr, nullptr));
     k_mix_true_residual<S><<<nblocks(vh), kBlock, 0, c->stream>>>(ax, b, r, vh, c->red);
-    k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(c->red, nblocks(vh), nullptr, FinMixTrue{st, first});
+    k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(c->red, nblocks(vh), nullptr, FinMixTrue{st, first, next_note(c)});
     HB_HIP(hipGetLastError());
     if (!first && HB_MIX_REORTH) {
       k_mix_rdotp<S><<<nblocks(vh), kBlock, 0, c->stream>>>(ring, r, vh, st, c->red);
@@ -592,40 +602,35 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
   // partials of <p, A p> and of |r|^2
   const int na = dslash_grid<S, G>(vh), n = mix_count<S>(vh), grid = mix_grid<S>(vh), block = mix_block<S>(vh);
   double *pa = c->red, *pb = c->red + na + 1;
-  int chunk = 8;  // iterations between looks at the state; a multiple of four, so that each chunk ends in slot 0
-  for (;;) {
-    for (int k = 0; k < chunk; k++) {
-      const int *skip = &st->s[k & 1].flag;
-      const SpinorPtr<S> pk = ring.p[k & 3];
-      HB_TRY((mtil_lp<S, G>(c, false, kappa, r_op, y, pk, t, nullptr, SpinorPtr<S>{}, skip)));
-      HB_TRY((mtil_lp<S, G>(c, true, kappa, r_op, q, y, t, pa, pk, skip)));
-      const double *sum = pa;
-      int nsum = na;
-      HB_TRY(shorten_partials(c, sum, nsum, skip, sums ? kMaxParts : 1));
-      if (sums) {
-        k_mix_update<S, true><<<grid, block, 0, c->stream>>>(r, q, n, st, k, sum, nsum, pb);
-        k_mix_pupdate<S><<<grid, block, 0, c->stream>>>(p, r, xlo, n, st, k, pb, grid);
-      } else {
-        k_mix_update<S, false><<<grid, block, 0, c->stream>>>(r, q, n, st, k, sum, nsum, pb);
-        k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(pb, grid, nullptr, FinMixStep{st, k});
-        if constexpr (!kLinear<S>) k_mix_pupdate_ring<S><<<grid, block, 0, c->stream>>>(ring, r, xlo, n, st, k);
-      }
-      HB_HIP(hipGetLastError());
+  Watch watch(c);
+  for (int k = 0, flag = 0;;) {
+    const int *skip = &st->s[k & 1].flag;
+    const SpinorPtr<S> pk = ring.p[k & 3];
+    HB_TRY((mtil_lp<S, G>(c, false, kappa, r_op, y, pk, t, nullptr, SpinorPtr<S>{}, skip)));
+    HB_TRY((mtil_lp<S, G>(c, true, kappa, r_op, q, y, t, pa, pk, skip)));
+    const double *sum = pa;
+    int nsum = na;
+    HB_TRY(shorten_partials(c, sum, nsum, skip, sums ? kMaxParts : 1));
+    const Note note = next_note(c);
+    if (sums) {
+      k_mix_update<S, true><<<grid, block, 0, c->stream>>>(r, q, n, st, k, sum, nsum, pb);
+      k_mix_pupdate<S><<<grid, block, 0, c->stream>>>(p, r, xlo, n, st, k, pb, grid, note);
+    } else {
+      k_mix_update<S, false><<<grid, block, 0, c->stream>>>(r, q, n, st, k, sum, nsum, pb);
+      k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(pb, grid, nullptr, FinMixStep{st, k, note});
+      if constexpr (!kLinear<S>) k_mix_pupdate_ring<S><<<grid, block, 0, c->stream>>>(ring, r, xlo, n, st, k);
     }
-    HB_HIP(hipMemcpyAsync(hs, st, sizeof(MixState), hipMemcpyDeviceToHost, c->stream));
-    HB_HIP(hipStreamSynchronize(c->stream));
-    if (hs->s[0].flag == 2 || hs->s[0].flag == 3) break;
-    if (hs->s[0].flag == 1) {
+    HB_HIP(hipGetLastError());
+    HB_TRY(watch.look(&flag));
+    k++;
+    if (flag > 1) break;
+    if (flag == 1) {
       HB_TRY(reliable(0));
-      HB_HIP(hipMemcpyAsync(hs, st, sizeof(MixState), hipMemcpyDeviceToHost, c->stream));
-      HB_HIP(hipStreamSynchronize(c->stream));
-      if (hs->s[0].flag == 2 || hs->s[0].flag == 3) break;
-      // next chunk length: about the iterations one reliable interval took
-      chunk = 8;
-    } else if (chunk < 32) {
-      chunk *= 2;
+      k = 0;  // goes on from slot 0 with the direction the restart left there
     }
   }
+  HB_HIP(hipMemcpyAsync(hs, st, sizeof(MixState), hipMemcpyDeviceToHost, c->stream));
+  HB_HIP(hipStreamSynchronize(c->stream));
   HB_TRY(tm.stop(c->stream));
   float ms = 0.f;
   HB_TRY(tm.elapsed(&ms));
