@@ -36,27 +36,31 @@ int ensure_host_stage(Context *c, size_t bytes) {
   return HB_OK;
 }
 
-int Watch::look(int *flag) {
-  const uint64_t last = c_->note_seq;
-  uint64_t v;
+int wait_note(Context *c, int k, uint64_t seq, uint64_t *v) {
   for (unsigned spin = 1;; spin++) {
-    v = __atomic_load_n(c_->note, __ATOMIC_ACQUIRE);
-    if ((v >> 2) + 1 >= last) break;
+    *v = __atomic_load_n(c->note + k, __ATOMIC_ACQUIRE);
+    if (*v >> 2 >= seq) return HB_OK;
     __builtin_ia32_pause();
     if (spin % 4096) continue;
     // every report has been written once the stream is empty: the wait ends
     // there also when a kernel failed
-    const hipError_t e = hipStreamQuery(c_->stream);
+    const hipError_t e = hipStreamQuery(c->stream);
     if (e == hipErrorNotReady) {
       (void)hipGetLastError();
       continue;
     }
     HB_HIP(e);
-    v = __atomic_load_n(c_->note, __ATOMIC_ACQUIRE);
-    HB_CHECK((v >> 2) + 1 >= last, HB_E_HIP, "a solve's progress was not reported");
-    break;
+    *v = __atomic_load_n(c->note + k, __ATOMIC_ACQUIRE);
+    HB_CHECK(*v >> 2 >= seq, HB_E_HIP, "a solve's progress was not reported");
+    return HB_OK;
   }
-  const bool set = (v & 3) != 0, follows = (v >> 2) < last || set_;
+}
+
+int Watch::look(int *flag) {
+  const uint64_t last = c_->note_seq;
+  uint64_t v = 0;
+  HB_TRY(wait_note(c_, 0, last - 1, &v));
+  const bool set = (v & 3) != 0, follows = v >> 2 < last || set_;
   set_ = set && !follows;
   *flag = set && follows ? (int)(v & 3) : 0;
   return HB_OK;
@@ -135,13 +139,13 @@ int hb_init(const int L[4], const int bc[4], int device, hb_context **out) {
   // reduction partials: up to 16 values per block of a site-parallel grid
   c->red_blocks = nblocks(2 * c->g.vh) + 64;
   e = hipMalloc(&c->red, sizeof(double) * 16 * (size_t)c->red_blocks);
-  if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&c->note), 64, hipHostMallocDefault);
+  if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&c->note), kNotes * sizeof(uint64_t), hipHostMallocDefault);
   if (e != hipSuccess) {
     set_error("hb_init: %s", hipGetErrorString(e));
     hb_finalize(reinterpret_cast<hb_context *>(c));
     return HB_E_HIP;
   }
-  *c->note = 0;
+  std::memset(c->note, 0, kNotes * sizeof(uint64_t));
   *out = reinterpret_cast<hb_context *>(c);
   return HB_OK;
 }

@@ -150,7 +150,7 @@ struct Context {
   int red_blocks = 0;
   void *host_stage = nullptr;        // pinned staging
   size_t host_stage_bytes = 0;
-  uint64_t *note = nullptr;          // pinned word a running solve reports to (Note)
+  uint64_t *note = nullptr;          // pinned words (kNotes) a running solve reports to (Note)
   uint64_t note_seq = 0;             // of the last report enqueued
   void *dev_stage = nullptr;         // device staging (AoS copies)
   size_t dev_stage_bytes = 0;
@@ -183,13 +183,16 @@ int ensure_host_stage(Context *c, size_t bytes);
 // FP64 8^4 37.1 / 30.9, 12^3x24 52.2 / 51.2; FP32 14x20x12x30 69.5 / 65.7; 16-bit
 // 12^3x24 46.8 / 38.2, 16^3x32 69.7 / 53.5, 32^3x64 503 / 497.  Two reports behind
 // instead of one: 8^4 30.9 / 30.9 in FP64, 38.9 / 32.3 in FP32.
+constexpr int kNotes = 16;  // the block solver: a word per right-hand side
 struct Note {
   uint64_t *word, seq;
   __device__ __forceinline__ void tell(int flag) const {
     __hip_atomic_store(word, seq << 2 | (uint64_t)flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 };
-inline Note next_note(Context *c) { return Note{c->note, ++c->note_seq}; }
+inline Note next_note(Context *c, int k = 0) { return Note{c->note + k, ++c->note_seq}; }
+// waits until word k holds a report of number `seq` or later; its value in *v
+int wait_note(Context *c, int k, uint64_t seq, uint64_t *v);
 
 class Watch {
  public:

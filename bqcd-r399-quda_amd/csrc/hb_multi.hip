@@ -30,6 +30,7 @@ struct MultiState {
   double alpha[4][16];  // of each RHS's last iterations, for its x_lo update (MultiRing)
   int xpend[16];        // the iteration ran: its p update is due
   int cur[16];          // slot of the ring that holds its search direction at a reliable update
+  int from[16];         // first slot that x_lo has not taken up
   int flag[16];   // 0 iterate, 1 reliable update due, 2 converged, 3 maxiter, 4 unused lane
   int iter[16], since[16], nrel[16];
   double delta;
@@ -239,12 +240,18 @@ struct FinMultiStore {
 
 struct FinMultiUpdate {
   MultiState *st;
-  int slot;  // of the iteration in the ring
+  int slot;   // of the iteration in the ring
+  Note note;  // the first RHS's
   __device__ void operator()(int k, double rn) const {
+    update(k, rn);
+    Note{note.word + k, note.seq}.tell(st->flag[k] & 3);
+  }
+  __device__ __forceinline__ void update(int k, double rn) const {
     if (st->flag[k] != 0) {
       st->xpend[k] = 0;  // the p update of a skipped iteration adds nothing to x_lo
       return;
     }
+    if (slot == 0) st->from[k] = 0;
     st->alpha[slot][k] = st->rtr[k] / st->pap[k];  // the alpha of k_multi_update
     st->xpend[k] = 1;
     st->cur[k] = slot;
@@ -316,7 +323,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_pupdate(MultiRing<S> ring, Spi
     float2 x[12];
 #pragma unroll
     for (int k = 0; k < 12; k++) x[k] = xlo[(size_t)k * vhe + tid];
-    for (int q = 0; q <= slot; q++) {
+    for (int q = st->from[k0]; q <= slot; q++) {
       const float alpha = (float)st->alpha[q][k0];
       load_spinor<S>(pv, ring.p[q], tid, vhe);
 #pragma unroll
@@ -381,7 +388,8 @@ __global__ __launch_bounds__(kBlock) void k_multi_true_residual(double2 *__restr
 
 struct FinMultiTrue {
   MultiState *st;
-  int k0, first;
+  int k0, first, slot;  // the ring's slot of the RHS's next iteration
+  Note note;
   __device__ void operator()(const double (&t)[1]) const {
     const double rt = t[0];
     st->res[k0] = rt;
@@ -397,12 +405,14 @@ struct FinMultiTrue {
       st->rtr[k0] = rt;
       st->flag[k0] = 0;
     }
+    st->from[k0] = slot;
+    note.tell(st->flag[k0]);
   }
 };
 
 template <class S, int NR>
 __global__ __launch_bounds__(kBlock) void k_multi_prestart(MultiRing<S> ring, SpinorPtr<S> r, int vh,
-                                                           int k0, const MultiState *st) {
+                                                           int k0, const MultiState *st, int slot) {
   using V = typename S::V;
   if (st->flag[k0] != 0) return;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -421,7 +431,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_prestart(MultiRing<S> ring, Sp
     pv[k].x = rv[k].x + beta * pv[k].x;
     pv[k].y = rv[k].y + beta * pv[k].y;
   }
-  store_spinor<S>(ring.p[0], ie, vhe, pv);
+  store_spinor<S>(ring.p[slot], ie, vhe, pv);
 }
 
 // conversions of the per-group clover fields --------------------------------------
@@ -658,7 +668,8 @@ int cg_multi_block(Context *c, const MultiPlan &plan, const MultiFields<S, G> &f
   HB_TRY(rc);
   // FP64 true residual of RHS k -> r_lo[k], state; uses the RHS's kappa-group
   // clover term (or none), swapped into the context for the FP64 operator
-  auto reliable = [&](int k, int first) -> int {
+  uint64_t told[NR] = {};  // last report enqueued for each RHS
+  auto reliable = [&](int k, int first, int slot) -> int {
     double2 *sa = c->clov[HB_CLOVER_A], *si = c->clov[HB_CLOVER_AINV];
     const bool ha = c->have_clover[HB_CLOVER_A], hi = c->have_clover[HB_CLOVER_AINV];
     c->have_clover[HB_CLOVER_A] = c->have_clover[HB_CLOVER_AINV] = plan.clover;
@@ -677,80 +688,47 @@ int cg_multi_block(Context *c, const MultiPlan &plan, const MultiFields<S, G> &f
     c->have_clover[HB_CLOVER_AINV] = hi;
     HB_TRY(rr);
     k_multi_true_residual<S, NR><<<nblocks(vh), kBlock, 0, c->stream>>>(ax, b[idx[k]], r, vh, k, c->red);
-    k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(c->red, nblocks(vh), nullptr, FinMultiTrue{st, k, first});
-    k_multi_prestart<S, NR><<<nblocks(vh), kBlock, 0, c->stream>>>(ring, r, vh, k, st);
+    k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(c->red, nblocks(vh), nullptr,
+                                                    FinMultiTrue{st, k, first, slot, next_note(c, k)});
+    told[k] = c->note_seq;
+    k_multi_prestart<S, NR><<<nblocks(vh), kBlock, 0, c->stream>>>(ring, r, vh, k, st, slot);
     HB_HIP(hipGetLastError());
     return HB_OK;
   };
-  for (int k = 0; k < nb; k++) HB_TRY(reliable(k, 1));
+  for (int k = 0; k < nb; k++) HB_TRY(reliable(k, 1, 0));
 
-  // one batched iteration; captured once into a graph and replayed
+  // one batched iteration
   auto iteration = [&](int slot) -> int {
     HB_TRY((multi_apply<S, G, NR>(c, f, plan.ngroups, grp, kap, rh, q, ring.p[slot], t, y, st, plan.clover)));
     const int tile = c->multi_tile;
     const int grid = nblocks(vh * NR, tile);
     k_multi_update<S, NR><<<grid, tile, 0, c->stream>>>(r, q, vh, st, part);
-    k_finalize_each<NR><<<1, kFinThreads, 0, c->stream>>>(part, grid, FinMultiUpdate{st, slot});
+    k_finalize_each<NR><<<1, kFinThreads, 0, c->stream>>>(part, grid, FinMultiUpdate{st, slot, next_note(c)});
     k_multi_pupdate<S, NR><<<grid, tile, 0, c->stream>>>(ring, r, xlo, vh, st, slot);
     HB_HIP(hipGetLastError());
     return HB_OK;
   };
-  const int chunk = 8;  // a multiple of the ring's four slots
-  // the captured chunk and its executable, destroyed on every return path
-  struct Graph {
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    ~Graph() {
-      if (exec) (void)hipGraphExecDestroy(exec);
-      if (graph) (void)hipGraphDestroy(graph);
-    }
-  } gr;
-  HB_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  int crc = HB_OK;
-  for (int k = 0; k < chunk && crc == HB_OK; k++) crc = iteration(k & 3);
-  hipError_t ce = hipStreamEndCapture(c->stream, &gr.graph);
-  HB_TRY(crc);
-  if (ce != hipSuccess) {
-    set_error("hipStreamEndCapture: %s", hipGetErrorString(ce));
-    return HB_E_HIP;
-  }
-  HB_HIP(hipGraphInstantiate(&gr.exec, gr.graph, nullptr, nullptr, 0));
-  int result = HB_OK;
-  for (;;) {
-    hipError_t le = hipGraphLaunch(gr.exec, c->stream);
-    if (le == hipSuccess) le = hipMemcpyAsync(hs, st, sizeof(MultiState), hipMemcpyDeviceToHost, c->stream);
-    if (le == hipSuccess) le = hipStreamSynchronize(c->stream);
-    if (le != hipSuccess) {
-      set_error("multi-RHS iteration: %s", hipGetErrorString(le));
-      result = HB_E_HIP;
-      break;
-    }
-    bool any_active = false, any_rel = false;
+  // an iteration is enqueued once the one before the last is known to have run: an
+  // RHS waits one iteration for its reliable update (see Note).  In a captured
+  // graph of eight iterations its lanes idled for four on average: us per
+  // iteration of 4 RHS, graph / this, 8^4 68.8 / 62.5, 12^3x24 94.1 / 81.7, 16^3x32
+  // 155 / 140, 24^3x48 654 / 612; of 2 RHS 57.3 / 55.3 and 333 / 336.
+  for (int it = 0, active = 1; active; it++) {
+    uint64_t want[NR];
+    for (int k = 0; k < nb; k++) want[k] = told[k];
+    HB_TRY(iteration(it & 3));
+    for (int k = 0; k < nb; k++) told[k] = c->note_seq;
+    active = 0;
     for (int k = 0; k < nb; k++) {
-      if (hs->flag[k] == 0) any_active = true;
-      if (hs->flag[k] == 1) any_rel = true;
+      uint64_t v;
+      HB_TRY(wait_note(c, k, want[k], &v));
+      const int flag = (int)(v & 3);
+      if (flag == 1) HB_TRY(reliable(k, 0, (it + 1) & 3));
+      active |= flag <= 1;
     }
-    if (any_rel) {
-      for (int k = 0; k < nb; k++)
-        if (hs->flag[k] == 1) {
-          result = reliable(k, 0);
-          if (result) break;
-        }
-      if (result) break;
-      hipError_t le2 = hipMemcpyAsync(hs, st, sizeof(MultiState), hipMemcpyDeviceToHost, c->stream);
-      if (le2 == hipSuccess) le2 = hipStreamSynchronize(c->stream);
-      if (le2 != hipSuccess) {
-        set_error("multi-RHS reliable update: %s", hipGetErrorString(le2));
-        result = HB_E_HIP;
-        break;
-      }
-      any_active = false;
-      for (int k = 0; k < nb; k++)
-        if (hs->flag[k] == 0) any_active = true;
-    }
-    if (!any_active) break;
   }
-  HB_TRY(result);
+  HB_HIP(hipMemcpyAsync(hs, st, sizeof(MultiState), hipMemcpyDeviceToHost, c->stream));
+  HB_HIP(hipStreamSynchronize(c->stream));
   for (int k = 0; k < nb; k++) {
     if (iters) iters[idx[k]] = hs->iter[k];
     if (true_rtr) true_rtr[idx[k]] = hs->res[k];

@@ -67,3 +67,22 @@ def test_end_by_convergence_and_without_iterations(problem):
             want = x.clone()
             it, _, _ = g.cg_mixed_d("mtdagmt", x, b, KAPPA, rest=1e-15 * bb, maxiter=500, precision=prec)
             assert it == 0 and torch.equal(x, want)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f16"])
+@pytest.mark.parametrize("n", [1, 3, 4])
+def test_right_hand_sides_that_end_apart(problem, prec, n):
+    """each has its reliable updates and its end in iterations of its own, so
+    that they start again from any of the four buffers; the residual returned
+    is the true one, formed as above"""
+    import torch
+    g, b = problem
+    bs = [b, b.roll(1, 1), b.roll(5, 1), -b.flip(0)][:n]
+    bs = [v.contiguous() for v in bs]
+    xs = [torch.zeros_like(v) for v in bs]
+    rests = [float(v.square().sum()) * 10.0 ** -(5 + 3 * k) for k, v in enumerate(bs)]
+    its, rtrs, _ = g.cg_multi_d("mtdagmt", xs, bs, [KAPPA] * n, csw=-1.0, rests=rests, maxiter=500,
+                                precision=prec, block=1 if n == 1 else 4)
+    assert its == sorted(its) and its[0] > 0
+    for x, v, rest, rtr in zip(xs, bs, rests, rtrs):
+        assert rtr <= (1.0 + 1e-6) * rest and abs(rtr - residual(g, x, v)) < 1e-6 * rtr
