@@ -256,7 +256,8 @@ def cpu_baseline(g, b_dev, kappa, csw, gpu_iters, cpu_iters, what="the GPU FP64 
                       "the %d iterations of %s" % (lat_s, threads, model, it, cg_s, 1e3 * per_iter,
                                                   wall, gpu_iters, what),
         }
-    # oracle port (single thread)
+    # oracle port (single thread: a second per iteration at 32^3x64)
+    cpu_iters = min(cpu_iters, 20)
     sys.path.insert(0, os.path.join(REPO, "tests"))
     import oracle_lib as ol
 

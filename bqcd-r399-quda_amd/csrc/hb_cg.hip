@@ -155,7 +155,7 @@ double2 *spinor_scratch(Context *c, int slot, int *rc) {
 
 // The FP64 CG iteration on device fields, with its work fields given: x is
 // the initial guess in and the solution out.  `hs` is host memory the state
-// is read back into between chunks of iterations.
+// is read back into at the end.
 int cg_f64_run(Context *c, const CgWork &w, int op, double kappa, double rho, double2 *x,
                const double2 *b, float rest, int maxiter, int log, int *iters, double *true_rtr,
                int *n_matvec) {

@@ -18,19 +18,6 @@ __device__ __forceinline__ M3 m3_zero() {
   for (int k = 0; k < 9; k++) r.m[k] = make_double2(0.0, 0.0);
   return r;
 }
-__device__ __forceinline__ M3 m3_one() {
-  M3 r = m3_zero();
-  r.m[0].x = r.m[4].x = r.m[8].x = 1.0;
-  return r;
-}
-__device__ __forceinline__ M3 m3_dag(const M3 &a) {
-  M3 r;
-#pragma unroll
-  for (int i = 0; i < 3; i++)
-#pragma unroll
-    for (int j = 0; j < 3; j++) r.m[3 * i + j] = cconj(a.m[3 * j + i]);
-  return r;
-}
 // s += a' b' with a' = conj(a) if CA, b' = conj(b) if CB: four chained FMAs
 // (the force, clover and link-update kernels are bound by FP64 issue; the
 // sign flips are free operand modifiers)
