@@ -60,7 +60,7 @@ int cg_update(Context *c, double2 *r, const double2 *q, CgState *st, int k, cons
 // Search directions: p of iteration k is p[k & 3].  Four buffers on lattices
 // that are bound by the bytes of the updates: x then takes up four directions
 // at a time, in the order and with the sums of one at a time.  One (all four
-// the same) elsewhere.
+// the same) elsewhere, and where there is no memory for the others (spare()).
 struct CgRing {
   double2 *p[4];
 };

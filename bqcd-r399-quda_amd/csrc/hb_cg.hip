@@ -106,7 +106,7 @@ int ensure_links_two_rows(Context *c, bool *use) {
   if (c->link_recon != 12) return HB_OK;
   if (c->r64_gauge_version != c->gauge_version) {
     const size_t vh = c->g.vh;
-    if (!c->gauge64r) HB_HIP(hipMalloc(&c->gauge64r, sizeof(double2) * 48 * vh));
+    if (!c->gauge64r) HB_HIP(device_alloc(c, &c->gauge64r, sizeof(double2) * 48 * vh));
     unsigned int *dev = reinterpret_cast<unsigned int *>(c->red);
     HB_TRY(zero_f64(c, reinterpret_cast<double2 *>(c->red), 1));
     k_links_two_rows<<<dim3(nblocks((int)vh), 8), kBlock, 0, c->stream>>>(c->gauge64r, c->gauge, (int)vh, dev);
@@ -216,17 +216,17 @@ int cg_f64(Context *c, int op, double kappa, double rho, double2 *x, const doubl
   w.t = spinor_scratch(c, SLOT_T, &rc); HB_TRY(rc);
   w.y = spinor_scratch(c, SLOT_Y, &rc); HB_TRY(rc);
   w.r = spinor_scratch(c, SLOT_R, &rc); HB_TRY(rc);
-  const bool ring = operator_policy<SF64, SF64R>(c->g.vh) == kNT;
-  for (int q = 0; q < 4; q++) {
-    w.p.p[q] = spinor_scratch(c, ring && q > 0 ? SLOT_P1 + q - 1 : SLOT_P, &rc);
-    HB_TRY(rc);
-  }
+  double2 *p = spinor_scratch(c, SLOT_P, &rc); HB_TRY(rc);
   w.q = spinor_scratch(c, SLOT_Q, &rc); HB_TRY(rc);
   w.st = static_cast<CgState *>(scratch(c, SLOT_STATE, sizeof(CgState), &rc)); HB_TRY(rc);
   w.red = c->red;
   HB_TRY(ensure_host_stage(c, sizeof(CgState)));
   w.hs = static_cast<CgState *>(c->host_stage);
   HB_TRY(ensure_links_two_rows(c, &w.recon));
+  const size_t n = 12 * (size_t)c->g.vh;
+  double2 *ring = operator_policy<SF64, SF64R>(c->g.vh) == kNT
+                      ? static_cast<double2 *>(spare(c, 3 * n * sizeof(double2))) : nullptr;
+  for (int q = 0; q < 4; q++) w.p.p[q] = ring && q > 0 ? ring + (q - 1) * n : p;
 
   EventTimer tm;
   HB_TRY(tm.create());

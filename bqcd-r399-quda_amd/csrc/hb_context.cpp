@@ -21,7 +21,7 @@ int ensure_dev_stage(Context *c, size_t bytes) {
   if (c->dev_stage) HB_HIP(hipFree(c->dev_stage));
   c->dev_stage = nullptr;
   c->dev_stage_bytes = 0;
-  HB_HIP(hipMalloc(&c->dev_stage, bytes));
+  HB_HIP(device_alloc(c, &c->dev_stage, bytes));
   c->dev_stage_bytes = bytes;
   return HB_OK;
 }
@@ -66,6 +66,34 @@ int Watch::look(int *flag) {
   return HB_OK;
 }
 
+static bool release_spare(Context *c) {
+  if (!c->spare.p) return false;
+  (void)hipFree(c->spare.p);
+  c->spare = Field{};
+  return true;
+}
+
+hipError_t device_alloc_bytes(Context *c, void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory || !release_spare(c)) return e;
+  (void)hipGetLastError();
+  return hipMalloc(p, bytes);
+}
+
+void *spare(Context *c, size_t bytes) {
+  if (c->spare.bytes >= bytes) return c->spare.p;
+  release_spare(c);
+  size_t free = 0, total = 0;
+  if (hipMemGetInfo(&free, &total) != hipSuccess || free < bytes + total / 4 ||
+      hipMalloc(&c->spare.p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    c->spare = Field{};
+    return nullptr;
+  }
+  c->spare.bytes = bytes;
+  return c->spare.p;
+}
+
 // Scratch slots grow on demand and are kept for the life of the context.
 void *scratch(Context *c, int slot, size_t bytes, int *rc) {
   *rc = HB_OK;
@@ -82,7 +110,7 @@ void *scratch(Context *c, int slot, size_t bytes, int *rc) {
   }
   f.p = nullptr;
   f.bytes = 0;
-  hipError_t e = hipMalloc(&f.p, bytes);
+  hipError_t e = device_alloc(c, &f.p, bytes);
   if (e != hipSuccess) {
     set_error("hipMalloc(scratch %zu bytes): %s", bytes, hipGetErrorString(e));
     *rc = HB_E_NOMEM;
@@ -164,6 +192,7 @@ int hb_finalize(hb_context *ctx) {
   (void)hipFree(c->gauge16);
   for (auto *p : c->clov16) (void)hipFree(p);
   for (auto &f : c->scratch) (void)hipFree(f.p);
+  (void)hipFree(c->spare.p);
   (void)hipFree(c->red);
   (void)hipFree(c->dev_stage);
   if (c->host_stage) (void)hipHostFree(c->host_stage);

@@ -155,9 +155,9 @@ int gen_download(Context *c, double *host, const double *src_d, int stride) {
 
 int alloc_fp64_fields(Context *c) {
   size_t vh = c->g.vh;
-  if (!c->gauge) HB_HIP(hipMalloc(&c->gauge, sizeof(double2) * 72 * vh));
+  if (!c->gauge) HB_HIP(device_alloc(c, &c->gauge, sizeof(double2) * 72 * vh));
   for (int k = 0; k < 3; k++)
-    if (!c->clov[k]) HB_HIP(hipMalloc(&c->clov[k], sizeof(double2) * 72 * vh));
+    if (!c->clov[k]) HB_HIP(device_alloc(c, &c->clov[k], sizeof(double2) * 72 * vh));
   return HB_OK;
 }
 

@@ -362,7 +362,7 @@ int hb_gauge_smear(hb_context *ctx, int sweeps, double alpha) {
   HB_TRY(check_ready(c));
   HB_HIP(hipSetDevice(c->device));
   double2 *tmp = nullptr;
-  HB_HIP(hipMalloc(&tmp, sizeof(double2) * 72 * (size_t)c->g.vh));
+  HB_HIP(device_alloc(c, &tmp, sizeof(double2) * 72 * (size_t)c->g.vh));
   for (int s = 0; s < sweeps; s++) {
     k_ape<<<dim3(nblocks(c->g.vh, 128), 8), 128, 0, c->stream>>>(tmp, c->gauge, c->g, alpha);
     hipError_t e = hipGetLastError();

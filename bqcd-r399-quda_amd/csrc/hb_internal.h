@@ -146,6 +146,7 @@ struct Context {
   uint64_t lp_gauge_version = 0, lp_clover_version = 0;
   // scratch
   std::vector<Field> scratch;
+  Field spare;                       // see spare()
   double *red = nullptr;             // per-block partial sums of the reductions
   int red_blocks = 0;
   void *host_stage = nullptr;        // pinned staging
@@ -169,6 +170,19 @@ struct Context {
   // scratch slots (0: none); a backward test trajectory integrates with them
   char hmc_phi_model = 0;
 };
+
+// hipMalloc for the context; memory held by spare() gives way to it
+hipError_t device_alloc_bytes(Context *c, void **p, size_t bytes);
+template <class T> hipError_t device_alloc(Context *c, T **p, size_t bytes) {
+  return device_alloc_bytes(c, reinterpret_cast<void **>(p), bytes);
+}
+// Memory that a solve is faster with and can do without (the further search
+// directions of its ring), one area for all solvers, kept for the next solve.
+// Null if less than a quarter of the GPU's memory would be left, so that the
+// gain in speed costs neither another field of this context (device_alloc) nor
+// the rest of the program its room.  A solver asks for it after all else: any
+// later allocation may take it back.
+void *spare(Context *c, size_t bytes);
 
 int ensure_dev_stage(Context *c, size_t bytes);
 int ensure_host_stage(Context *c, size_t bytes);

@@ -252,12 +252,14 @@ __global__ __launch_bounds__(kBlock) void k_mix_pupdate(SpinorPtr<S> p, SpinorPt
 // slot k & 3, and x_lo takes up four of them at a time (or those there are,
 // when a reliable update is due): the same sums in the same order.  16-bit
 // storage at 32^3x64: 34.9 us a launch against 43.0, an iteration 474 against 493.
+// Without memory for three of the buffers (last = 0: the only slot of the ring)
+// x_lo takes up every direction as it comes.
 template <class S> struct MixRing {
   SpinorPtr<S> p[4];
 };
 struct FinMixStep {
   MixState *st;
-  int k;
+  int k, last;
   Note note;
   __device__ void operator()(const double (&t)[1]) const {
     const MixSlot c = st->s[k & 1];
@@ -265,9 +267,9 @@ struct FinMixStep {
     st->go = c.flag == 0;
     if (c.flag == 0) {
       mix_decide(d, c, st, t[0]);
-      st->alpha[k & 3] = c.rtr / st->pap;
+      st->alpha[k & last] = c.rtr / st->pap;
       st->beta = t[0] / c.rtr;
-      st->cur = k & 3;
+      st->cur = k & last;
     }
     st->s[~k & 1] = d;
     note.tell(d.flag);
@@ -275,15 +277,15 @@ struct FinMixStep {
 };
 template <class S>
 __global__ __launch_bounds__(kBlock) void k_mix_pupdate_ring(MixRing<S> ring, SpinorPtr<S> r, float2 *__restrict__ xlo,
-                                                             int n, const MixState *st, int k) {
+                                                             int n, const MixState *st, int k, int last) {
   using V = typename S::V;
   if (!st->go) return;
   const bool next = st->s[~k & 1].flag == 0;
-  const int slot = k & 3;
+  const int slot = k & last;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   V pv[12];
-  if (slot == 3 || !next) {
+  if (slot == last || !next) {
     float2 x[12];
 #pragma unroll
     for (int m = 0; m < 12; m++) x[m] = xlo[(size_t)m * n + i];
@@ -310,7 +312,7 @@ __global__ __launch_bounds__(kBlock) void k_mix_pupdate_ring(MixRing<S> ring, Sp
     pv[m].x = rv[m].x + beta * pv[m].x;
     pv[m].y = rv[m].y + beta * pv[m].y;
   }
-  store_spinor<S>(ring.p[(k + 1) & 3], i, n, pv);
+  store_spinor<S>(ring.p[(k + 1) & last], i, n, pv);
 }
 
 // ---- reliable update kernels ------------------------------------------------------
@@ -461,23 +463,23 @@ int ensure_lowprec(Context *c, int prec) {
     return HB_OK;
   const int grid = nblocks((int)std::min<size_t>(72 * vh, (size_t)1 << 22));
   if (prec == 32) {
-    if (!c->gauge32) HB_HIP(hipMalloc(&c->gauge32, sizeof(float2) * 48 * vh));
+    if (!c->gauge32) HB_HIP(device_alloc(c, &c->gauge32, sizeof(float2) * 48 * vh));
     k_cvt_gauge_rows<SF32><<<grid, kBlock, 0, c->stream>>>(c->gauge32, c->gauge, vh);
     HB_HIP(hipGetLastError());
     if (clov) {
       for (int k = 0; k < 2; k++) {
-        if (!c->clov32[k]) HB_HIP(hipMalloc(&c->clov32[k], sizeof(float2) * 72 * vh));
+        if (!c->clov32[k]) HB_HIP(device_alloc(c, &c->clov32[k], sizeof(float2) * 72 * vh));
         k_cvt_field<SF32><<<grid, kBlock, 0, c->stream>>>(c->clov32[k], c->clov[k], 72 * vh);
         HB_HIP(hipGetLastError());
       }
     }
   } else {
-    if (!c->gauge16) HB_HIP(hipMalloc(&c->gauge16, sizeof(short2) * 48 * vh));
+    if (!c->gauge16) HB_HIP(device_alloc(c, &c->gauge16, sizeof(short2) * 48 * vh));
     k_cvt_gauge16<<<dim3(nblocks((int)vh), 8), kBlock, 0, c->stream>>>(c->gauge16, c->gauge, (int)vh);
     HB_HIP(hipGetLastError());
     if (clov) {
       for (int k = 0; k < 2; k++) {
-        if (!c->clov16[k]) HB_HIP(hipMalloc(&c->clov16[k], sizeof(short2) * 4 * kClov16Words * vh));
+        if (!c->clov16[k]) HB_HIP(device_alloc(c, &c->clov16[k], sizeof(short2) * 4 * kClov16Words * vh));
         k_cvt_clover16<<<dim3(nblocks((int)vh), 4), kBlock, 0, c->stream>>>(c->clov16[k], c->clov[k], (int)vh);
         HB_HIP(hipGetLastError());
       }
@@ -551,12 +553,6 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
   // low-precision fields (norm slots follow SLOT_LPN)
   SpinorPtr<S> p = SpinorAlloc<S>::get(c, SLOT_LP0, SLOT_LPN, &rc); HB_TRY(rc);
   const bool sums = mix_sum<S>(vh);
-  MixRing<S> ring{{p, p, p, p}};
-  if (!sums)
-    for (int q = 1; q < 4; q++) {
-      ring.p[q] = SpinorAlloc<S>::get(c, SLOT_LPR + 2 * q, SLOT_LPR + 2 * q + 1, &rc);
-      HB_TRY(rc);
-    }
   SpinorPtr<S> r = SpinorAlloc<S>::get(c, SLOT_LP1, SLOT_LPN1, &rc); HB_TRY(rc);
   SpinorPtr<S> q = SpinorAlloc<S>::get(c, SLOT_LP2, SLOT_LPN2, &rc); HB_TRY(rc);
   SpinorPtr<S> t = SpinorAlloc<S>::get(c, SLOT_LP3, SLOT_LPN3, &rc); HB_TRY(rc);
@@ -565,6 +561,8 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
   HB_TRY(ensure_host_stage(c, sizeof(MixState)));
   MixState *hs = static_cast<MixState *>(c->host_stage);
   HB_TRY(ensure_lowprec(c, G::kBytes == 8 ? 32 : 16));
+  MixRing<S> ring{{p, p, p, p}};
+  const int last = !sums && spare_fields<S>(c, &ring.p[1], vh) ? 3 : 0;  // slot of the ring
 
   EventTimer tm;
   HB_TRY(tm.create());
@@ -605,7 +603,7 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
   Watch watch(c);
   for (int k = 0, flag = 0;;) {
     const int *skip = &st->s[k & 1].flag;
-    const SpinorPtr<S> pk = ring.p[k & 3];
+    const SpinorPtr<S> pk = ring.p[k & last];
     HB_TRY((mtil_lp<S, G>(c, false, kappa, r_op, y, pk, t, nullptr, SpinorPtr<S>{}, skip)));
     HB_TRY((mtil_lp<S, G>(c, true, kappa, r_op, q, y, t, pa, pk, skip)));
     const double *sum = pa;
@@ -617,8 +615,8 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
       k_mix_pupdate<S><<<grid, block, 0, c->stream>>>(p, r, xlo, n, st, k, pb, grid, note);
     } else {
       k_mix_update<S, false><<<grid, block, 0, c->stream>>>(r, q, n, st, k, sum, nsum, pb);
-      k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(pb, grid, nullptr, FinMixStep{st, k, note});
-      if constexpr (!kLinear<S>) k_mix_pupdate_ring<S><<<grid, block, 0, c->stream>>>(ring, r, xlo, n, st, k);
+      k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(pb, grid, nullptr, FinMixStep{st, k, last, note});
+      if constexpr (!kLinear<S>) k_mix_pupdate_ring<S><<<grid, block, 0, c->stream>>>(ring, r, xlo, n, st, k, last);
     }
     HB_HIP(hipGetLastError());
     HB_TRY(watch.look(&flag));

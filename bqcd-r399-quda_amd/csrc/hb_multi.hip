@@ -305,13 +305,14 @@ __global__ __launch_bounds__(kBlock) void k_multi_update(SpinorPtr<S> r, SpinorP
 // p = r + beta p for every RHS that goes on.  Search directions go round four
 // buffers, and x_lo takes up four of them at a time, or those there are when a
 // reliable update of the RHS is due (the same sums in the same order): half of
-// the bytes of this kernel were x_lo's.  4 RHS at 24^3x48: 70 -> 57 us
+// the bytes of this kernel were x_lo's.  4 RHS at 24^3x48: 70 -> 57 us.  Without
+// memory for three of them (last = 0: the only slot of the ring) x_lo takes up every one.
 template <class S> struct MultiRing {
   SpinorPtr<S> p[4];
 };
 template <class S, int NR>
 __global__ __launch_bounds__(kBlock) void k_multi_pupdate(MultiRing<S> ring, SpinorPtr<S> r, float2 *__restrict__ xlo,
-                                                          int vh, const MultiState *st, int slot) {
+                                                          int vh, const MultiState *st, int slot, int last) {
   using V = typename S::V;
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
   const int site = tid / NR, k0 = tid - site * NR;
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_pupdate(MultiRing<S> ring, Spi
   const int vhe = vh * NR;
   const bool next = st->flag[k0] == 0;
   V pv[12];
-  if (slot == 3 || !next) {
+  if (slot == last || !next) {
     float2 x[12];
 #pragma unroll
     for (int k = 0; k < 12; k++) x[k] = xlo[(size_t)k * vhe + tid];
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_pupdate(MultiRing<S> ring, Spi
     pv[k].x = rv[k].x + beta * pv[k].x;
     pv[k].y = rv[k].y + beta * pv[k].y;
   }
-  store_spinor<S>(ring.p[(slot + 1) & 3], tid, vhe, pv);
+  store_spinor<S>(ring.p[(slot + 1) & last], tid, vhe, pv);
 }
 
 // reliable update of RHS k0: x += x_lo[k0]; x_lo[k0] = 0
@@ -625,11 +626,6 @@ int cg_multi_block(Context *c, const MultiPlan &plan, const MultiFields<S, G> &f
   const int vh = c->g.vh, nb = (int)idx.size();
   int rc = 0;
   SpinorPtr<S> p = block_field<S>(c, SLOT_MULTI + 0, SLOT_MULTI + 10, NR, &rc); HB_TRY(rc);
-  MultiRing<S> ring{{p, p, p, p}};
-  for (int q = 1; q < 4; q++) {
-    ring.p[q] = block_field<S>(c, SLOT_MULTI_RING + 2 * q - 2, SLOT_MULTI_RING + 2 * q - 1, NR, &rc);
-    HB_TRY(rc);
-  }
   SpinorPtr<S> r = block_field<S>(c, SLOT_MULTI + 1, SLOT_MULTI + 11, NR, &rc); HB_TRY(rc);
   SpinorPtr<S> q = block_field<S>(c, SLOT_MULTI + 2, SLOT_MULTI + 12, NR, &rc); HB_TRY(rc);
   SpinorPtr<S> t = block_field<S>(c, SLOT_MULTI + 3, SLOT_MULTI + 13, NR, &rc); HB_TRY(rc);
@@ -666,6 +662,8 @@ int cg_multi_block(Context *c, const MultiPlan &plan, const MultiFields<S, G> &f
 
   double *part = multi_partials(c, NR, &rc);
   HB_TRY(rc);
+  MultiRing<S> ring{{p, p, p, p}};
+  const int last = spare_fields<S>(c, &ring.p[1], vh * NR) ? 3 : 0;  // slot of the ring
   // FP64 true residual of RHS k -> r_lo[k], state; uses the RHS's kappa-group
   // clover term (or none), swapped into the context for the FP64 operator
   uint64_t told[NR] = {};  // last report enqueued for each RHS
@@ -704,7 +702,7 @@ int cg_multi_block(Context *c, const MultiPlan &plan, const MultiFields<S, G> &f
     const int grid = nblocks(vh * NR, tile);
     k_multi_update<S, NR><<<grid, tile, 0, c->stream>>>(r, q, vh, st, part);
     k_finalize_each<NR><<<1, kFinThreads, 0, c->stream>>>(part, grid, FinMultiUpdate{st, slot, next_note(c)});
-    k_multi_pupdate<S, NR><<<grid, tile, 0, c->stream>>>(ring, r, xlo, vh, st, slot);
+    k_multi_pupdate<S, NR><<<grid, tile, 0, c->stream>>>(ring, r, xlo, vh, st, slot, last);
     HB_HIP(hipGetLastError());
     return HB_OK;
   };
@@ -716,14 +714,14 @@ int cg_multi_block(Context *c, const MultiPlan &plan, const MultiFields<S, G> &f
   for (int it = 0, active = 1; active; it++) {
     uint64_t want[NR];
     for (int k = 0; k < nb; k++) want[k] = told[k];
-    HB_TRY(iteration(it & 3));
+    HB_TRY(iteration(it & last));
     for (int k = 0; k < nb; k++) told[k] = c->note_seq;
     active = 0;
     for (int k = 0; k < nb; k++) {
       uint64_t v;
       HB_TRY(wait_note(c, k, want[k], &v));
       const int flag = (int)(v & 3);
-      if (flag == 1) HB_TRY(reliable(k, 0, (it + 1) & 3));
+      if (flag == 1) HB_TRY(reliable(k, 0, (it + 1) & last));
       active |= flag <= 1;
     }
   }
@@ -979,8 +977,8 @@ int hb_cg_multi(hb_context *ctx, int op, int nrhs, const double *kappa, const do
   std::vector<double2 *> dx(nrhs), db(nrhs);
   int rc = HB_OK;
   for (int k = 0; k < nrhs && rc == HB_OK; k++) {
-    hipError_t e = hipMalloc(&dx[k], bytes);
-    if (e == hipSuccess) e = hipMalloc(&db[k], bytes);
+    hipError_t e = device_alloc(c, &dx[k], bytes);
+    if (e == hipSuccess) e = device_alloc(c, &db[k], bytes);
     if (e != hipSuccess) {
       set_error("hb_cg_multi: %s", hipGetErrorString(e));
       rc = HB_E_NOMEM;

@@ -18,9 +18,6 @@ enum {
   SLOT_IN,
   SLOT_OUT,
   SLOT_STATE,      // CgState
-  SLOT_P1,         // further search directions (CgRing)
-  SLOT_P2,
-  SLOT_P3,
   SLOT_LP0,        // low-precision fields of the mixed solver
   SLOT_LP1,
   SLOT_LP2,
@@ -31,8 +28,6 @@ enum {
   SLOT_LPN2,
   SLOT_LPN3,
   SLOT_LPN4,
-  SLOT_LPR,        // search directions of the mixed solver's ring and their norms: +2 .. +7
-  SLOT_LPR_LAST = SLOT_LPR + 7,
   SLOT_MIX0,       // FP64 fields of the mixed solver
   SLOT_MIX1,
   SLOT_FORCE0,     // force temporaries
@@ -61,8 +56,7 @@ enum {
   SLOT_HMC_MV = SLOT_HMC + 24,                      // kMaxMre products M v_i
   SLOT_HMC_MRE = SLOT_HMC_MV + kMaxMre,             // 2 bases of kMaxMre vectors
   SLOT_PLUGIN = SLOT_HMC_MRE + 2 * kMaxMre,         // staging of the plugin entry points (hb_plugin.hip), 6 slots
-  SLOT_MULTI_RING = SLOT_PLUGIN + 6,                // search directions of the multi-RHS ring and their norms, 6 slots
-  SLOT_END = SLOT_MULTI_RING + 6
+  SLOT_END = SLOT_PLUGIN + 6
 };
 static_assert(SLOT_SINGLE_END <= SLOT_MULTI, "single-RHS slots overlap the multi-RHS range");
 static_assert(SLOT_MULTI_LAST < SLOT_MULTI_CLOVER_B, "multi-RHS fields overlap the clover scratch");
@@ -90,6 +84,19 @@ int mtil_f64(Context *c, bool dag, double kappa, double rho, double2 *out, const
 int apply_f64(Context *c, int op, double kappa, double rho, double2 *out, const double2 *in,
               double2 *t, double2 *y, double *dot, const int *skip, bool recon = false);
 int ensure_links_two_rows(Context *c, bool *use);
+
+// three further fields of n sites for a solver's ring of search directions, if
+// spare() has them
+template <class S> bool spare_fields(Context *c, SpinorPtr<S> *f, int n) {
+  const size_t field = sizeof(typename S::ST) * 12 * n, norm = S::kNorm ? sizeof(float) * n : 0;
+  char *m = static_cast<char *>(spare(c, 3 * (field + norm)));
+  if (!m) return false;
+  for (int q = 0; q < 3; q++) {
+    f[q].p = reinterpret_cast<typename S::ST *>(m + q * field);
+    f[q].norm = S::kNorm ? reinterpret_cast<float *>(m + 3 * field + q * norm) : nullptr;
+  }
+  return true;
+}
 
 // work fields of the FP64 CG: operator temporaries t (odd) and y (even), the
 // CG vectors r, p, q = A p, the device state, the reduction partials
