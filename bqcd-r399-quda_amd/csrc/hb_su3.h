@@ -154,9 +154,9 @@ __device__ __forceinline__ void m3_reunitarize(M3 &u) {
   double len = 0.0;
 #pragma unroll
   for (int r = 0; r < 3; r++) len += u.m[3 * r].x * u.m[3 * r].x + u.m[3 * r].y * u.m[3 * r].y;
-  len = 1.0 / sqrt(len);
+  len = sqrt(len);
 #pragma unroll
-  for (int r = 0; r < 3; r++) u.m[3 * r] = cscale<double2>(len, u.m[3 * r]);
+  for (int r = 0; r < 3; r++) u.m[3 * r] = make_double2(u.m[3 * r].x / len, u.m[3 * r].y / len);
   double2 f = make_double2(0.0, 0.0);
 #pragma unroll
   for (int r = 0; r < 3; r++) cfmac(f, u.m[3 * r], u.m[3 * r + 1]);  // sum conj(u_r0) u_r1
@@ -166,9 +166,9 @@ __device__ __forceinline__ void m3_reunitarize(M3 &u) {
 #pragma unroll
   for (int r = 0; r < 3; r++)
     len += u.m[3 * r + 1].x * u.m[3 * r + 1].x + u.m[3 * r + 1].y * u.m[3 * r + 1].y;
-  len = 1.0 / sqrt(len);
+  len = sqrt(len);
 #pragma unroll
-  for (int r = 0; r < 3; r++) u.m[3 * r + 1] = cscale<double2>(len, u.m[3 * r + 1]);
+  for (int r = 0; r < 3; r++) u.m[3 * r + 1] = make_double2(u.m[3 * r + 1].x / len, u.m[3 * r + 1].y / len);
   u.m[2] = cconj(csub(cmul(u.m[3], u.m[7]), cmul(u.m[6], u.m[4])));
   u.m[5] = cconj(csub(cmul(u.m[6], u.m[1]), cmul(u.m[0], u.m[7])));
   u.m[8] = cconj(csub(cmul(u.m[0], u.m[4]), cmul(u.m[3], u.m[1])));
