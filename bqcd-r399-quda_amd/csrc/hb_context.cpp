@@ -2,6 +2,7 @@
 #include <cstdarg>
 #include <cstring>
 #include <mutex>
+#include <thread>
 
 #include "hb_internal.h"
 
@@ -42,6 +43,7 @@ int wait_note(Context *c, int k, uint64_t seq, uint64_t *v) {
     if (*v >> 2 >= seq) return HB_OK;
     __builtin_ia32_pause();
     if (spin % 4096) continue;
+    std::this_thread::yield();  // there may be more threads with a context than cores
     // every report has been written once the stream is empty: the wait ends
     // there also when a kernel failed
     const hipError_t e = hipStreamQuery(c->stream);
@@ -167,7 +169,10 @@ int hb_init(const int L[4], const int bc[4], int device, hb_context **out) {
   // reduction partials: up to 16 values per block of a site-parallel grid
   c->red_blocks = nblocks(2 * c->g.vh) + 64;
   e = hipMalloc(&c->red, sizeof(double) * 16 * (size_t)c->red_blocks);
-  if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&c->note), kNotes * sizeof(uint64_t), hipHostMallocDefault);
+  // the host reads the notes while the kernels that write them are in flight, so
+  // the words must be coherent whatever the runtime's default is (HIP_HOST_COHERENT)
+  if (e == hipSuccess)
+    e = hipHostMalloc(reinterpret_cast<void **>(&c->note), kNotes * sizeof(uint64_t), hipHostMallocCoherent);
   if (e != hipSuccess) {
     set_error("hb_init: %s", hipGetErrorString(e));
     hb_finalize(reinterpret_cast<hb_context *>(c));

@@ -54,6 +54,7 @@ int main() {
   const int L[4] = {2, 2, 2, 2}, bc[4] = {1, 1, 1, -1};
   hb_context *h = nullptr;
   EXPECT(hb_init(L, bc, 0, &h) == HB_OK);
+  EXPECT(host_flags & hipHostMallocCoherent);  // the words that running kernels report to
   hb::Context *c = reinterpret_cast<hb::Context *>(h);
   const size_t base = used, unit = (total - base) / 16;
   int rc = 0;
