@@ -1,7 +1,7 @@
-"""The context's allocations on the CPU: hb_context.cpp with a HIP runtime of a
-few functions that counts bytes, so that running out of memory is a matter of
-arithmetic.  What spare() holds gives way to every other field, and spare()
-itself leaves a quarter of the memory free."""
+"""The context's allocations and its wait for a solve's progress on the CPU:
+hb_context.cpp with a HIP runtime of a few functions that counts bytes, so that
+running out of memory is a matter of arithmetic.  What spare() holds gives way
+to every other field, and spare() itself leaves a quarter of the memory free."""
 import os
 import subprocess
 
@@ -12,6 +12,7 @@ CSRC = os.path.join(REPO, "bqcd-r399-quda_amd", "csrc")
 CLANG = "/opt/rocm/llvm/bin/clang++"
 
 RUNTIME = r"""
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -21,6 +22,7 @@ RUNTIME = r"""
 static size_t total = 1 << 20, used = 0;
 static std::map<void *, size_t> blocks;
 static unsigned host_flags = ~0u;
+static int queries = 0;
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n) {
   *p = nullptr;
@@ -42,7 +44,7 @@ hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipStreamCreate(hipStream_t *s) { *s = nullptr; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamQuery(hipStream_t) { return ++queries < 3 ? hipErrorNotReady : hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "error"; }
@@ -77,6 +79,14 @@ int main() {
   EXPECT(hb::device_alloc(c, &p, 8 * unit) == hipErrorOutOfMemory);
   EXPECT(hb::device_alloc(c, &p, 2 * unit) == hipSuccess);
   (void)hipFree(p);
+  // the wait for a report asks the runtime now and then, and ends with an error
+  // when the stream is empty and nothing has been reported
+  uint64_t v = 0;
+  const auto t = std::chrono::steady_clock::now();
+  EXPECT(hb::wait_note(c, 0, 5, &v) == HB_E_HIP && queries == 3);
+  EXPECT(std::chrono::steady_clock::now() - t > std::chrono::milliseconds(100));
+  c->note[0] = 5 << 2 | 1;
+  EXPECT(hb::wait_note(c, 0, 5, &v) == HB_OK && v == (5 << 2 | 1) && queries == 3);
   hb_finalize(h);
   EXPECT(used == 0);
   return 0;
@@ -85,7 +95,7 @@ int main() {
 
 
 @pytest.mark.skipif(not os.path.exists(CLANG), reason="no HIP compiler")
-def test_spare_memory_gives_way(tmp_path):
+def test_allocations_and_wait(tmp_path):
     (tmp_path / "runtime.cpp").write_text(RUNTIME)
     exe = str(tmp_path / "context")
     subprocess.run([CLANG, "-O1", "-std=c++17", "-x", "hip", "--offload-host-only", "-I" + CSRC,
