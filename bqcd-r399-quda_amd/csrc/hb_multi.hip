@@ -706,11 +706,15 @@ int cg_multi_block(Context *c, const MultiPlan &plan, const MultiFields<S, G> &f
     HB_HIP(hipGetLastError());
     return HB_OK;
   };
-  // an iteration is enqueued once the one before the last is known to have run: an
-  // RHS waits one iteration for its reliable update (see Note).  In a captured
-  // graph of eight iterations its lanes idled for four on average: us per
-  // iteration of 4 RHS, graph / this, 8^4 68.8 / 62.5, 12^3x24 94.1 / 81.7, 16^3x32
-  // 155 / 140, 24^3x48 654 / 612; of 2 RHS 57.3 / 55.3 and 333 / 336.
+  // An iteration of a block is enqueued once the one before has reported: an RHS
+  // whose reliable update is due has it before the next.  The GPU waits for the
+  // host meanwhile, but with the next iteration enqueued ahead (as for one RHS,
+  // see Note) that RHS's lanes idle through it while the others go on, and the
+  // systems of a block, which begin together, drift apart and idle by turns.  us
+  // per iteration, in a captured graph of eight / one ahead / this: FP32 32^3x48,
+  // 2 RHS 1584 / 1620 / 1560, 4 RHS 3099 / 3143 / 3020; 20^3x40, 4 RHS 635 / 636 /
+  // 609; 16-bit 16^3x32, 8 RHS 403 / 357 / 341; 8^4, 4 RHS 121 / 71.2 / 69.0; one RHS,
+  // 16-bit 16^4 77.2 / 56.8 / 58.5
   for (int it = 0, active = 1; active; it++) {
     uint64_t want[NR];
     for (int k = 0; k < nb; k++) want[k] = told[k];
@@ -719,7 +723,7 @@ int cg_multi_block(Context *c, const MultiPlan &plan, const MultiFields<S, G> &f
     active = 0;
     for (int k = 0; k < nb; k++) {
       uint64_t v;
-      HB_TRY(wait_note(c, k, want[k], &v));
+      HB_TRY(wait_note(c, k, NR > 1 ? told[k] : want[k], &v));
       const int flag = (int)(v & 3);
       if (flag == 1) HB_TRY(reliable(k, 0, (it + 1) & last));
       active |= flag <= 1;
