@@ -25,24 +25,34 @@ template <class S, class G = S> struct DslashArgs {
 };
 
 // Load policy of the links and clover words, which a kernel reads once: kept
-// in the caches while the operator and the vectors of a solve are up to half
-// as large again as the 256 MB last-level cache, streamed past them (so that
-// the neighbour spinors stay) beyond.  CG iteration streamed / kept:
-//   FP64    12^3x24 (62 MB) 96.6 / 79.5 us, 16^3x32 (195 MB) 130 / 116 us,
-//           24^3x48 (987 MB) 605 / 666 us
-//   FP32    14x20x12x30 (77 MB) 88.1 / 77.5 us, 24^3x48 (510 MB) 356 / 361 us
-//   16-bit  24^3x48 (288 MB) 219 / 200 us, 32^3x64 (910 MB) 522 / 584 us;
-//           two right-hand sides at 24^3x48 (406 MB) 340 / 352 us
-//   FP32 spinors, 16-bit links and clover: 24^3x48 (361 MB) 273 / 263 us
-constexpr size_t kResidentBytes = (size_t)360 << 20;
+// in the caches while the operator and the vectors of a solve are not much
+// larger than the 256 MB last-level cache, streamed past them (so that the
+// neighbour spinors stay) beyond.  The lines in MiB of that working set, with
+// us streamed / kept on either side (sites per parity):
+//   M~^+M~ in FP64, 18-real links 340: 104 k (332 MiB) 175 / 171, 112 k (359) 183 / 188;
+//       D alone, which reads no clover words, 360: 112 k 34.1 / 32.0, 120 k 35.7 / 36.0
+//   CG iteration, FP64 372: 120 k (341) 215 / 205, 128 k (363) 225 / 216, 141 k (400) 254 / 288
+//   FP32 450: 249 k (364) 294 / 271, 304 k (446) 345 / 334, 332 k (486) 390 / 392; blocks of
+//       two 219 k (441) 423 / 416, 249 k (501) 480 / 485, of four 141 k (438) 561 / 544,
+//       200 k (623) 776 / 785
+//   16-bit 434: 470 k (389) 335 / 319, 524 k (434) 336 / 331, 655 k (543) 423 / 431; blocks 360:
+//       two 304 k (355) 361 / 360, 359 k (420) 441 / 444, four 200 k (369) 478 / 474,
+//       249 k (459) 578 / 580
+//   FP32 spinors, 16-bit links and clover 385: 359 k (373) 321 / 311, 432 k (448) 386 / 390
+template <class S, class G> constexpr size_t resident_bytes(int nr, bool clover) {
+  const size_t mib = std::is_same<S, SF64>::value   ? (G::kRecon ? 372 : clover ? 340 : 360)
+                     : std::is_same<S, SF16>::value ? (nr == 1 ? 434 : 360)
+                     : std::is_same<G, SF16>::value ? 385 : 450;
+  return mib << 20;
+}
 template <class S, class G> constexpr size_t solve_bytes_per_site(int nr = 1) {
   const size_t link = std::is_same<G, SF16>::value ? 24 : G::kRecon ? 6 * G::kBytes : 9 * G::kBytes;
   const size_t clov = std::is_same<G, SF16>::value ? 2 * kClov16 : 36 * G::kBytes;
   const size_t spin = 12 * S::kBytes + (S::kNorm ? 4 : 0);
   return 8 * link + 2 * clov + (5 * spin + 96) * nr;  // p, r, q, t, y and the FP32 increment
 }
-template <class S, class G> inline int operator_policy(int vh, int nr = 1) {
-  return solve_bytes_per_site<S, G>(nr) * (size_t)vh <= kResidentBytes ? 0 : kNT;
+template <class S, class G> inline int operator_policy(int vh, int nr = 1, bool clover = true) {
+  return solve_bytes_per_site<S, G>(nr) * (size_t)vh <= resident_bytes<S, G>(nr, clover) ? 0 : kNT;
 }
 
 // Waves that share a site (1: k_dslash, else k_dslash_split).  us per CG

@@ -257,7 +257,7 @@ static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t
 
 template <class S, class G>
 int launch_dslash(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
-  const int nw = split_waves<S, G>(a.g.vh), pol = operator_policy<S, G>(a.g.vh);
+  const int nw = split_waves<S, G>(a.g.vh), pol = operator_policy<S, G>(a.g.vh, 1, a.C != nullptr);
   if (nw == 4) {
     launch_split<S, G, 4, 0>(a, dag, epi, st);
   } else if (nw == 2) {
