@@ -67,6 +67,8 @@ template <class S, class G> inline int operator_policy(int vh, int nr = 1, bool 
 //           72.2, 24^3x48 (332 k) 365 / 356 / 358, 32^3x64 1010 / 1056 / 1067
 //   16-bit  12^3x24 60.9 / 55.4 / 52.2, 50 k 62.9 / 58.7 / 60.6, 24^3x48
 //           207 / 200 / 214, 32^3x64 522 / 548 / 580
+//   around the line of both, at 1 / 2: FP32 470 k 547 / 547, 524 k 559 / 573, 590 k 653 / 668,
+//           655 k 717 / 735; 16-bit 334 / 334, 329 / 336, 394 / 400, 424 / 432
 // Eight waves (one hop each) were slower than four from 4 k sites on.
 template <class S, class G> inline int split_waves(int vh) {
   if (vh <= (1 << 15)) return 4;
@@ -79,8 +81,9 @@ template <class S, class G> inline int split_waves(int vh) {
 // less of it idle in the last one.  256 / 64 sites, us, FP64 CG iteration and
 // M~^+M~ with 18-real links: 24x20x12x36 (104 k sites per parity, one round) 184 /
 // 183 and 170 / 176, 20^3x40 (160 k) 288 / 276 and 265 / 257, 24^3x48 (332 k) 592 /
-// 574 and 569 / 545, 32^3x64 (1049 k) 1693 / 1699 and 1621 / 1624.  FP32 and 16-bit
-// fields, at higher occupancy: 354 / 352 and 196 / 194 at 24^3x48, 998 / 1023 and
+// 574 and 569 / 545, 28x28x28x36 (395 k) 689 / 666 and 627 / 600, 32x32x32x28 (459 k) 771 /
+// 768 and 725 / 732, 28x28x30x40 (470 k) 834 / 826 and 807 / 792, 32^4 (524 k) 854 / 856 and
+// 810 / 805, 32^3x64 (1049 k) 1693 / 1699 and 1621 / 1624.  FP32 and 16-bit fields, at higher occupancy: 354 / 352 and 196 / 194 at 24^3x48, 998 / 1023 and
 // 503 / 507 at 32^3x64.
 template <class S, class G> inline int dslash_tile(int vh) {
   if (split_waves<S, G>(vh) > 1) return 64;

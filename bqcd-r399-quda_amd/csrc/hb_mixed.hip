@@ -108,8 +108,12 @@ __global__ void k_spinor_to_f64(double2 *__restrict__ dst, SpinorPtr<S> src, int
 // 16-bit fields one site per thread; n counts what a thread works on.
 template <class S> constexpr bool kLinear = !S::kNorm;
 template <class S> inline int mix_count(int vh) { return kLinear<S> ? 12 * vh : vh; }
+// 16-bit site kernels in workgroups of 64 / 256 sites, us per iteration: 2 k sites per
+// parity 35.1 / 35.6, 21 k 42.8 / 43.6, 50 k 57.7 / 57.4, 74 k 76.0 / 74.3, 104 k 94.7 / 92.0
 template <class S> inline int mix_block(int vh) { return !kLinear<S> && vh <= (1 << 16) ? 64 : kBlock; }
-// (linear fields in at most 2048 blocks that go round)
+// (linear fields in at most 2048 blocks that go round; at most 1024 / 2048 / 4096, us
+// per iteration: FP32 66 k 81.2 / 81.6 / 87.8, 200 k 218 / 220 / 228; FP64, which has the
+// same cap, 104 k 178 / 178 / 187, 332 k 578 / 578 / 581)
 template <class S> inline int mix_grid(int vh) {
   const int b = nblocks(mix_count<S>(vh), mix_block<S>(vh));
   return kLinear<S> && b > 2048 ? 2048 : b;
@@ -119,7 +123,9 @@ template <class S> inline int mix_grid(int vh) {
 // operands are on their way (SUM), except in the site kernels of large
 // lattices, which hold a whole site's operands in registers meanwhile and wait
 // at the barrier: 16-bit updates at 32^3x64 74 us, with a finalize launch for
-// each sum 64 + 8 us; at 12^3x24 7.2 against 6.3 + 5 us.
+// each sum 64 + 8 us; at 12^3x24 7.2 against 6.3 + 5 us.  us per iteration, with the
+// ring below in place of SUM / SUM: 104 k 96.1 / 92.2, 174 k 133 / 131, 249 k 170 / 171,
+// 332 k 227 / 228, 432 k 296 / 299.
 template <class S> inline bool mix_sum(int vh) { return kLinear<S> || vh <= (1 << 18); }
 template <bool SUM> __device__ __forceinline__ double mix_total(const double *p, int n) {
   if constexpr (SUM) return partials_total(p, n);
