@@ -54,6 +54,10 @@ template <class S, class G> constexpr size_t solve_bytes_per_site(int nr = 1) {
 template <class S, class G> inline int operator_policy(int vh, int nr = 1, bool clover = true) {
   return solve_bytes_per_site<S, G>(nr) * (size_t)vh <= resident_bytes<S, G>(nr, clover) ? 0 : kNT;
 }
+// the largest lattice (sites per parity) whose operator is kept
+template <class S, class G> constexpr int kept_sites(bool clover) {
+  return (int)(resident_bytes<S, G>(1, clover) / solve_bytes_per_site<S, G>());
+}
 
 // Waves that share a site (1: k_dslash, else k_dslash_split).  us per CG
 // iteration at 1 / 2 / 4 waves:
@@ -70,10 +74,12 @@ template <class S, class G> inline int operator_policy(int vh, int nr = 1, bool 
 //   around the line of both, at 1 / 2: FP32 470 k 547 / 547, 524 k 559 / 573, 590 k 653 / 668,
 //           655 k 717 / 735; 16-bit 334 / 334, 329 / 336, 394 / 400, 424 / 432
 // Eight waves (one hop each) were slower than four from 4 k sites on.
+constexpr int kFourWaveSites = 1 << 15;
+template <class S, class G> constexpr int two_wave_sites() {
+  return !std::is_same<S, SF64>::value ? 1 << 19 : G::kRecon ? 1 << 17 : 3 << 14;
+}
 template <class S, class G> inline int split_waves(int vh) {
-  if (vh <= (1 << 15)) return 4;
-  constexpr int two = !std::is_same<S, SF64>::value ? 1 << 19 : G::kRecon ? 1 << 17 : 3 << 14;
-  return vh <= two ? 2 : 1;
+  return vh <= kFourWaveSites ? 4 : vh <= two_wave_sites<S, G>() ? 2 : 1;
 }
 
 // Sites per workgroup.  One wave per site in FP64 runs two workgroups of 256

@@ -205,7 +205,9 @@ static void launch_split(const DslashArgs<S, G> &a, bool dag, int epi, hipStream
 #define HB_DS(D, E) hipLaunchKernelGGL((k_dslash_split<S, G, D, E, NW, POL>), grid, block, 0, st, a)
   if (!dag) {
     switch (epi) {
-      case EPI_PLAIN: HB_DS(false, EPI_PLAIN); break;
+      case EPI_PLAIN:
+        if constexpr (std::is_same<G, SF64>::value) HB_DS(false, EPI_PLAIN);
+        break;
       case EPI_CLINV: HB_DS(false, EPI_CLINV); break;
       case EPI_MTIL: HB_DS(false, EPI_MTIL); break;
       case EPI_SOLVE:
@@ -215,7 +217,9 @@ static void launch_split(const DslashArgs<S, G> &a, bool dag, int epi, hipStream
     }
   } else {
     switch (epi) {
-      case EPI_PLAIN: HB_DS(true, EPI_PLAIN); break;
+      case EPI_PLAIN:
+        if constexpr (std::is_same<G, SF64>::value) HB_DS(true, EPI_PLAIN);
+        break;
       case EPI_CLINV: HB_DS(true, EPI_CLINV); break;
       case EPI_MTIL: HB_DS(true, EPI_MTIL); break;
       case EPI_SOLVE:
@@ -233,7 +237,9 @@ static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t
 #define HB_DS(D, E) hipLaunchKernelGGL((k_dslash<S, G, D, E, POL>), grid, block, 0, st, a)
   if (!dag) {
     switch (epi) {
-      case EPI_PLAIN: HB_DS(false, EPI_PLAIN); break;
+      case EPI_PLAIN:
+        if constexpr (std::is_same<G, SF64>::value) HB_DS(false, EPI_PLAIN);
+        break;
       case EPI_CLINV: HB_DS(false, EPI_CLINV); break;
       case EPI_MTIL: HB_DS(false, EPI_MTIL); break;
       case EPI_SOLVE:
@@ -243,7 +249,9 @@ static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t
     }
   } else {
     switch (epi) {
-      case EPI_PLAIN: HB_DS(true, EPI_PLAIN); break;
+      case EPI_PLAIN:
+        if constexpr (std::is_same<G, SF64>::value) HB_DS(true, EPI_PLAIN);
+        break;
       case EPI_CLINV: HB_DS(true, EPI_CLINV); break;
       case EPI_MTIL: HB_DS(true, EPI_MTIL); break;
       case EPI_SOLVE:
@@ -257,15 +265,30 @@ static void launch_pol(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t
 
 template <class S, class G>
 int launch_dslash(const DslashArgs<S, G> &a, bool dag, int epi, hipStream_t st) {
-  const int nw = split_waves<S, G>(a.g.vh), pol = operator_policy<S, G>(a.g.vh, 1, a.C != nullptr);
+  HB_CHECK((epi != EPI_PLAIN && epi != EPI_SOLVE) || (std::is_same<G, SF64>::value), HB_E_ARG,
+           "launch_dslash: epilogue %d is built for FP64 links of 18 reals", epi);
+  const int vh = a.g.vh, nw = split_waves<S, G>(vh);
+  const bool stream = operator_policy<S, G>(vh, 1, a.C != nullptr) == kNT;
+  // policies that the lines never combine with a form are not built
+  constexpr int two = two_wave_sites<S, G>();
+  constexpr int least = kept_sites<S, G>(true), most = kept_sites<S, G>(false);
+  static_assert(least >= kFourWaveSites && most >= least, "four waves share a site where the operator is kept");
   if (nw == 4) {
     launch_split<S, G, 4, 0>(a, dag, epi, st);
   } else if (nw == 2) {
-    if (pol == kNT) launch_split<S, G, 2, kNT>(a, dag, epi, st);
-    else launch_split<S, G, 2, 0>(a, dag, epi, st);
+    if constexpr (least < two) {
+      if (stream) launch_split<S, G, 2, kNT>(a, dag, epi, st);
+      else launch_split<S, G, 2, 0>(a, dag, epi, st);
+    } else {
+      launch_split<S, G, 2, 0>(a, dag, epi, st);
+    }
   } else {
-    if (pol == kNT) launch_pol<S, G, kNT>(a, dag, epi, st);
-    else launch_pol<S, G, 0>(a, dag, epi, st);
+    if constexpr (most > two) {
+      if (stream) launch_pol<S, G, kNT>(a, dag, epi, st);
+      else launch_pol<S, G, 0>(a, dag, epi, st);
+    } else {
+      launch_pol<S, G, kNT>(a, dag, epi, st);
+    }
   }
   HB_HIP(hipGetLastError());
   return HB_OK;

@@ -619,10 +619,10 @@ int cg_mixed_impl(Context *c, int op, double kappa, double rho, double2 *x, cons
     if (sums) {
       k_mix_update<S, true><<<grid, block, 0, c->stream>>>(r, q, n, st, k, sum, nsum, pb);
       k_mix_pupdate<S><<<grid, block, 0, c->stream>>>(p, r, xlo, n, st, k, pb, grid, note);
-    } else {
+    } else if constexpr (!kLinear<S>) {
       k_mix_update<S, false><<<grid, block, 0, c->stream>>>(r, q, n, st, k, sum, nsum, pb);
       k_finalize<1><<<1, kFinThreads, 0, c->stream>>>(pb, grid, nullptr, FinMixStep{st, k, last, note});
-      if constexpr (!kLinear<S>) k_mix_pupdate_ring<S><<<grid, block, 0, c->stream>>>(ring, r, xlo, n, st, k, last);
+      k_mix_pupdate_ring<S><<<grid, block, 0, c->stream>>>(ring, r, xlo, n, st, k, last);
     }
     HB_HIP(hipGetLastError());
     HB_TRY(watch.look(&flag));
