@@ -3,10 +3,12 @@
 // (dsg.F90), link update (hmc_u.F90) and the clover action
 // (clover/clover_action.F90), all in FP64 on device-resident fields.
 //
-// Every force kernel is a gather over links: one thread owns one link
-// (mu, eo, i) and adds all terms of that link to its 8 momentum coordinates,
-// so no atomics are needed and the result is deterministic.  Momenta are
-// device SoA P[4 mu][2 eo][8][vh].
+// The force kernels gather: all terms of a link are added to its 8 momentum
+// coordinates by one thread, so no atomics are needed and the result is
+// deterministic.  In the fermion and clover forces one thread owns one link
+// (mu, eo, i); in the gauge force a wave owns a plane of 64 sites, and the
+// shares of the six planes meet in LDS.  Momenta are device SoA
+// P[4 mu][2 eo][8][vh].
 #include "hb_ops.h"
 #include "hb_su3.h"
 
@@ -629,13 +631,11 @@ int dsf_dev(Context *c, double *P, double step, double kappa, double csw_kappa, 
     DslashArgs<SF64> d2 = dslash_args64(c, 1, bt, b);
     d2.C = d1.C;
     HB_TRY(launch_dslash(d2, true, clov ? EPI_SOLVE : EPI_PLAIN, c->stream));
-  } else {
-    HB_TRY(zero_f64(c, at, 12 * (size_t)vh));
-    HB_TRY(zero_f64(c, bt, 12 * (size_t)vh));
   }
   const LinkGrid lg(c->g);
   const HopForce hop{a, b, at, bt, -step * 2.0 * kappa * kappa};
-  // clover part (dsf.F90:103-109) on physical links
+  // clover part (dsf.F90:103-109) on physical links; at kappa = 0 neither the
+  // hopping part nor the odd sites' clover part is there and nothing reads at, bt
   const double s1 = -step * 2.0 * (csw_kappa / 8.0);
   const double s2 = s1 * kappa * kappa;
   if (s1 != 0.0)
