@@ -485,10 +485,10 @@ __global__ __launch_bounds__(kLinkBlock, 2) void k_clover_force(double *P, const
 // ten links and nine products per plane, where the two links' staples taken
 // apart read fourteen; the sites' own links, which every plane needs, are
 // shared through LDS, and so are the six waves' shares of the four forces.
-// Bound by the addresser of the vector memory path (busy 77 % with the links
-// in memory, 60 % here, FP64 issue 36 %): 32^3x64 1.30 ms, one wave per
-// direction 1.54 ms; 16^3x32 118 -> 87 us.  Registers for one link fetched
-// ahead spill (1.37 ms); two waves per SIMD with both own links held: 1.67 ms.
+// No unit is saturated (vector memory addresser 59 % busy, 77 % with the own
+// links in memory; FP64 issue 37 %): 32^3x64 1.30 ms, one wave per direction
+// 1.54 ms; 16^3x32 118 -> 87 us.  Registers for one link fetched ahead spill
+// (1.37 ms); two waves per SIMD with both own links held: 1.67 ms.
 constexpr int kPlaneBlock = 384;
 __global__ __launch_bounds__(kPlaneBlock, 3) void k_gauge_force(double *P, const double2 *__restrict__ U, Geom g, int run,
                                                                 double s) {
