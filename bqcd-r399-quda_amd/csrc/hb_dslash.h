@@ -25,9 +25,9 @@ template <class S, class G = S> struct DslashArgs {
 };
 
 // Load policy of the links and clover words, which a kernel reads once: kept
-// in the caches while the operator and the vectors of a solve are not much
-// larger than the 256 MB last-level cache, streamed past them (so that the
-// neighbour spinors stay) beyond.  The lines in MiB of that working set, with
+// in the caches while the operator and the vectors of a solve are up to 1.4 to
+// 1.8 times as large as the 256 MB last-level cache, streamed past them (so that
+// the neighbour spinors stay) beyond.  The lines in MiB of that working set, with
 // us streamed / kept on either side (sites per parity):
 //   M~^+M~ in FP64, 18-real links 340: 104 k (332 MiB) 175 / 171, 112 k (359) 183 / 188;
 //       D alone, which reads no clover words, 360: 112 k 34.1 / 32.0, 120 k 35.7 / 36.0
